@@ -1164,6 +1164,555 @@ __global__ __launch_bounds__(1024) void k_mg_coarse_global(LvArgs a, const float
   }
 }
 
+// ---------------------------------------------------------------- tail
+// The V-cycle from level `t` down and back up in one launch of one workgroup,
+// for the levels that fit its LDS: two sweeps and the restriction on each
+// level, all SOR iterations of the coarsest (sim.rs:472-473), then the
+// prolongation and two sweeps on the way up -- the per-cell arithmetic and the
+// order of every sum are those of the kernels above.  On these levels (8 k
+// cells and fewer) a launch per sweep or transfer takes 4-5 us, all of it
+// launch and load latency, and the coarsest solve is a chain of 160 dependent
+// colour passes: both are bound by latency, which one workgroup with
+// everything in LDS and registers shortens.  Per launch, before and after:
+// levels 16x24x16 + 8x12x8 88 -> 47 us (two sweeps, restriction, solve,
+// prolongation, two sweeps), 10x20x10 alone 71 -> 39 us, 14x30x14 142 -> 97 us.
+//
+// Layout: an x-pair (2g, 2g + 1) of a row holds one cell of each colour, and
+// the two colours live in two LDS arrays indexed by pair (TL_CS floats apart,
+// an immediate offset): a colour pass then reads and writes consecutive words
+// in consecutive lanes (x with stride 2 would meet each bank twice).  For the
+// cell of colour c in pair (g, y, z), at x = 2g + o with o = (y + z + c) & 1,
+// the neighbours are in the other colour's array: x -+ 1 at pair g and at
+// g + (o ? 1 : -1), y -+ 1 and z -+ 1 at the pairs of the same g.  (The two x
+// terms open the sum, so their order does not matter.)  Rows have a pitch of
+// hx + 1, planes of (d1 + 1) rows: one ghost column, row and plane between
+// neighbours holds the phi = 0 beyond the box.
+constexpr int TL_NT = 1024, TL_MAX = 5, TL_CS = 12288, TL_K = 8, TL_TOP = 4, TL_INNER = 4096;
+
+struct TailLv {
+  int d0, d1, d2, hx, py, pz;
+  int off, np, n;  // LDS offset of the level's pairs, pairs, cells
+  int io, bo;      // offsets of the level's codes and of an inner level's b in LDS
+  float hh, wdir;
+  FastDiv dhx, dd0, dd1;
+  const __attribute__((address_space(1))) uint8_t *nc;  // global memory
+  __attribute__((address_space(1))) float *phi, *b;
+};
+struct TailArgs {
+  int nl, iters;
+  float omega;
+  TailLv l[TL_MAX];
+};
+
+// x / c for a count c = fluid + wdir * outside given r = RN(1/c): div_count's
+// corrected product.  Over every float x with 2^-102 <= |x| < infinity and
+// each c of the levels 1..11 (214 values) it equals the IEEE quotient; a
+// smaller nonzero x (the remainder's low bits underflow) and an infinity (NaN
+// product) take the division.  c = r = 0 gives 0.
+template <bool ICNT>
+__device__ __forceinline__ bool div_redo(float x, float q, float r) {
+  if (ICNT) return __builtin_amdgcn_classf(q, 0x90);  // -subnormal | +subnormal
+  return r != 0.0f && ((fabsf(x) < 0x1p-100f && x != 0.0f) || q != q);
+}
+
+// LDS of the tail: phi (colour 0, then colour 1 at + TL_CS); b of the inner
+// levels and the neighbour codes of all, by cell; (count, RN(1/count)) of
+// level k's codes at ctab + 64 k.
+#define TAIL_SH float *sp, float *bl, uint8_t *cl, const float2 *ctab
+
+__device__ __forceinline__ void tail_pair(const TailLv &L, int p, int &g, int &y, int &z) {
+  const uint32_t r = fdiv((uint32_t)p, L.dhx), q = fdiv(r, L.dd1);
+  g = p - (int)r * L.hx;
+  z = (int)q;
+  y = (int)r - z * L.d1;
+}
+__device__ __forceinline__ int tail_li(const TailLv &L, int g, int y, int z) {
+  return L.off + (z + 1) * L.pz + (y + 1) * L.py + g + 1;
+}
+
+// The pairs t + 1024 j of thread t on one level: LDS index, cell 2g, codes of
+// the two colours | o of colour 0 << 16 | cell 2g in the level << 17 | cell
+// 2g + 1 << 18, h^2 b.
+template <int K>
+struct TailOwn {
+  int li[K], gi[K];
+  uint32_t cd[K];
+  float hb[K][2];
+};
+template <int K, bool inner>
+__device__ __forceinline__ void tail_own(const TailLv &L, TAIL_SH, TailOwn<K> &W) {
+#pragma unroll
+  for (int j = 0; j < K; j++) {
+    const int p = (int)threadIdx.x + TL_NT * j;
+    const bool act = p < L.np;
+    int g, y, z;
+    tail_pair(L, act ? p : 0, g, y, z);
+    const int o = (y + z) & 1, gi = 2 * g + L.d0 * (y + L.d1 * z);
+    const bool two = 2 * g + 1 < L.d0;
+    const int i1 = two ? gi + 1 : gi;
+    const uint32_t a0 = inner ? cl[L.io + gi] : L.nc[gi], a1 = inner ? cl[L.io + i1] : L.nc[i1];
+    const float b0 = inner ? bl[L.bo + gi] : L.b[gi], b1 = inner ? bl[L.bo + i1] : L.b[i1];
+    const uint32_t c0 = act ? a0 : (uint32_t)NC_NONE, c1 = act && two ? a1 : (uint32_t)NC_NONE;
+    W.li[j] = tail_li(L, g, y, z);
+    W.gi[j] = gi;
+    W.cd[j] = (o ? c1 | (c0 << 8) : c0 | (c1 << 8)) | ((uint32_t)o << 16) | (act ? 1u << 17 : 0u) |
+              (act && two ? 1u << 18 : 0u);
+    const float h0 = L.hh * b0, h1 = L.hh * b1;
+    W.hb[j][0] = o ? h1 : h0;
+    W.hb[j][1] = o ? h0 : h1;
+  }
+}
+
+// Two red-black sweeps (omega 1) over the owned pairs.
+template <int K, bool ICNT>
+__device__ __forceinline__ void tail_sweeps(const TailLv &L, TAIL_SH, int k, const TailOwn<K> &W) {
+  const float2 *ct = ctab + 64 * k;
+  const int py = L.py, pz = L.pz;
+  for (int s = 0; s < 2; s++) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      float *A = sp + c * TL_CS;
+      const float *O = sp + (1 - c) * TL_CS;
+      constexpr int KC = K < 2 ? K : 2;  // cells in flight (16 waves share the CU)
+#pragma unroll
+      for (int j0 = 0; j0 < K; j0 += KC) {
+        if (TL_NT * j0 >= L.np) break;  // no thread owns a pair here (uniform)
+        float nb[KC][6], cen[KC];
+        float2 cr[KC];
+#pragma unroll
+        for (int q = 0; q < KC; q++) {
+          const int j = j0 + q, i = W.li[j];
+          const int o = (int)((W.cd[j] >> 16) & 1u) ^ c;
+          nb[q][0] = O[i];
+          nb[q][1] = O[i + 2 * o - 1];
+          nb[q][2] = O[i + py];
+          nb[q][3] = O[i - py];
+          nb[q][4] = O[i + pz];
+          nb[q][5] = O[i - pz];
+          cen[q] = A[i];
+          cr[q] = ct[(W.cd[j] >> (8 * c)) & 63u];
+        }
+        float xs[KC], qs[KC];
+        bool redo = false;
+#pragma unroll
+        for (int q = 0; q < KC; q++) {
+          float sum = nb[q][0];
+#pragma unroll
+          for (int m = 1; m < 6; m++) sum += nb[q][m];
+          xs[q] = sum - W.hb[j0 + q][c];
+          const float q0 = xs[q] * cr[q].y;
+          const float e = __builtin_fmaf(-q0, cr[q].x, xs[q]);
+          qs[q] = __builtin_fmaf(e, cr[q].y, q0);
+          redo |= div_redo<ICNT>(xs[q], qs[q], cr[q].y);
+        }
+        if (redo) {
+#pragma unroll
+          for (int q = 0; q < KC; q++)
+            if (div_redo<ICNT>(xs[q], qs[q], cr[q].y)) {
+              float x = xs[q];
+              asm volatile("" : "+v"(x));
+              qs[q] = x / cr[q].x;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < KC; q++) {
+          const float nv = mixf_(cen[q], qs[q], 1.0f);
+          if (!((W.cd[j0 + q] >> (8 * c)) & (uint32_t)(NC_SOLID | NC_NONE))) A[W.li[j0 + q]] = nv;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// Residual of level F averaged over the fluid children of each cell of C
+// (k_mg_restrict; phi of C is 0 from the fill): a coarse cell's x-children
+// are one pair.
+template <bool inner>
+__device__ __forceinline__ void tail_restrict(const TailLv &F, const TailLv &C, TAIL_SH) {
+  for (int i = threadIdx.x; i < C.n; i += TL_NT) {
+    const uint32_t r = fdiv((uint32_t)i, C.dd0), zq = fdiv(r, C.dd1);
+    const int x = i - (int)r * C.d0, z = (int)zq, y = (int)r - z * C.d1;
+    const bool two = 2 * x + 1 < F.d0;
+    const int f0 = 2 * x + F.d0 * (2 * y + F.d1 * 2 * z), q0 = tail_li(F, x, 2 * y, 2 * z);
+    float bv[8];
+    uint32_t cv[8];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const int dy = m & 1, dz = m >> 1;
+      const bool in = 2 * y + dy < F.d1 && 2 * z + dz < F.d2;
+      const int f = in ? f0 + F.d0 * (dy + F.d1 * dz) : f0, f1 = two ? f + 1 : f;
+      const uint32_t a0 = cl[F.io + f], a1 = cl[F.io + f1];
+      bv[2 * m] = inner ? bl[F.bo + f] : F.b[f];
+      bv[2 * m + 1] = inner ? bl[F.bo + f1] : F.b[f1];
+      cv[2 * m] = in ? a0 : (uint32_t)NC_SOLID;
+      cv[2 * m + 1] = in && two ? a1 : (uint32_t)NC_SOLID;
+    }
+    float acc = 0.0f, nfl = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if (cv[k] & NC_SOLID) continue;  // solid or outside the level
+      const int o = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
+      const int col = (o + dy + dz) & 1;  // colour of x = 2 g + o at even y and z plus dy, dz
+      const float *A = sp + col * TL_CS, *O = sp + (1 - col) * TL_CS;
+      const int q = q0 + dy * F.py + dz * F.pz;
+      nfl += 1.0f;
+      float sum = 0.0f;
+      sum += O[q + o];      // x + 1
+      sum += O[q + o - 1];  // x - 1
+      sum += O[q + F.py];
+      sum += O[q - F.py];
+      sum += O[q + F.pz];
+      sum += O[q - F.pz];
+      acc += bv[k] - (sum - nc_count(cv[k], F.wdir) * A[q]) / F.hh;
+    }
+    const float bc = nfl > 0.0f ? acc / fmax_(nfl, 1.0f) : 0.0f;
+    bl[C.bo + i] = bc;
+    C.b[i] = bc;
+  }
+  __syncthreads();
+}
+
+// Masked, renormalised trilinear correction of level F from C (the general
+// form of k_mg_prolong), one coarse cell's eight children per thread: they
+// interpolate from its 27 neighbours, clamped at the level's sides.  A fine
+// index's fraction is 0.75 (even) or 0.25 (odd), so the weights are exact
+// products of constants, and without a solid coarse cell they sum to 1.
+__device__ __forceinline__ void tail_prolong(const TailLv &C, const TailLv &F, TAIL_SH, bool solid) {
+  for (int i = threadIdx.x; i < C.n; i += TL_NT) {
+    const uint32_t r = fdiv((uint32_t)i, C.dd0), zq = fdiv(r, C.dd1);
+    const int X = i - (int)r * C.d0, Z = (int)zq, Y = (int)r - Z * C.d1;
+    const int xs[3] = {X > 0 ? X - 1 : 0, X, X + 1 < C.d0 ? X + 1 : X};
+    float v[27];
+    uint32_t sm = 0u;
+#pragma unroll
+    for (int m = 0; m < 9; m++) {
+      const int cy = clampi(Y + m % 3 - 1, 0, C.d1 - 1), cz = clampi(Z + m / 3 - 1, 0, C.d2 - 1);
+      const int row = tail_li(C, 0, cy, cz), par = cy + cz;
+#pragma unroll
+      for (int u = 0; u < 3; u++)
+        v[3 * m + u] = sp[((xs[u] + par) & 1) * TL_CS + row + (xs[u] >> 1)];
+      if (solid) {
+        const int crow = C.io + C.d0 * (cy + C.d1 * cz);
+#pragma unroll
+        for (int u = 0; u < 3; u++) sm |= (cl[crow + xs[u]] & NC_SOLID) ? 1u << (3 * m + u) : 0u;
+      }
+    }
+    const int q0 = tail_li(F, X, 2 * Y, 2 * Z), f0 = F.io + 2 * X + F.d0 * (2 * Y + F.d1 * 2 * Z);
+#pragma unroll
+    for (int ch = 0; ch < 8; ch++) {
+      const int o = ch & 1, dy = (ch >> 1) & 1, dz = ch >> 2;
+      if (2 * X + o >= F.d0 || 2 * Y + dy >= F.d1 || 2 * Z + dz >= F.d2) continue;
+      if (cl[f0 + o + F.d0 * (dy + F.d1 * dz)] & NC_SOLID) continue;
+      const float frx = o ? 0.25f : 0.75f, fry = dy ? 0.25f : 0.75f, frz = dz ? 0.25f : 0.75f;
+      float acc = 0.0f, ws = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        const int ox = k & 1, oy = (k >> 1) & 1, oz = k >> 2;
+        const int e = 3 * (3 * (oz + dz) + (oy + dy)) + ox + o;
+        const float wx = ox ? frx : 1.0f - frx, wy = oy ? fry : 1.0f - fry, wz = oz ? frz : 1.0f - frz;
+        float wgt = (wx * wy) * wz;
+        if (solid) {
+          wgt = (sm >> e) & 1u ? 0.0f : wgt;
+          ws += wgt;
+        }
+        acc += wgt * v[e];
+      }
+      float corr = acc;
+      if (solid && ws != 1.0f) {
+        float a = acc;
+        asm volatile("" : "+v"(a));
+        corr = a / ws;
+      }
+      float *A = sp + ((o + dy + dz) & 1) * TL_CS + q0 + dy * F.py + dz * F.pz;
+      if (!solid || ws > 1e-4f) *A = *A + corr;
+    }
+  }
+  __syncthreads();
+}
+
+// The SOR iterations of the coarsest level: thread t owns K pairs of one
+// (g, y) column, z = z0 .. z0 + K - 1, with phi, h^2 b, count and reciprocal
+// of both colours in registers.  The pair's other cell and the z neighbours
+// inside the segment are registers too, so a cell costs three LDS reads plus
+// the segment's two ends.  A pass issues its reads first and stores the
+// branch-free quotients; one branch per pass redoes those that need the IEEE
+// division and stores them again.  K = 1 spreads a small level over the most
+// lanes: the pass is then its latency chain (LDS read, 13 dependent
+// operations, LDS write, barrier).  A slot that is never updated holds phi =
+// count = reciprocal = 0 and keeps 0, as in k_mg_coarse_z.
+template <int K, bool ICNT, bool inner>
+__device__ __forceinline__ void tail_sor(const TailLv &L, TAIL_SH, int k, int iters, float omega) {
+  const float2 *ct = ctab + 64 * k;
+  const int cols = L.hx * L.d1;
+  const int nseg = (L.d2 + K - 1) / K;
+  const int t = threadIdx.x;
+  if (__builtin_amdgcn_readfirstlane(t) >= cols * nseg) {  // a wave without columns only keeps the barriers
+    for (int it = 0; it < 2 * iters; it++) __syncthreads();
+    return;
+  }
+  const bool act = t < cols * nseg;
+  const int seg = act ? t / cols : 0, cg = act ? t - seg * cols : 0;
+  const int y = cg / L.hx, g = cg - y * L.hx, z0 = seg * K;
+  int li[K];
+  float ph[K][2], hb[K][2], cn[K][2], rc[K][2];
+#pragma unroll
+  for (int j = 0; j < K; j++) {
+    const int z = z0 + j;
+    const bool inz = act && z < L.d2;
+    // a slot past the level or a thread without a column points at the first
+    // pair: its reads stay in the level, it stores nothing
+    li[j] = inz ? tail_li(L, g, y, z) : tail_li(L, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const int x = 2 * g + ((y + z + c) & 1);
+      const bool in = inz && x < L.d0;
+      const int i = in ? x + L.d0 * (y + L.d1 * z) : 0;
+      const uint32_t code = cl[L.io + i];
+      const float b = inner ? bl[L.bo + i] : L.b[i];
+      const bool up = in && !(code & (uint32_t)(NC_SOLID | NC_NONE));
+      const float2 cr = ct[code & 63u];
+      ph[j][c] = up ? sp[c * TL_CS + li[j]] : 0.0f;
+      cn[j][c] = up ? cr.x : 0.0f;
+      rc[j][c] = up ? cr.y : 0.0f;
+      hb[j][c] = up ? L.hh * b : 0.0f;
+    }
+  }
+  const int e = ((y + z0) & 1) ? 1 : -1;  // side of the LDS x neighbour of slot 0, colour 0
+  const int nz = act ? (L.d2 - z0 < K ? L.d2 - z0 : K) : 0;  // slots inside the level
+  const int zt = li[0] - L.pz, zb = nz == K ? li[K - 1] + L.pz : li[0] - L.pz;
+  const int py = L.py;
+  for (int it = 0; it < iters; it++) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const float *O = sp + (1 - c) * TL_CS;
+      float nb[K][3];
+#pragma unroll
+      for (int j = 0; j < K; j++) {
+        nb[j][0] = O[li[j] + (((j + c) & 1) ? -e : e)];
+        nb[j][1] = O[li[j] + py];
+        nb[j][2] = O[li[j] - py];
+      }
+      const float zlo = O[zt], zhi = O[zb];
+      float xs[K], qs[K], old[K];
+      bool redo = false;
+#pragma unroll
+      for (int j = 0; j < K; j++) {
+        float sum = ph[j][1 - c] + nb[j][0];
+        sum += nb[j][1];
+        sum += nb[j][2];
+        sum += j + 1 < K ? ph[j + 1][1 - c] : zhi;
+        sum += j > 0 ? ph[j - 1][1 - c] : zlo;
+        xs[j] = sum - hb[j][c];
+        const float q0 = xs[j] * rc[j][c];
+        const float er = __builtin_fmaf(-q0, cn[j][c], xs[j]);
+        qs[j] = __builtin_fmaf(er, rc[j][c], q0);
+        old[j] = ph[j][c];
+        ph[j][c] = mixf_(old[j], qs[j], omega);
+        if (j < nz) sp[c * TL_CS + li[j]] = ph[j][c];
+        redo |= div_redo<ICNT>(xs[j], qs[j], rc[j][c]);
+      }
+      if (redo) {
+#pragma unroll
+        for (int j = 0; j < K; j++)
+          if (div_redo<ICNT>(xs[j], qs[j], rc[j][c])) {
+            float x = xs[j];
+            asm volatile("" : "+v"(x));
+            ph[j][c] = mixf_(old[j], x / cn[j][c], omega);
+            if (j < nz) sp[c * TL_CS + li[j]] = ph[j][c];
+          }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+template <int KT, int KC, bool ICNT>
+__global__ __launch_bounds__(TL_NT) void k_mg_tail(TailArgs) {
+  // the levels are indexed at run time: read where they are (uniform scalar
+  // loads from the kernel arguments), a copy of the argument would be indexed
+  // in scratch memory
+  const TailArgs &a = *(const TailArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  __shared__ __align__(16) float sp[2 * TL_CS];
+  __shared__ float bl[TL_INNER];
+  __shared__ uint8_t cl[2 * TL_NT * TL_K + TL_INNER];
+  __shared__ float2 ct[64 * TL_MAX];
+  const int t = threadIdx.x;
+  if (t < 64 * a.nl) {
+    const uint32_t code = (uint32_t)t & 63u;
+    const float c = nc_count(code, a.l[t / 64].wdir);
+    ct[t] = make_float2(c, c > 0.0f ? 1.0f / c : 0.0f);
+  }
+  for (int i = t; i < 2 * TL_CS / 4; i += TL_NT)
+    reinterpret_cast<float4 *>(sp)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  uint32_t solid = 0u;  // bit l: level l has a solid cell
+  for (int l = 1; l < a.nl; l++) {
+    bool sl = false;
+    for (int i = t; i < a.l[l].n; i += TL_NT) {
+      const uint8_t code = a.l[l].nc[i];
+      cl[a.l[l].io + i] = code;
+      sl |= (code & NC_SOLID) != 0;
+    }
+    solid |= __syncthreads_or(sl) ? 1u << l : 0u;
+  }
+  TailOwn<KT> W;
+  {
+    // the top level's codes, h^2 b and phi (a solid reads 0 in the sums and keeps its phi in memory)
+    const TailLv &T = a.l[0];
+    tail_own<KT, false>(T, sp, bl, cl, ct, W);
+    float p[KT][2];
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+      p[j][0] = T.phi[W.gi[j]];
+      p[j][1] = T.phi[W.gi[j] + ((W.cd[j] >> 18) & 1u)];
+    }
+    __syncthreads();  // the zero fill is complete
+#pragma unroll
+    for (int j = 0; j < KT; j++) {
+      const uint32_t o = (W.cd[j] >> 16) & 1u;
+      const uint32_t c0 = (W.cd[j] >> (8 * o)) & 0xffu, c1 = (W.cd[j] >> (8 * (o ^ 1u))) & 0xffu;
+      if (W.cd[j] & (1u << 17)) {
+        sp[(int)o * TL_CS + W.li[j]] = (c0 & NC_SOLID) ? 0.0f : p[j][0];
+        cl[T.io + W.gi[j]] = (uint8_t)c0;
+      }
+      if (W.cd[j] & (1u << 18)) {
+        sp[(int)(o ^ 1u) * TL_CS + W.li[j]] = (c1 & NC_SOLID) ? 0.0f : p[j][1];
+        cl[T.io + W.gi[j] + 1] = (uint8_t)c1;
+      }
+    }
+    __syncthreads();
+  }
+  auto smooth = [&](int l) __attribute__((always_inline)) {
+    if (l == 0) {
+      tail_sweeps<KT, ICNT>(a.l[0], sp, bl, cl, ct, 0, W);
+    } else {
+      TailOwn<2> I;
+      tail_own<2, true>(a.l[l], sp, bl, cl, ct, I);
+      tail_sweeps<2, ICNT>(a.l[l], sp, bl, cl, ct, l, I);
+    }
+  };
+  for (int l = 0; l < a.nl - 1; l++) {
+    smooth(l);
+    if (l == 0) tail_restrict<false>(a.l[0], a.l[1], sp, bl, cl, ct);
+    else tail_restrict<true>(a.l[l], a.l[l + 1], sp, bl, cl, ct);
+  }
+  if (a.nl == 1) tail_sor<KC, ICNT, false>(a.l[0], sp, bl, cl, ct, 0, a.iters, a.omega);
+  else tail_sor<KC, ICNT, true>(a.l[a.nl - 1], sp, bl, cl, ct, a.nl - 1, a.iters, a.omega);
+  for (int l = a.nl - 2; l >= 0; l--) {
+    tail_prolong(a.l[l + 1], a.l[l], sp, bl, cl, ct, (solid >> (l + 1)) & 1u);
+    smooth(l);
+  }
+  // phi back to memory: the top level's from the owned pairs (solids and, of
+  // a coarsest level alone, the cells its solve skips keep theirs)
+  const uint32_t keep = a.nl == 1 ? NC_SOLID | NC_NONE : NC_SOLID;
+#pragma unroll
+  for (int j = 0; j < KT; j++) {
+    const uint32_t o = (W.cd[j] >> 16) & 1u;
+    const uint32_t c0 = (W.cd[j] >> (8 * o)) & 0xffu, c1 = (W.cd[j] >> (8 * (o ^ 1u))) & 0xffu;
+    if ((W.cd[j] & (1u << 17)) && !(c0 & keep)) a.l[0].phi[W.gi[j]] = sp[(int)o * TL_CS + W.li[j]];
+    if ((W.cd[j] & (1u << 18)) && !(c1 & keep)) a.l[0].phi[W.gi[j] + 1] = sp[(int)(o ^ 1u) * TL_CS + W.li[j]];
+  }
+  for (int l = 1; l < a.nl; l++) {
+    const TailLv &L = a.l[l];
+    for (int i = t; i < L.n; i += TL_NT) {
+      const uint32_t r = fdiv((uint32_t)i, L.dd0), zq = fdiv(r, L.dd1);
+      const int x = i - (int)r * L.d0, z = (int)zq, y = (int)r - z * L.d1;
+      L.phi[i] = sp[((x + y + z) & 1) * TL_CS + tail_li(L, x >> 1, y, z)];
+    }
+  }
+}
+
+// Pairs per thread of the coarsest solve: the fewest with which the level's
+// columns, cut into z segments, fit the workgroup (0: none do).  Fewer pairs
+// on more lanes shorten the pass: 0.17 us at K = 1 (8x12x8), 0.35 at 2
+// (12x20x12), 0.6 at 4 (14x30x14).
+static int tail_k(const MgLevel &L) {
+  const int cols = ((L.d[0] + 1) / 2) * L.d[1];
+  for (int k : {1, 2, 4, 8})
+    if (cols * ((L.d[2] + k - 1) / k) <= TL_NT) return k;
+  return 0;
+}
+static int tail_floats(const MgLevel &L) {  // LDS words of one colour's pairs with their ghosts
+  const int py = (L.d[0] + 1) / 2 + 1, pz = py * (L.d[1] + 1);
+  return (L.d[2] + 2) * pz + py + 2;
+}
+// Whether levels t .. nl - 1 run as one tail.  A level that is smoothed in it
+// has at most 4 pairs per thread: each instruction per cell costs one CU what
+// 256 share in a launch of its own, and with a 16 k-cell level on top (8 pairs
+// per thread) the tail took 94 us against 39 us and six launches of 4.7 us.
+static bool tail_fits(const MgLevel *lv, int t, int nl) {
+  int64_t words = 0, inner = 0;
+  if (nl - t > TL_MAX || !tail_k(lv[nl - 1])) return false;
+  for (int l = t; l < nl; l++) {
+    const MgLevel &L = lv[l];
+    if (L.n > 2u * TL_NT * TL_K) return false;
+    const int np = ((L.d[0] + 1) / 2) * L.d[1] * L.d[2];
+    if (np > TL_NT * (t == nl - 1 ? TL_K : l == t ? TL_TOP : 2)) return false;
+    words += tail_floats(L);
+    if (l > t) inner += L.n;
+  }
+  return words <= TL_CS && inner <= TL_INNER;
+}
+static TailArgs tail_args(const MgLevel *lv, int t, int nl, int iters, float omega) {
+  TailArgs a;
+  a.nl = nl - t;
+  a.iters = iters;
+  a.omega = omega;
+  int off = 0, io = 0;
+  for (int l = t; l < nl; l++) {
+    const MgLevel &L = lv[l];
+    TailLv &T = a.l[l - t];
+    T.d0 = L.d[0]; T.d1 = L.d[1]; T.d2 = L.d[2];
+    T.hx = (L.d[0] + 1) / 2;
+    T.py = T.hx + 1;
+    T.pz = T.py * (L.d[1] + 1);
+    T.off = off;
+    T.np = T.hx * L.d[1] * L.d[2];
+    T.n = (int)L.n;
+    T.io = io;
+    T.bo = l > t ? io - a.l[0].n : 0;
+    off += tail_floats(L);
+    io += T.n;
+    T.hh = L.hh;
+    T.wdir = L.wdir;
+    T.dhx = make_fastdiv((uint32_t)T.hx);
+    T.dd0 = make_fastdiv((uint32_t)T.d0);
+    T.dd1 = make_fastdiv((uint32_t)T.d1);
+    T.nc = (const __attribute__((address_space(1))) uint8_t *)L.nc;
+    T.phi = (__attribute__((address_space(1))) float *)L.phi;
+    T.b = (__attribute__((address_space(1))) float *)L.b;
+  }
+  return a;
+}
+
+template <int KT, int KC>
+static void launch_tail(const TailArgs &a, bool icnt, hipStream_t s) {
+  if (icnt) k_mg_tail<KT, KC, true><<<1, TL_NT, 0, s>>>(a);
+  else k_mg_tail<KT, KC, false><<<1, TL_NT, 0, s>>>(a);
+}
+static void launch_mg_tail(const MgLevel *lv, int t, int nl, int iters, float omega, hipStream_t s) {
+  const TailArgs a = tail_args(lv, t, nl, iters, omega);
+  bool icnt = true;
+  for (int l = t; l < nl; l++) icnt = icnt && lv[l].wdir == 1.0f;
+  const int kc = tail_k(lv[nl - 1]);
+  const int kt = a.l[0].np <= 2 * TL_NT ? 2 : a.l[0].np <= 4 * TL_NT ? 4 : TL_K;
+  switch (kc) {
+    case 1:
+      if (kt == 2) launch_tail<2, 1>(a, icnt, s);
+      else launch_tail<TL_TOP, 1>(a, icnt, s);
+      break;
+    case 2:
+      if (kt == 2) launch_tail<2, 2>(a, icnt, s);
+      else launch_tail<TL_TOP, 2>(a, icnt, s);
+      break;
+    case 4:
+      launch_tail<TL_TOP, 4>(a, icnt, s);
+      break;
+    default: launch_tail<TL_K, 8>(a, icnt, s); break;
+  }
+}
+
 bool mg_coarse_fits_lds(const MgLevel &L) {
   uint32_t pad = (uint32_t)(L.d[0] + 2) * (uint32_t)(L.d[1] + 2) * (uint32_t)(L.d[2] + 2);
   uint32_t half = (uint32_t)((L.d[0] + 1) / 2) * (uint32_t)L.d[1] * (uint32_t)L.d[2];
@@ -1174,6 +1723,10 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
   LvArgs a = lv_args(L);
   const int ncol = L.d[0] * L.d[1];
   const bool colz = L.wdir == 1.0f && ncol <= CO_NT;
+  if (tail_fits(&L, 0, 1) && (!colz || tail_k(L) < 8)) {
+    launch_mg_tail(&L, 0, 1, iters, omega, s);
+    return;
+  }
   // one thread per column, whole waves only: a wave without columns would
   // still run every colour pass's arithmetic on the CU
   const int colt = ((ncol + 63) / 64) * 64;
@@ -1257,12 +1810,16 @@ void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s) 
     launch_mg_sweep(L, L.phi, L.tmp, 1.0f, s, fine);
     launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, fine);
   };
-  for (int l = 0; l < nl - 1; l++) {
+  // the levels from t on run in one launch where they fit
+  int t = nl - 1;
+  while (t > 0 && tail_fits(lv, t - 1, nl)) t--;
+  for (int l = 0; l < t; l++) {
     sweeps(lv[l], l == 0);
     launch_mg_restrict(lv[l], lv[l + 1], s);
   }
-  launch_mg_coarse(lv[nl - 1], coarse_iters, 1.6f, s);
-  for (int l = nl - 2; l >= 0; l--) {
+  if (t < nl - 1) launch_mg_tail(lv, t, nl, coarse_iters, 1.6f, s);
+  else launch_mg_coarse(lv[t], coarse_iters, 1.6f, s);
+  for (int l = t - 1; l >= 0; l--) {
     launch_mg_prolong(lv[l + 1], lv[l], s);
     sweeps(lv[l], l == 0);
   }
