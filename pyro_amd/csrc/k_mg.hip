@@ -1138,32 +1138,6 @@ __global__ __launch_bounds__(EX ? CZ_EX_NT : CO_NT) void k_mg_coarse_z(LvArgs a,
   }
 }
 
-// Same schedule for a coarsest level larger than LDS: one workgroup, phi in
-// global memory (L2-resident), a workgroup barrier between colour passes.
-__global__ __launch_bounds__(1024) void k_mg_coarse_global(LvArgs a, const float *__restrict__ b,
-                                                            const uint8_t *__restrict__ f, float *p, int iters,
-                                                            float omega) {
-  for (int it = 0; it < iters; it++) {
-    for (int color = 0; color < 2; color++) {
-      for (uint32_t t = threadIdx.x; t < a.nhalf; t += 1024) {
-        uint32_t r = fdiv(t, a.dhx);
-        int gx = (int)(t - r * a.dhx.d);
-        uint32_t zq = fdiv(r, a.dny);
-        int y = (int)(r - zq * (uint32_t)a.d1), z = (int)zq;
-        int x = 2 * gx + ((y + z + color) & 1);
-        if (x >= a.d0) continue;
-        uint32_t i = (uint32_t)x + (uint32_t)a.d0 * ((uint32_t)y + (uint32_t)a.d1 * (uint32_t)z);
-        if (f[i] == 1) continue;
-        float sum, cnt;
-        nsum(a.d0, a.d1, a.d2, p, f, x, y, z, i, a.wdir, sum, cnt);
-        if (cnt < 0.5f) continue;
-        p[i] = mixf_(p[i], (sum - a.hh * b[i]) / cnt, omega);
-      }
-      __syncthreads();
-    }
-  }
-}
-
 // ---------------------------------------------------------------- tail
 // The V-cycle from level `t` down and back up in one launch of one workgroup,
 // for the levels that fit its LDS: two sweeps and the restriction on each
@@ -1769,8 +1743,12 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
     const uint32_t nt = a.nhalf >= (uint32_t)CO_NT ? (uint32_t)CO_NT : ((a.nhalf + 63u) / 64u) * 64u;
     k_mg_coarse<<<1, nt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
   }
-  else
-    k_mg_coarse_global<<<1, 1024, 0, s>>>(a, L.b, L.f, L.phi, iters, omega);
+  else {
+    for (int it = 0; it < iters; it += 2) {
+      launch_mg_sweep(L, L.phi, L.tmp, omega, s, false);
+      launch_mg_sweep(L, L.tmp, L.phi, omega, s, false);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- resid
