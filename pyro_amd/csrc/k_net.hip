@@ -42,10 +42,9 @@ int conv_groups(int ca, int cb, int cout) {
   return (ca / cca) * (cca == 32 ? 27 : 14) + (cb == 16 ? 14 : (cb / 32) * 27);
 }
 
-__global__ __launch_bounds__(256) void k_pack_conv(const float *__restrict__ W, int cout, int cin, int ca_e, int cb_e,
-                                                   int cout_e, int transposed, uint32_t total, bf16 *__restrict__ wp) {
-  const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-  if (e >= total) return;
+// element e of the packed weights of one conv (see net.hpp)
+__device__ __forceinline__ bf16 packed_weight(const float *__restrict__ W, int cout, int cin, int ca_e, int cb_e,
+                                              int cout_e, bool transposed, uint32_t e) {
   const int kk = (int)(e % 32u);
   const int co_e = (int)((e / 32u) % (uint32_t)cout_e);
   int grp = (int)(e / (32u * (uint32_t)cout_e));
@@ -77,13 +76,55 @@ __global__ __launch_bounds__(256) void k_pack_conv(const float *__restrict__ W, 
     else  // adjoint: input channel = original output channel, taps mirrored
       v = W[((size_t)ci_e * cin + co_e) * 27 + (26 - tap)];
   }
-  wp[e] = tobf(v);
+  return tobf(v);
+}
+// All packed copies of one parameter vector in one launch: a training step
+// repacks every layer in both directions, and fourteen launches of a few
+// thousand elements took 4.5 us each.
+struct PackEntry {
+  const __attribute__((address_space(1))) float *W;
+  __attribute__((address_space(1))) bf16 *wp;
+  int cout, cin, ca_e, cb_e, cout_e, transposed;
+  uint32_t total, block0;  // elements, first block
+};
+struct PackArgs {
+  int n;
+  PackEntry e[PACK_MAX];
+};
+__global__ __launch_bounds__(256) void k_pack_conv(PackArgs) {
+  // indexed by block where the arguments lie (a copy would be indexed in scratch memory)
+  const PackArgs &a = *(const PackArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  int k = 0;
+  while (k + 1 < a.n && blockIdx.x >= a.e[k + 1].block0) k++;
+  const PackEntry &p = a.e[k];
+  const uint32_t e = (blockIdx.x - p.block0) * 256u + threadIdx.x;
+  if (e >= p.total) return;
+  p.wp[e] = packed_weight((const float *)p.W, p.cout, p.cin, p.ca_e, p.cb_e, p.cout_e, p.transposed != 0, e);
+}
+void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s) {
+  PackArgs a;
+  uint32_t blocks = 0;
+  a.n = n < PACK_MAX ? n : PACK_MAX;
+  for (int k = 0; k < a.n; k++) {
+    const ConvSpec &c = jobs[k].c;
+    PackEntry &p = a.e[k];
+    p.W = (const __attribute__((address_space(1))) float *)jobs[k].W;
+    p.wp = (__attribute__((address_space(1))) bf16 *)jobs[k].wp;
+    p.cout = c.cout;
+    p.cin = c.cin();
+    p.ca_e = jobs[k].transposed ? 0 : c.ca;
+    p.cb_e = jobs[k].transposed ? c.cout : c.cb;
+    p.cout_e = jobs[k].transposed ? c.cin() : c.cout;
+    p.transposed = jobs[k].transposed ? 1 : 0;
+    p.total = (uint32_t)conv_groups(p.ca_e, p.cb_e, p.cout_e) * (uint32_t)p.cout_e * 32u;
+    p.block0 = blocks;
+    blocks += nblk(p.total);
+  }
+  k_pack_conv<<<blocks, 256, 0, s>>>(a);
 }
 void launch_pack_conv(const float *W, const ConvSpec &c, bool transposed, bf16 *wp, hipStream_t s) {
-  const int ca_e = transposed ? 0 : c.ca, cb_e = transposed ? c.cout : c.cb;
-  const int cout_e = transposed ? c.cin() : c.cout;
-  const uint32_t total = (uint32_t)conv_groups(ca_e, cb_e, cout_e) * (uint32_t)cout_e * 32u;
-  k_pack_conv<<<nblk(total), 256, 0, s>>>(W, c.cout, c.cin(), ca_e, cb_e, cout_e, transposed ? 1 : 0, total, wp);
+  const PackJob j{W, wp, c, transposed};
+  launch_pack_convs(&j, 1, s);
 }
 __global__ __launch_bounds__(256) void k_pack_bf16(const float *__restrict__ w, uint32_t n, bf16 *__restrict__ o) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -555,9 +596,11 @@ void launch_head_bwd(const G3 &g, const bf16 *d0, const float *gy, const float *
 // ------------------------------------------------------------ weight gradients
 // dW[co][ci][t] = sum_v g[v][co] * X[v + off(t)][ci].  The MFMA contracts over
 // voxels, so both operands are first written channel-major: GT[co][z][y][x]
-// and, for each x shift dx in {-1, 0, 1}, XT_dx[ci][z+1][y+1][x] =
-// X[x+dx][y][z] (zero outside the grid), rows padded to a pitch P multiple of
-// 32.  Every fragment is then one aligned 16-byte load.
+// (rows of P, a multiple of 32) and XT[ci][z + 1][y + 1][x + 8] (rows of
+// P + 16, zero outside the grid).  A B fragment is eight consecutive x of one
+// channel: the three x shifts of a row come from one aligned 16-byte load and
+// the words beside it (in other lanes), by funnel shifts.
+constexpr int DW_PAD = 8;  // elements before x = 0 and after x = P - 1
 DwPlan dw_plan(const G3 &g, const ConvSpec &c) {
   DwPlan d;
   d.P = (g.nx + 31) / 32 * 32;
@@ -571,223 +614,386 @@ DwPlan dw_plan(const G3 &g, const ConvSpec &c) {
 }
 size_t dw_xt_elems(const G3 &g, const ConvSpec &c) {
   const DwPlan d = dw_plan(g, c);
-  return (size_t)3 * d.rows_x * (size_t)(g.nz + 2) * (size_t)(g.ny + 2) * (size_t)d.P;
+  return (size_t)d.rows_x * (size_t)(g.nz + 2) * (size_t)(g.ny + 2) * (size_t)(d.P + 2 * DW_PAD);
 }
 size_t dw_gt_elems(const G3 &g, const ConvSpec &c) {
   const DwPlan d = dw_plan(g, c);
   return (size_t)c.cout * (size_t)g.nz * (size_t)g.ny * (size_t)d.P;
 }
+constexpr int BG_BLOCKS = 256;  // partials of the bias gradient
+static size_t dw_bias_at(const DwPlan &d, int cout) { return (size_t)d.S * 27 * cout * d.rows_x; }
 size_t dw_part_elems(const G3 &g, const ConvSpec &c) {
-  const DwPlan d = dw_plan(g, c);
-  const size_t dwp = (size_t)d.S * 27 * c.cout * d.rows_x;
-  const size_t bp = (size_t)256 * c.cout;
-  return dwp > bp ? dwp : bp;
+  return dw_bias_at(dw_plan(g, c), c.cout) + (size_t)BG_BLOCKS * c.cout;
 }
 
-// XT from the concatenated conv input [up(a) (ca ch), b (cb ch)]; 8 channels per thread
-__global__ __launch_bounds__(256) void k_to_xt(int nx, int ny, int nz, int P, int anx, int any, const bf16 *__restrict__ a,
-                                               int ca, const bf16 *__restrict__ b, int cb, int rows_x,
-                                               bf16 *__restrict__ xt) {
-  const int ng = (ca + cb) / 8;
-  const size_t plane = (size_t)(nz + 2) * (ny + 2) * P;
-  const size_t total = 3 * (size_t)ng * plane;
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= total) return;
-  const int xp = (int)(t % P);
-  size_t r = t / P;
-  const int yy = (int)(r % (ny + 2));
-  r /= (ny + 2);
-  const int zz = (int)(r % (nz + 2));
-  r /= (nz + 2);
-  const int cg = (int)(r % ng);
-  const int d = (int)(r / ng);
-  const int x = xp + d - 1, y = yy - 1, z = zz - 1;
-  bf16x8 v;
+// (Three shifted copies of XT, one per x tap, took three times the writes: 34
+// + 10 us a layer against 22 us for both operands.)
+// XT of the concatenated conv input [up(a) (ca ch), b (cb ch)] (cb = 2: the
+// network input, rows 2..15 zero) in the first xgroups rows of blocks, GT in
+// the rest: a row takes eight channels, a thread two x of them, one 4-byte
+// store per channel.
+struct TransArgs {
+  int nx, ny, nz, P, anx, any, ca, cb, cout, xgroups;
+  const bf16 *a, *b, *g;
+  bf16 *xt, *gt;
+  uint32_t x_items, g_items;  // per group of eight channels
+  FastDiv dxp, dxy, dgp, dgy;  // (P + 16) / 2, ny + 2; P / 2, ny
+};
+__device__ __forceinline__ uint32_t pair_of(bf16 lo, bf16 hi) {
+  return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
+}
+__global__ __launch_bounds__(256) void k_to_t(TransArgs p) {
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  bf16x8 v[2];
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = tobf(0.0f);
-  if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) {
-    const int c = 8 * cg;
-    if (c < ca) {
-      const size_t u = (size_t)(x >> 1) + (size_t)anx * ((size_t)(y >> 1) + (size_t)any * (size_t)(z >> 1));
-      v = *reinterpret_cast<const bf16x8 *>(a + u * ca + c);
-    } else {
-      const size_t w = (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * (size_t)z);
-      v = *reinterpret_cast<const bf16x8 *>(b + w * cb + (c - ca));
+  for (int e = 0; e < 2; e++)
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[e][i] = tobf(0.0f);
+  if ((int)blockIdx.y < p.xgroups) {
+    if (t >= p.x_items) return;
+    const uint32_t hp = p.dxp.d, h2 = p.dxy.d, r = fdiv(t, p.dxp), zz = fdiv(r, p.dxy), yy = r - zz * h2;
+    const int xp = 2 * (int)(t - r * hp);
+    const int y = (int)yy - 1, z = (int)zz - 1, c = 8 * (int)blockIdx.y;
+    if (y >= 0 && y < p.ny && z >= 0 && z < p.nz) {
+#pragma unroll
+      for (int e = 0; e < 2; e++) {
+        const int x = xp + e - DW_PAD;
+        if (x < 0 || x >= p.nx) continue;
+        const size_t w = (size_t)x + (size_t)p.nx * ((size_t)y + (size_t)p.ny * (size_t)z);
+        if (p.cb == 2) {
+          if (c == 0) {
+            v[e][0] = p.b[2 * w];
+            v[e][1] = p.b[2 * w + 1];
+          }
+        } else if (c < p.ca) {
+          const size_t u = (size_t)(x >> 1) + (size_t)p.anx * ((size_t)(y >> 1) + (size_t)p.any * (size_t)(z >> 1));
+          v[e] = *reinterpret_cast<const bf16x8 *>(p.a + u * p.ca + c);
+        } else {
+          v[e] = *reinterpret_cast<const bf16x8 *>(p.b + w * p.cb + (c - p.ca));
+        }
+      }
     }
-  }
-  const size_t base = ((size_t)d * rows_x + 8 * cg) * plane + ((size_t)zz * (ny + 2) + yy) * P + xp;
+    const size_t plane = 2 * (size_t)p.x_items;
+    const size_t base = (size_t)c * plane + 2 * (size_t)t;
 #pragma unroll
-  for (int i = 0; i < 8; i++) xt[base + (size_t)i * plane] = v[i];
-}
-// XT of the 2-channel network input (rows 2..15 zero)
-__global__ __launch_bounds__(256) void k_to_xt_in(int nx, int ny, int nz, int P, const bf16 *__restrict__ x0,
-                                                  bf16 *__restrict__ xt) {
-  const size_t plane = (size_t)(nz + 2) * (ny + 2) * P;
-  const size_t total = 3 * plane;
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= total) return;
-  const int xp = (int)(t % P);
-  size_t r = t / P;
-  const int yy = (int)(r % (ny + 2));
-  r /= (ny + 2);
-  const int zz = (int)(r % (nz + 2));
-  const int d = (int)(r / (nz + 2));
-  const int x = xp + d - 1, y = yy - 1, z = zz - 1;
-  bf16 v0 = tobf(0.0f), v1 = tobf(0.0f);
-  if (x >= 0 && x < nx && y >= 0 && y < ny && z >= 0 && z < nz) {
-    const size_t w = (size_t)x + (size_t)nx * ((size_t)y + (size_t)ny * (size_t)z);
-    v0 = x0[2 * w];
-    v1 = x0[2 * w + 1];
+    for (int i = 0; i < 8; i++)
+      *reinterpret_cast<uint32_t *>(p.xt + base + (size_t)i * plane) = pair_of(v[0][i], v[1][i]);
+    return;
   }
-  const size_t base = (size_t)d * 16 * plane + ((size_t)zz * (ny + 2) + yy) * P + xp;
-  xt[base] = v0;
-  xt[base + plane] = v1;
-  for (int i = 2; i < 16; i++) xt[base + (size_t)i * plane] = tobf(0.0f);
-}
-// GT[co][z][y][x] (zero for x >= nx)
-__global__ __launch_bounds__(256) void k_to_gt(int nx, int ny, int nz, int P, int cout, const bf16 *__restrict__ g,
-                                               bf16 *__restrict__ gt) {
-  const int ng = cout / 8;
-  const size_t plane = (size_t)nz * ny * P;
-  const size_t total = (size_t)ng * plane;
-  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= total) return;
-  const int xp = (int)(t % P);
-  size_t r = t / P;
-  const int y = (int)(r % ny);
-  r /= ny;
-  const int z = (int)(r % nz);
-  const int cg = (int)(r / nz);
-  bf16x8 v;
+  if (t >= p.g_items) return;
+  const uint32_t r = fdiv(t, p.dgp), z = fdiv(r, p.dgy), y = r - z * p.dgy.d;
+  const int xp = 2 * (int)(t - r * p.dgp.d), c = 8 * ((int)blockIdx.y - p.xgroups);
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = tobf(0.0f);
-  if (xp < nx) {
-    const size_t w = (size_t)xp + (size_t)nx * ((size_t)y + (size_t)ny * (size_t)z);
-    v = *reinterpret_cast<const bf16x8 *>(g + w * cout + 8 * cg);
+  for (int e = 0; e < 2; e++) {
+    if (xp + e >= p.nx) continue;
+    const size_t w = (size_t)(xp + e) + (size_t)p.nx * ((size_t)y + (size_t)p.ny * (size_t)z);
+    v[e] = *reinterpret_cast<const bf16x8 *>(p.g + w * p.cout + c);
   }
-  const size_t base = (size_t)(8 * cg) * plane + ((size_t)z * ny + y) * P + xp;
+  const size_t plane = 2 * (size_t)p.g_items;
+  const size_t base = (size_t)c * plane + 2 * (size_t)t;
 #pragma unroll
-  for (int i = 0; i < 8; i++) gt[base + (size_t)i * plane] = v[i];
+  for (int i = 0; i < 8; i++)
+    *reinterpret_cast<uint32_t *>(p.gt + base + (size_t)i * plane) = pair_of(v[0][i], v[1][i]);
 }
 
-// One block per (tap, 16-channel input block, row split); its 4 waves take
-// interleaved quarters of the split's rows and are summed through LDS.
-template <int COUT>
-__global__ __launch_bounds__(256) void k_dw(int nx, int ny, int nz, int P, int rows_x, int S,
-                                            const bf16 *__restrict__ gt, const bf16 *__restrict__ xt,
-                                            float *__restrict__ part) {
+// One block per (z tap, 16-channel input block, row split); its 4 waves take
+// interleaved quarters of the split's rows and are summed through LDS.  A
+// wave keeps the sums of the nine (y, x) taps, so an A fragment (g) and the
+// three rows of X are loaded once for nine products each; with one block per
+// tap, every product loaded both of its fragments and the kernel ran at the
+// L2's rate (the 16-channel layers at 80x160x80: 446 us on average).  One wave
+// runs per SIMD, so the latency of its loads is hidden by fetching ahead: 133
+// us, and 80 us with the rows kept (NC below); the products alone are 20 us.  Each tap's sum runs over the same
+// rows in the same order whatever shares the loads.
+//
+// NC = P / 32 up to 3 (rows of 96): the three rows stay in registers and a
+// step down y loads one new row, two rows ahead (the wave's rows exceed L1,
+// so every row would come from L2 three times); NC = 0 loads the three rows
+// of a step three steps ahead.
+template <int COUT, int NC>
+__global__ __launch_bounds__(256) void k_dw(int ny, int nz, int P, int rows_x, int S, const bf16 *__restrict__ gt,
+                                            const bf16 *__restrict__ xt, float *__restrict__ part) {
   constexpr int MB = COUT / 16;
   const int ncib = rows_x / 16;
-  const int task = blockIdx.x % (27 * ncib), split = blockIdx.x / (27 * ncib);
-  const int tap = task / ncib, cib = task % ncib;
-  const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane >> 4, col = lane & 15;
+  const int task = blockIdx.x % (3 * ncib), split = blockIdx.x / (3 * ncib);
+  const int dzi = task / ncib, cib = task % ncib;
+  const int lane = threadIdx.x & 63, j = lane >> 4, col = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int rows = nz * ny;
   const int pid = split * 4 + w, np = S * 4;
   const int r0 = (int)((int64_t)rows * pid / np), r1 = (int)((int64_t)rows * (pid + 1) / np);
-  const size_t xplane = (size_t)(nz + 2) * (ny + 2) * P;
+  const int PX = P + 2 * DW_PAD;
+  const size_t xplane = (size_t)(nz + 2) * (ny + 2) * PX;
   const size_t gplane = (size_t)nz * ny * P;
-  const bf16 *xbase = xt + ((size_t)(dx + 1) * rows_x + cib * 16 + col) * xplane;
-  f32x4 acc[MB];
+  const bf16 *xb = xt + (size_t)(cib * 16 + col) * xplane + DW_PAD + 8 * j;
+  const bf16 *gb = gt + (size_t)col * gplane + 8 * j;
+  f32x4 acc[9][MB];
 #pragma unroll
-  for (int m = 0; m < MB; m++) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int r = r0; r < r1; r++) {
-    const int z = r / ny, y = r - z * ny;
-    const bf16 *xrow = xbase + ((size_t)(z + dz + 1) * (ny + 2) + (y + dy + 1)) * P;
-    const bf16 *grow = gt + ((size_t)z * ny + y) * P;
-    for (int xc = 0; xc < P; xc += 32) {
-      const bf16x8 B = *reinterpret_cast<const bf16x8 *>(xrow + xc + 8 * j);
+  for (int t = 0; t < 9; t++)
 #pragma unroll
-      for (int m = 0; m < MB; m++) {
-        const bf16x8 A = *reinterpret_cast<const bf16x8 *>(grow + (size_t)(m * 16 + col) * gplane + xc + 8 * j);
-        acc[m] = mfma16x16x32(A, B, acc[m]);
+    for (int m = 0; m < MB; m++) acc[t][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // the words beside a lane's eight x lie in the lanes 16 away, for the first
+  // and last of a step in the neighbouring step's fragment of the row (0
+  // beyond the row: x = -1, and x = P, which meets zeros of g)
+  const int from_lo = ((lane + 48) & 63) * 4, from_hi = ((lane + 16) & 63) * 4;
+  // the nine products of one step: row d's fragment c, the last word bw of
+  // the step before it and the first word aw of the step after it
+  auto multiply = [&](const bf16x8 *A, int d, const uint4 &c, uint32_t bw, uint32_t aw)
+      __attribute__((always_inline)) {
+    const uint32_t p = (uint32_t)__builtin_amdgcn_ds_bpermute(from_lo, (int)(j == 3 ? bw : c.w));
+    const uint32_t n = (uint32_t)__builtin_amdgcn_ds_bpermute(from_hi, (int)(j == 0 ? aw : c.x));
+    const uint32_t s1 = __builtin_amdgcn_alignbit(c.y, c.x, 16), s2 = __builtin_amdgcn_alignbit(c.z, c.y, 16),
+                   s3 = __builtin_amdgcn_alignbit(c.w, c.z, 16);
+    const uint4 lo = make_uint4(__builtin_amdgcn_alignbit(c.x, p, 16), s1, s2, s3);  // x - 1
+    const uint4 hi = make_uint4(s1, s2, s3, __builtin_amdgcn_alignbit(n, c.w, 16));  // x + 1
+#pragma unroll
+    for (int m = 0; m < MB; m++) {
+      acc[3 * d][m] = mfma16x16x32(A[m], __builtin_bit_cast(bf16x8, lo), acc[3 * d][m]);
+      acc[3 * d + 1][m] = mfma16x16x32(A[m], __builtin_bit_cast(bf16x8, c), acc[3 * d + 1][m]);
+      acc[3 * d + 2][m] = mfma16x16x32(A[m], __builtin_bit_cast(bf16x8, hi), acc[3 * d + 2][m]);
+    }
+  };
+  if constexpr (NC > 0) {
+    struct Row {
+      bf16x8 A[NC][MB];  // g of the row
+      uint4 c[NC];       // X two rows below its first
+    };
+    auto load_x = [&](uint4 *c, int z, int yy) __attribute__((always_inline)) {
+      const bf16 *xr = xb + ((size_t)(z + dzi) * (ny + 2) + yy) * PX;
+#pragma unroll
+      for (int q = 0; q < NC; q++) c[q] = *reinterpret_cast<const uint4 *>(xr + 32 * q);
+    };
+    constexpr int D = 2;  // rows ahead
+    Row Q[D];
+    int ar = r0, az = r0 / ny, ay = r0 - az * ny;  // the next row to fetch
+    auto fetch = [&](Row &to) __attribute__((always_inline)) {
+      if (ar >= r1) return;
+      const bf16 *gr = gb + (size_t)ar * P;
+#pragma unroll
+      for (int q = 0; q < NC; q++)
+#pragma unroll
+        for (int m = 0; m < MB; m++)
+          to.A[q][m] = *reinterpret_cast<const bf16x8 *>(gr + (size_t)m * 16 * gplane + 32 * q);
+      load_x(to.c, az, ay + 2);
+      ar++;
+      if (++ay == ny) {
+        ay = 0;
+        az++;
+      }
+    };
+    int z = az, y = ay;
+    uint4 W[3][NC];
+#pragma unroll
+    for (int u = 0; u < D; u++) fetch(Q[u]);
+    bool fresh = true;
+    for (int r = r0; r < r1; r += D) {
+#pragma unroll
+      for (int u = 0; u < D; u++) {
+        if (r + u < r1) {
+          if (fresh) {  // the first row, or the first of a plane
+            load_x(W[0], z, y);
+            load_x(W[1], z, y + 1);
+          }
+#pragma unroll
+          for (int q = 0; q < NC; q++) W[2][q] = Q[u].c[q];
+#pragma unroll
+          for (int q = 0; q < NC; q++)
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+              multiply(Q[u].A[q], d, W[d][q], q > 0 ? W[d][q > 0 ? q - 1 : 0].w : 0u,
+                       q + 1 < NC ? W[d][q + 1 < NC ? q + 1 : 0].x : 0u);
+          fetch(Q[u]);
+#pragma unroll
+          for (int q = 0; q < NC; q++) {
+            W[0][q] = W[1][q];
+            W[1][q] = W[2][q];
+          }
+          fresh = ++y == ny;
+          if (fresh) {
+            y = 0;
+            z++;
+          }
+        }
+      }
+    }
+  } else if (r0 < r1) {
+    struct Frag {
+      bf16x8 A[MB];
+      uint4 c[3];
+    };
+    int r = r0, z = r0 / ny, y = r0 - z * ny, xc = 0;  // the next step to fetch
+    constexpr int D = 4;  // fragments in flight: a load is issued three steps before its use
+    const int steps = (r1 - r0) * (P / 32);
+    Frag f[D];
+    int ahead = 0, at = 0;  // steps fetched; x of the step that multiplies
+    auto fetch = [&](Frag &to) __attribute__((always_inline)) {
+      if (ahead >= steps) return;
+      const bf16 *gr = gb + (size_t)r * P + xc;
+#pragma unroll
+      for (int m = 0; m < MB; m++) to.A[m] = *reinterpret_cast<const bf16x8 *>(gr + (size_t)m * 16 * gplane);
+      const bf16 *xr = xb + ((size_t)(z + dzi) * (ny + 2) + y) * PX + xc;
+#pragma unroll
+      for (int d = 0; d < 3; d++) to.c[d] = *reinterpret_cast<const uint4 *>(xr + d * PX);
+      ahead++;
+      xc += 32;
+      if (xc < P) return;
+      xc = 0;
+      r++;
+      if (++y == ny) {
+        y = 0;
+        z++;
+      }
+    };
+    uint32_t before[3] = {0u, 0u, 0u};  // last words of the step before
+#pragma unroll
+    for (int u = 0; u < D - 1; u++) fetch(f[u]);
+    for (int k = 0; k < steps; k += D) {
+#pragma unroll
+      for (int u = 0; u < D; u++) {
+        fetch(f[(u + D - 1) % D]);
+        if (k + u < steps) {
+          const bool first = at == 0, last = at == P - 32;
+#pragma unroll
+          for (int d = 0; d < 3; d++) {
+            multiply(f[u].A, d, f[u].c[d], first ? 0u : before[d], last ? 0u : f[(u + 1) % D].c[d].x);
+            before[d] = f[u].c[d].w;
+          }
+          at = last ? 0 : at + 32;
+        }
       }
     }
   }
   __shared__ float red[4][COUT * 16];
 #pragma unroll
-  for (int m = 0; m < MB; m++)
+  for (int t = 0; t < 9; t++) {
+    if (t) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; i++) red[w][(m * 16 + 4 * j + i) * 16 + col] = acc[m][i];
-  __syncthreads();
-  for (int e = threadIdx.x; e < COUT * 16; e += 256) {
-    const float s = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
-    const int co = e / 16, c = e % 16;
-    part[(((size_t)split * 27 + tap) * COUT + co) * rows_x + cib * 16 + c] = s;
+    for (int m = 0; m < MB; m++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) red[w][(m * 16 + 4 * j + i) * 16 + col] = acc[t][m][i];
+    __syncthreads();
+    for (int e = threadIdx.x; e < COUT * 16; e += 256) {
+      const float s = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+      const int co = e / 16, c = e % 16;
+      part[(((size_t)split * 27 + 9 * dzi + t) * COUT + co) * rows_x + cib * 16 + c] = s;
+    }
   }
 }
+// a[first] + a[first + step] + ... (count terms) in that order, U loads in flight
+template <int U>
+__device__ __forceinline__ float seq_sum32(const float *__restrict__ a, int count, size_t first, size_t step) {
+  float s = 0.0f;
+  for (int k0 = 0; k0 < count; k0 += U) {
+    float x[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) x[u] = k0 + u < count ? a[first + (size_t)(k0 + u) * step] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (k0 + u < count) s += x[u];
+  }
+  return s;
+}
+// dW from the row splits' partials (input channel fastest, as they lie), and
+// in the last block the bias gradient from its partials
 __global__ __launch_bounds__(256) void k_dw_reduce(int cout, int cin, int rows_x, int S, const float *__restrict__ part,
-                                                   float *__restrict__ dW, int accumulate) {
+                                                   const float *__restrict__ bpart, float *__restrict__ dW,
+                                                   float *__restrict__ db, int accumulate) {
+  if (blockIdx.x == gridDim.x - 1) {
+    const int c = threadIdx.x;
+    if (c >= cout) return;
+    const float s = seq_sum32<32>(bpart, BG_BLOCKS, (size_t)c, (size_t)cout);
+    db[c] = accumulate ? db[c] + s : s;
+    return;
+  }
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= cout * cin * 27) return;
-  const int t = e % 27, ci = (e / 27) % cin, co = e / (27 * cin);
-  float s = 0.0f;
-  for (int k = 0; k < S; k++) s += part[(((size_t)k * 27 + t) * cout + co) * rows_x + ci];
-  dW[e] = accumulate ? dW[e] + s : s;
+  const int ci = e % cin, co = (e / cin) % cout, t = e / (cin * cout);
+  const float s = seq_sum32<16>(part, S, ((size_t)t * cout + co) * rows_x + ci, (size_t)27 * cout * rows_x);
+  float *o = dW + ((size_t)co * cin + ci) * 27 + t;
+  *o = accumulate ? *o + s : s;
 }
-// bias gradient: db[c] = sum_v g[v][c]
-constexpr int BG_BLOCKS = 256;
+// bias gradient: partials of db[c] = sum_v g[v][c], sixteen loads in flight
 template <int C>
 __global__ __launch_bounds__(256) void k_bias_grad(uint32_t n, const bf16 *__restrict__ g, float *__restrict__ part) {
-  constexpr int VL = 256 / C;
-  const int c = threadIdx.x % C, vl = threadIdx.x / C;
+  constexpr uint32_t VL = 256 / C, STEP = BG_BLOCKS * VL, U = 16;
+  const uint32_t c = threadIdx.x % C, vl = threadIdx.x / C;
   float s = 0.0f;
-  for (uint32_t v = blockIdx.x * VL + vl; v < n; v += BG_BLOCKS * VL) s += bf(g[(size_t)v * C + c]);
+  uint32_t v = blockIdx.x * VL + vl;
+  for (; (uint64_t)v + (U - 1) * STEP < n; v += U * STEP) {
+    bf16 x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) x[u] = g[(size_t)(v + u * STEP) * C + c];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) s += bf(x[u]);
+  }
+  for (; v < n; v += STEP) s += bf(g[(size_t)v * C + c]);
   __shared__ float sh[256];
   sh[threadIdx.x] = s;
   __syncthreads();
   if (vl == 0) {
     float t = 0.0f;
-    for (int k = 0; k < VL; k++) t += sh[k * C + c];
+    for (uint32_t k = 0; k < VL; k++) t += sh[k * C + c];
     part[blockIdx.x * C + c] = t;
   }
 }
-__global__ __launch_bounds__(64) void k_bias_reduce(int C, const float *__restrict__ part, float *__restrict__ db,
-                                                    int accumulate) {
-  const int c = threadIdx.x;
-  if (c >= C) return;
-  float s = 0.0f;
-  for (int b = 0; b < BG_BLOCKS; b++) s += part[b * C + c];
-  db[c] = accumulate ? db[c] + s : s;
-}
-static void launch_bias_grad(uint32_t n, int c, const bf16 *g, float *part, float *db, bool acc, hipStream_t s) {
-  if (c == 16) k_bias_grad<16><<<BG_BLOCKS, 256, 0, s>>>(n, g, part);
-  else if (c == 32) k_bias_grad<32><<<BG_BLOCKS, 256, 0, s>>>(n, g, part);
-  else k_bias_grad<64><<<BG_BLOCKS, 256, 0, s>>>(n, g, part);
-  k_bias_reduce<<<1, 64, 0, s>>>(c, part, db, acc ? 1 : 0);
-}
 
-static void launch_dw_core(const G3 &g, int cout, int cin_real, const DwPlan &d, const bf16 *gt, const bf16 *xt,
-                           float *part, float *dW, bool acc, hipStream_t s) {
-  const unsigned nb = (unsigned)(27 * (d.rows_x / 16) * d.S);
-  if (cout == 16) k_dw<16><<<nb, 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part);
-  else if (cout == 32) k_dw<32><<<nb, 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part);
-  else k_dw<64><<<nb, 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part);
-  k_dw_reduce<<<nblk((uint64_t)cout * cin_real * 27), 256, 0, s>>>(cout, cin_real, d.rows_x, d.S, part, dW, acc ? 1 : 0);
+template <int COUT>
+static void launch_dw(unsigned nb, const G3 &g, const DwPlan &d, const bf16 *gt, const bf16 *xt, float *part,
+                      hipStream_t s) {
+  switch (d.P) {
+    case 32: k_dw<COUT, 1><<<nb, 256, 0, s>>>(g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part); break;
+    case 64: k_dw<COUT, 2><<<nb, 256, 0, s>>>(g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part); break;
+    case 96:
+      if constexpr (COUT < 64) {  // 64 channels and three steps do not fit the registers
+        k_dw<COUT, 3><<<nb, 256, 0, s>>>(g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part);
+        break;
+      }
+      [[fallthrough]];
+    default: k_dw<COUT, 0><<<nb, 256, 0, s>>>(g.ny, g.nz, d.P, d.rows_x, d.S, gt, xt, part); break;
+  }
 }
-
+// weight and bias gradients of one layer (cb = 2: the first)
+static void launch_dw_layer(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b,
+                            const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW, float *db, bool accumulate,
+                            hipStream_t s) {
+  const DwPlan d = dw_plan(g, c);
+  TransArgs p;
+  p.nx = g.nx; p.ny = g.ny; p.nz = g.nz;
+  p.P = d.P;
+  p.anx = ga.nx; p.any = ga.ny;
+  p.ca = c.ca; p.cb = c.cb; p.cout = c.cout;
+  p.a = a; p.b = b; p.g = gpre;
+  p.xt = xt; p.gt = gt;
+  p.xgroups = d.rows_x / 8;
+  p.dxp = make_fastdiv((uint32_t)(d.P + 2 * DW_PAD) / 2);
+  p.dxy = make_fastdiv((uint32_t)g.ny + 2);
+  p.dgp = make_fastdiv((uint32_t)d.P / 2);
+  p.dgy = make_fastdiv((uint32_t)g.ny);
+  p.x_items = (uint32_t)(g.nz + 2) * (uint32_t)(g.ny + 2) * p.dxp.d;
+  p.g_items = (uint32_t)g.nz * (uint32_t)g.ny * p.dgp.d;
+  k_to_t<<<dim3(nblk(p.x_items > p.g_items ? p.x_items : p.g_items), p.xgroups + c.cout / 8), 256, 0, s>>>(p);
+  const unsigned nb = (unsigned)(3 * (d.rows_x / 16) * d.S);
+  float *bpart = part + dw_bias_at(d, c.cout);
+  if (c.cout == 16) {
+    launch_dw<16>(nb, g, d, gt, xt, part, s);
+    k_bias_grad<16><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
+  } else if (c.cout == 32) {
+    launch_dw<32>(nb, g, d, gt, xt, part, s);
+    k_bias_grad<32><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
+  } else {
+    launch_dw<64>(nb, g, d, gt, xt, part, s);
+    k_bias_grad<64><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
+  }
+  k_dw_reduce<<<nblk((uint64_t)c.cout * c.cin() * 27) + 1, 256, 0, s>>>(c.cout, c.cin(), d.rows_x, d.S, part, bpart, dW,
+                                                                        db, accumulate ? 1 : 0);
+}
 void launch_conv_dw(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre,
                     bf16 *xt, bf16 *gt, float *part, float *dW, float *db, bool accumulate, hipStream_t s) {
-  const DwPlan d = dw_plan(g, c);
-  const size_t xplane = (size_t)(g.nz + 2) * (g.ny + 2) * d.P;
-  k_to_xt<<<nblk(3 * (size_t)(c.cin() / 8) * xplane), 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, ga.nx, ga.ny, a, c.ca, b,
-                                                                    c.cb, d.rows_x, xt);
-  const size_t gplane = (size_t)g.nz * g.ny * d.P;
-  k_to_gt<<<nblk((size_t)(c.cout / 8) * gplane), 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, c.cout, gpre, gt);
-  launch_dw_core(g, c.cout, c.cin(), d, gt, xt, part, dW, accumulate, s);
-  launch_bias_grad(g.n(), c.cout, gpre, part, db, accumulate, s);
+  launch_dw_layer(g, c, a, ga, b, gpre, xt, gt, part, dW, db, accumulate, s);
 }
-
 void launch_conv_in_dw(const G3 &g, const bf16 *x0, const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW,
                        float *db, bool accumulate, hipStream_t s) {
-  const ConvSpec c{0, 2, 16};
-  const DwPlan d = dw_plan(g, c);
-  const size_t xplane = (size_t)(g.nz + 2) * (g.ny + 2) * d.P;
-  k_to_xt_in<<<nblk(3 * xplane), 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, x0, xt);
-  const size_t gplane = (size_t)g.nz * g.ny * d.P;
-  k_to_gt<<<nblk(2 * gplane), 256, 0, s>>>(g.nx, g.ny, g.nz, d.P, 16, gpre, gt);
-  launch_dw_core(g, 16, 2, d, gt, xt, part, dW, accumulate, s);
-  launch_bias_grad(g.n(), 16, gpre, part, db, accumulate, s);
+  launch_dw_layer(g, ConvSpec{0, 2, 16}, nullptr, g, x0, gpre, xt, gt, part, dW, db, accumulate, s);
 }
 
 // ------------------------------------------------------------ solver transforms
@@ -856,8 +1062,8 @@ __global__ __launch_bounds__(256) void k_loss(uint32_t n, const float *__restric
     part[LOSS_BLOCKS + blockIdx.x] = b;
   }
 }
-__global__ __launch_bounds__(256) void k_loss_final(double *__restrict__ part) {
-  // part[2*NB], part[2*NB+1] = totals (fixed order)
+__global__ __launch_bounds__(256) void k_loss_final(double *__restrict__ part, float *__restrict__ rec) {
+  // part[2*NB], part[2*NB+1] = totals (fixed order); rec (if not null) their ratio
   __shared__ double sh[256 / 64];
   double a = 0.0, b = 0.0;
   for (int i = threadIdx.x; i < LOSS_BLOCKS; i += 256) {
@@ -869,19 +1075,13 @@ __global__ __launch_bounds__(256) void k_loss_final(double *__restrict__ part) {
   if (threadIdx.x == 0) {
     part[2 * LOSS_BLOCKS] = a;
     part[2 * LOSS_BLOCKS + 1] = b;
-  }
-}
-__global__ __launch_bounds__(64) void k_loss_record(const double *__restrict__ part, float *__restrict__ rec) {
-  if (threadIdx.x == 0) {
-    const double d = part[2 * LOSS_BLOCKS + 1];
-    rec[0] = (float)(d > 0.0 ? part[2 * LOSS_BLOCKS] / d : part[2 * LOSS_BLOCKS]);
+    if (rec) rec[0] = (float)(b > 0.0 ? a / b : a);
   }
 }
 void launch_loss(const G3 &g, const float *y, const float *t, const bf16 *x0, double *part, float *rec,
                  hipStream_t s) {
   k_loss<<<LOSS_BLOCKS, 256, 0, s>>>(g.n(), y, t, x0, part);
-  k_loss_final<<<1, 256, 0, s>>>(part);
-  if (rec) k_loss_record<<<1, 64, 0, s>>>(part, rec);
+  k_loss_final<<<1, 256, 0, s>>>(part, rec);
 }
 __global__ __launch_bounds__(256) void k_loss_grad(uint32_t n, const float *__restrict__ y, const float *__restrict__ t,
                                                    const bf16 *__restrict__ x0, const double *__restrict__ den,

@@ -151,10 +151,13 @@ int work_alloc(Work &W, const G3 &g, bool train) {
 
 void repack(PyroNet *N) {
   launch_pack_conv_in(N->params + N->w0a, N->w0a_bf, N->stream);
+  PackJob jobs[2 * NCONV];
+  static_assert(2 * NCONV <= PACK_MAX, "one launch packs every conv");
   for (int l = 0; l < NCONV; l++) {
-    launch_pack_conv(N->params + N->w[l], kSpec[l], false, N->wp[l], N->stream);
-    launch_pack_conv(N->params + N->w[l], kSpec[l], true, N->wpt[l], N->stream);
+    jobs[2 * l] = {N->params + N->w[l], N->wp[l], kSpec[l], false};
+    jobs[2 * l + 1] = {N->params + N->w[l], N->wpt[l], kSpec[l], true};
   }
+  launch_pack_convs(jobs, 2 * NCONV, N->stream);
 }
 
 void forward(PyroNet *N, Work &W, const bf16 *x0) {

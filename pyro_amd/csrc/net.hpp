@@ -49,6 +49,15 @@ struct ConvSpec {
 int conv_a_chunk(int cout);
 int conv_groups(int ca, int cb, int cout);
 void launch_pack_conv(const float *W, const ConvSpec &c, bool transposed, bf16 *wp, hipStream_t s);
+// the same for up to PACK_MAX copies in one launch
+constexpr int PACK_MAX = 14;
+struct PackJob {
+  const float *W;
+  bf16 *wp;
+  ConvSpec c;
+  bool transposed;
+};
+void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s);
 void launch_pack_bf16(const float *w, uint32_t n, bf16 *out, hipStream_t s);
 
 // out[v][0..cout) = act(bias + sum_taps W * in), in = [up(a), b]; false (and
