@@ -37,10 +37,12 @@ __device__ __forceinline__ float spongeSide(const Params *__restrict__ P, const 
   int e = x < g.nx - 1 - x ? x : g.nx - 1 - x;
   int e2 = z < g.nz - 1 - z ? z : g.nz - 1 - z;
   if (e2 < e) e = e2;
+  if (P->sponge > 0.0f && (float)e >= P->sponge) return 0.0f;  // smoothstep is exactly 1 there
   return 1.0f - smoothstep_(0.0f, P->sponge, (float)e);
 }
 __device__ __forceinline__ float spongeTop(const Params *__restrict__ P, const Geo &g, int y) {
   float h = (float)g.ny;
+  if (P->sponge > 1.0f && (float)y <= h - 1.5f * P->sponge) return 0.0f;  // smoothstep is exactly 0 there
   return smoothstep_(h - 1.5f * P->sponge, h - 1.0f, (float)y);
 }
 
@@ -62,6 +64,8 @@ constexpr int FC_R = (FC_N + NT - 1) / NT, FW_R = (FW_N + NT - 1) / NT;
 // smoke and curl w; m points at the cell's |curl| in the |curl| tile, whose
 // entries m[+-1], m[+-FW_X], m[+-FW_X FW_Y] are the clamped neighbours.
 __device__ __forceinline__ float confine_gate(const Params *__restrict__ P, float T, float smoke) {
+  // each smoothstep is exactly 0 up to its lower edge (both arguments there: a closed gate)
+  if (T <= P->vort_t && smoke <= 0.0f) return 0.0f;
   return fmax_(smoothstep_(P->vort_t, P->vort_t + 500.0f, T), 0.35f * smoothstep_(0.0f, 2e-4f, smoke));
 }
 __device__ __forceinline__ void confine_tile(const Params *__restrict__ P, float gate, float4 w, const float *m,
@@ -187,6 +191,17 @@ __global__ __launch_bounds__(NT) void k_forces(const Params *__restrict__ P, Geo
   const float dt = P->dt;
   const int cb = (x - x0 + 1) + FC_X * ((y - y0 + 1) + FC_Y * (z - z0 + 1));
   const bool ib = sc[cb] & 1u;
+  // wind relaxation, the same for the two horizontal components: sponge and
+  // hot-gas factor at the face's own cell.  Below 350 K and from 900 K on the
+  // hot factor is exactly 0 or 1.
+  const int cx = clampi(x, 0, g.nx - 1), cy = clampi(y, 0, g.ny - 1), cz = clampi(z, 0, g.nz - 1);
+  const float ss = spongeSide(P, g, cx, cz);
+  float Tl = P->t0;
+  if (ib) Tl = st[cb];
+  float hot = Tl <= 350.0f ? 0.0f : 1.0f;
+  if (!(Tl <= 350.0f || Tl >= 900.0f)) hot = smoothstep_(350.0f, 900.0f, Tl);
+  const float kr = P->wind_relax * (1.0f - 0.85f * hot) + 8.0f * ss;
+  const float relax = 1.0f - pexp(-kr * dt);
   // the face's own cell (x, y, z) is the b side of all three components
   const float cbx = sf[0][cb], cby = sf[1][cb], cbz = sf[2][cb];
 #pragma unroll
@@ -213,19 +228,14 @@ __global__ __launch_bounds__(NT) void k_forces(const Params *__restrict__ P, Geo
     if (ib) {
       fcx += cbx; fcy += cby; fcz += cbz; n += 1.0f;
     }
-    if (n > 0.0f) f += (k == 0 ? fcx : (k == 1 ? fcy : fcz)) / n;
+    // the mean of one or two cells (x 0.5 is x / 2, correctly rounded either way)
+    if (n > 0.0f) f += (k == 0 ? fcx : (k == 1 ? fcy : fcz)) * (n == 2.0f ? 0.5f : 1.0f);
     float *C = k == 0 ? U : (k == 1 ? V : W);
     float u = uvw[k];
     u += f * dt;
-    int cx = clampi(x, 0, g.nx - 1), cy = clampi(y, 0, g.ny - 1), cz = clampi(z, 0, g.nz - 1);
-    float ss = spongeSide(P, g, cx, cz);
     if (k != 1) {
-      float Tl = P->t0;
-      if (ib) Tl = st[cb];
-      float hot = smoothstep_(350.0f, 900.0f, Tl);
-      float kr = P->wind_relax * (1.0f - 0.85f * hot) + 8.0f * ss;
       float wv = k == 0 ? P->wind_x : P->wind_z;
-      u = mixf_(u, wv, 1.0f - pexp(-kr * dt));
+      u = mixf_(u, wv, relax);
     } else {
       float stp = spongeTop(P, g, cy);
       if (stp > 0.0f) u = mixf_(u, fmax_(u, 0.0f), 1.0f - pexp(-8.0f * stp * dt));
