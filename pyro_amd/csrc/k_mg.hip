@@ -608,7 +608,8 @@ __global__ __launch_bounds__(SW_NT) void k_mg_sweep(LvArgs a, int ntx, int nty, 
   const int sy = a.d0, sz = a.d0 * a.d1;
   const RB rbb = rb_of(b, VEC ? a.n * 4u : 0u);
   if (VEC) {
-    const RB rp = rb_of(pin, a.n * 4u), rcd = rb_of(nc, a.n);
+    // pin null: phi is 0 (an empty resource reads 0)
+    const RB rp = rb_of(pin, pin ? a.n * 4u : 0u), rcd = rb_of(nc, a.n);
     float4 pv[4];
     uint32_t cv[4];
     {
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(SW_NT) void k_mg_sweep(LvArgs a, int ntx, int nty, 
       const bool in = gx >= 0 && gx < a.d0 && gy >= 0 && gy < a.d1 && gz >= 0 && gz < a.d2;
       const int g = in ? gx + sy * gy + sz * gz : 0;
       const uint8_t c = nc[g];
-      const float p = pin[g];
+      const float p = pin ? pin[g] : 0.0f;
       if (i < SW_PN) {
         sp[i] = (in && !(c & NC_SOLID)) ? p : 0.0f;
         sc[i] = in ? c : NC_NONE;
@@ -732,7 +733,7 @@ __global__ __launch_bounds__(SW_NT) void k_mg_sweep(LvArgs a, int ntx, int nty, 
       const int pi = ((lz + 2) * SW_PY + (ly + 2)) * SW_PX + 4 + 4 * q;
       float4 v = *reinterpret_cast<const float4 *>(sp + pi);
       const uint32_t cv = *reinterpret_cast<const uint32_t *>(sc + pi);
-      if (cv & 0x80808080u) {  // solid cells keep their phi (zeroed only in LDS)
+      if ((cv & 0x80808080u) && pin) {  // solid cells keep their phi (zeroed only in LDS)
         const float4 o = *reinterpret_cast<const float4 *>(pin + g);
         if (cv & 0x80u) v.x = o.x;
         if (cv & 0x8000u) v.y = o.y;
@@ -749,7 +750,7 @@ __global__ __launch_bounds__(SW_NT) void k_mg_sweep(LvArgs a, int ntx, int nty, 
       if (gx >= a.d0 || gy >= a.d1 || gz >= a.d2) continue;
       const int g = gx + sy * gy + sz * gz;
       const int pi = ((lz + 2) * SW_PY + (ly + 2)) * SW_PX + 4 + lx;
-      pout[g] = (sc[pi] & NC_SOLID) ? pin[g] : sp[pi];
+      pout[g] = (sc[pi] & NC_SOLID) && pin ? pin[g] : sp[pi];
     }
   }
 }
@@ -1783,16 +1784,17 @@ void launch_mg_resid(const MgLevel &L, StatParts *st, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- V-cycle
-void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s) {
-  auto sweeps = [&](const MgLevel &L, bool fine) {
-    launch_mg_sweep(L, L.phi, L.tmp, 1.0f, s, fine);
+void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero) {
+  auto sweeps = [&](const MgLevel &L, bool fine, bool zero = false) {
+    launch_mg_sweep(L, zero ? nullptr : L.phi, L.tmp, 1.0f, s, fine);
     launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, fine);
   };
   // the levels from t on run in one launch where they fit
   int t = nl - 1;
   while (t > 0 && tail_fits(lv, t - 1, nl)) t--;
+  if (from_zero && t == 0) launch_zero32(lv[0].n, lv[0].phi, s);  // the tail reads phi
   for (int l = 0; l < t; l++) {
-    sweeps(lv[l], l == 0);
+    sweeps(lv[l], l == 0, from_zero && l == 0);
     launch_mg_restrict(lv[l], lv[l + 1], s);
   }
   if (t < nl - 1) launch_mg_tail(lv, t, nl, coarse_iters, 1.6f, s);

@@ -53,6 +53,45 @@ __device__ __forceinline__ double apply_at(const Op64 &o, const uint8_t *__restr
   return (sum - cnt * xc) * o.ih2;
 }
 
+// The operator at cells i and i + 1 of a row of even length (i even): the
+// rows' values come as 16-byte pairs, so two cells cost seven loads instead
+// of fourteen (the kernels with one cell a thread were bound by their loads'
+// L1 accesses, not by HBM: 172 us for apply_dots at 256^3, 2.5 TB/s).
+__device__ __forceinline__ double2 ld2(const double *__restrict__ x, uint32_t i) {
+  return *reinterpret_cast<const double2 *>(x + i);
+}
+__device__ __forceinline__ void apply_pair(const Op64 &o, const uint8_t *__restrict__ nm,
+                                           const uint8_t *__restrict__ nc, const double *__restrict__ x, uint32_t i,
+                                           double2 &xc, double2 &y, bool &solid0, bool &solid1) {
+  const uint32_t sy = (uint32_t)o.d0, sz = (uint32_t)o.d0 * (uint32_t)o.d1;
+  const uint32_t codes = *reinterpret_cast<const uint16_t *>(nc + i);
+  const uint32_t masks = *reinterpret_cast<const uint16_t *>(nm + i);
+  xc = ld2(x, i);
+  // a row outside the arrays reads the cells themselves and is masked
+  const double2 yp = ld2(x, i + sy < o.n ? i + sy : i), ym = ld2(x, i >= sy ? i - sy : i);
+  const double2 zp = ld2(x, i + sz < o.n ? i + sz : i), zm = ld2(x, i >= sz ? i - sz : i);
+  const double xm = x[i > 0 ? i - 1 : i], xp = x[i + 2 < o.n ? i + 2 : i];
+  auto one = [&](uint32_t code, uint32_t m, double c, double v0, double v1, double v2, double v3, double v4,
+                 double v5) {
+    double sum = 0.0;
+    sum += (m & 1u) ? v0 : 0.0;
+    sum += (m & 2u) ? v1 : 0.0;
+    sum += (m & 4u) ? v2 : 0.0;
+    sum += (m & 8u) ? v3 : 0.0;
+    sum += (m & 16u) ? v4 : 0.0;
+    sum += (m & 32u) ? v5 : 0.0;
+    const double cnt = (double)((code & 7u) + ((code >> 3) & 7u));
+    return (code & 0x80u) ? 0.0 : (sum - cnt * c) * o.ih2;
+  };
+  y.x = one(codes & 0xffu, masks & 0xffu, xc.x, xc.y, xm, yp.x, ym.x, zp.x, zm.x);
+  y.y = one(codes >> 8, masks >> 8, xc.y, xp, xc.x, yp.y, ym.y, zp.y, zm.y);
+  solid0 = (codes & 0x80u) != 0;
+  solid1 = (codes & 0x8000u) != 0;
+}
+// Blocks of 256 threads with two cells each take tiles 2 b and 2 b + 1 of the
+// 256-cell tiles of the one-cell kernels.
+static int nblocks2(uint32_t n) { return (nblocks(n) + 1) / 2; }
+
 // r = b - A x  (fluid cells; 0 on solids)
 __global__ __launch_bounds__(NT) void k_resid64(Op64 o, const uint8_t *__restrict__ nm, const uint8_t *__restrict__ nc,
                                                  const double *__restrict__ x, const double *__restrict__ b,
@@ -61,6 +100,17 @@ __global__ __launch_bounds__(NT) void k_resid64(Op64 o, const uint8_t *__restric
   if (i >= o.n) return;
   r[i] = (nc[i] & 0x80) ? 0.0 : b[i] - apply_at(o, nm, nc, x, i);
 }
+__global__ __launch_bounds__(NT) void k_resid64_pair(Op64 o, const uint8_t *__restrict__ nm,
+                                                      const uint8_t *__restrict__ nc, const double *__restrict__ x,
+                                                      const double *__restrict__ b, double *__restrict__ r) {
+  const uint32_t i = 2u * ((uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x);
+  if (i >= o.n) return;
+  const double2 bv = ld2(b, i);
+  double2 c, y;
+  bool s0, s1;
+  apply_pair(o, nm, nc, x, i, c, y, s0, s1);
+  *reinterpret_cast<double2 *>(r + i) = make_double2(s0 ? 0.0 : bv.x - y.x, s1 ? 0.0 : bv.y - y.y);
+}
 // y = A x
 __global__ __launch_bounds__(NT) void k_apply64(Op64 o, const uint8_t *__restrict__ nm, const uint8_t *__restrict__ nc,
                                                  const double *__restrict__ x, double *__restrict__ y) {
@@ -68,12 +118,27 @@ __global__ __launch_bounds__(NT) void k_apply64(Op64 o, const uint8_t *__restric
   if (i >= o.n) return;
   y[i] = apply_at(o, nm, nc, x, i);
 }
+__global__ __launch_bounds__(NT) void k_apply64_pair(Op64 o, const uint8_t *__restrict__ nm,
+                                                      const uint8_t *__restrict__ nc, const double *__restrict__ x,
+                                                      double *__restrict__ y) {
+  const uint32_t i = 2u * ((uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x);
+  if (i >= o.n) return;
+  double2 c, v;
+  bool s0, s1;
+  apply_pair(o, nm, nc, x, i, c, v, s0, s1);
+  *reinterpret_cast<double2 *>(y + i) = v;
+}
 
+// Two cells a thread where the rows' length is even (a pair then lies in one
+// row and every row starts on 16 bytes).
+static bool pairs_of(const MgLevel &L) { return L.d[0] % 2 == 0; }
 void launch_resid64(const MgLevel &L, const double *x, const double *b, double *r, hipStream_t s) {
-  k_resid64<<<nblocks(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, b, r);
+  if (pairs_of(L)) k_resid64_pair<<<nblocks2(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, b, r);
+  else k_resid64<<<nblocks(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, b, r);
 }
 void launch_apply64(const MgLevel &L, const double *x, double *y, hipStream_t s) {
-  k_apply64<<<nblocks(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, y);
+  if (pairs_of(L)) k_apply64_pair<<<nblocks2(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, y);
+  else k_apply64<<<nblocks(L.n), NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, y);
 }
 
 // Up to 4 dot products at once: out[k] = sum_i a_k[i] * b_k[i].
@@ -181,9 +246,10 @@ __global__ __launch_bounds__(NT) void k_zero_u8(uint32_t n, uint8_t *a) {
 }
 
 // ---------------------------------------------------------------- fused CG steps
-// Per-block FP64 partial sums go to part[k * nb + block] (nb = blocks of the
-// launch); k_sum_final adds them in a fixed order into dev[slot + k], so the
-// scalars of the iteration stay on the device and every run is bit-reproducible.
+// Per-block FP64 partial sums of 256 cells go to part[k * nb + block] (nb
+// blocks of 256 cells); k_sum_final adds them in a fixed order into dev[slot +
+// k], so the scalars of the iteration stay on the device and every run is
+// bit-reproducible.
 __global__ __launch_bounds__(1024) void k_sum_final(const double *__restrict__ part, int nb, int k, double *dev,
                                                     int slot) {
   __shared__ double sh[1024];
@@ -198,6 +264,31 @@ __global__ __launch_bounds__(1024) void k_sum_final(const double *__restrict__ p
     if (threadIdx.x == 0) dev[slot + q] = sh[0];
     __syncthreads();
   }
+}
+
+// Sums of the two 256-cell tiles of a block with two cells a thread (cells 2 t
+// and 2 t + 1), each in the order block_sum adds one cell a thread: the
+// butterfly over 64 cells is one over 32 lanes on both halves of the pairs,
+// then the two halves; the four 64-cell sums of a tile are added in order.
+// Threads 0 and 1 return the tiles' sums.
+__device__ __forceinline__ double pair_sum(double v0, double v1, double *sh) {
+  for (int o = 16; o > 0; o >>= 1) {
+    v0 += __shfl_xor(v0, o, 64);
+    v1 += __shfl_xor(v1, o, 64);
+  }
+  const double v = v0 + v1;
+  __syncthreads();
+  if ((threadIdx.x & 31) == 0) sh[threadIdx.x >> 5] = v;
+  __syncthreads();
+  double r = 0.0;
+  if (threadIdx.x < 2)
+    for (int q = 0; q < 4; q++) r += sh[4 * threadIdx.x + q];
+  return r;
+}
+// The block of a launch of nb blocks that xcd_tile gives tile t.
+__device__ __forceinline__ int xcd_block(int t, int nb) {
+  const int q = nb >> 3;
+  return t >= (q << 3) ? t : (t % q) * 8 + t / q;
 }
 
 // q = A p with partials of p.q and p.r
@@ -220,25 +311,130 @@ __global__ __launch_bounds__(NT) void k_apply_dots(Op64 o, const uint8_t *__rest
     part[gridDim.x + blockIdx.x] = b;
   }
 }
-// alpha = dev[1] / dev[0]; x += alpha p; r -= alpha q; partials of r.r
-__global__ __launch_bounds__(NT) void k_update_rr(uint32_t n, const double *__restrict__ dev,
-                                                   const double *__restrict__ p, const double *__restrict__ q,
-                                                   double *__restrict__ x, double *__restrict__ r,
-                                                   double *__restrict__ part) {
-  const double alpha = dev[0] != 0.0 ? dev[1] / dev[0] : 0.0;
-  const uint32_t i = blockIdx.x * NT + threadIdx.x;
-  double rr = 0.0;
-  if (i < n) {
-    x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    rr = ri * ri;
+__global__ __launch_bounds__(NT) void k_apply_dots_pair(Op64 o, int nb, const uint8_t *__restrict__ nm,
+                                                         const uint8_t *__restrict__ nc, const double *__restrict__ p,
+                                                         const double *__restrict__ r, double *__restrict__ q,
+                                                         double *__restrict__ part) {
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t i = 2u * ((uint32_t)tile * NT + threadIdx.x);
+  double2 pq = make_double2(0.0, 0.0), pr = pq;
+  if (i < o.n) {
+    const double2 rv = ld2(r, i);
+    double2 c, y;
+    bool s0, s1;
+    apply_pair(o, nm, nc, p, i, c, y, s0, s1);
+    *reinterpret_cast<double2 *>(q + i) = y;
+    pq = make_double2(c.x * y.x, c.y * y.y);
+    pr = make_double2(c.x * rv.x, c.y * rv.y);
   }
-  __shared__ double sh[NT / 64];
-  const double a = block_sum<NT>(rr, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = a;
+  __shared__ double sh[NT / 32];
+  const double a = pair_sum(pq.x, pq.y, sh);
+  const double b = pair_sum(pr.x, pr.y, sh);
+  const int t = 2 * tile + (int)threadIdx.x;
+  if (threadIdx.x < 2 && t < nb) {
+    const int bid = xcd_block(t, nb);
+    part[bid] = a;
+    part[nb + bid] = b;
+  }
 }
-// preconditioner input: b32 = (float)r, phi = 0
+// alpha = dev[1] / dev[0]; r -= alpha q; partials of r.r; b32 = (float)r (the
+// next V-cycle's right-hand side) where given.  x += alpha p waits for the
+// step of p (k_step_p), which reads p anyway.
+__device__ __forceinline__ double cg_alpha(const double *__restrict__ dev) {
+  return dev[0] != 0.0 ? dev[1] / dev[0] : 0.0;
+}
+template <bool PAIR>
+__global__ __launch_bounds__(NT) void k_update_rr(uint32_t n, int nb, const double *__restrict__ dev,
+                                                   const double *__restrict__ q, double *__restrict__ r,
+                                                   float *__restrict__ b32, double *__restrict__ part) {
+  const double alpha = cg_alpha(dev);
+  __shared__ double sh[NT / 32];
+  if constexpr (PAIR) {
+    const uint32_t i = 2u * (blockIdx.x * NT + threadIdx.x);
+    double2 rr = make_double2(0.0, 0.0);
+    if (i < n) {
+      const double2 rv = ld2(r, i), qv = ld2(q, i);
+      const double2 ri = make_double2(rv.x - alpha * qv.x, rv.y - alpha * qv.y);
+      *reinterpret_cast<double2 *>(r + i) = ri;
+      if (b32) *reinterpret_cast<float2 *>(b32 + i) = make_float2((float)ri.x, (float)ri.y);
+      rr = make_double2(ri.x * ri.x, ri.y * ri.y);
+    }
+    const double a = pair_sum(rr.x, rr.y, sh);
+    const int t = 2 * (int)blockIdx.x + (int)threadIdx.x;
+    if (threadIdx.x < 2 && t < nb) part[t] = a;
+  } else {
+    const uint32_t i = blockIdx.x * NT + threadIdx.x;
+    double rr = 0.0;
+    if (i < n) {
+      const double ri = r[i] - alpha * q[i];
+      r[i] = ri;
+      if (b32) b32[i] = (float)ri;
+      rr = ri * ri;
+    }
+    const double a = block_sum<NT>(rr, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = a;
+  }
+}
+// partials of z.q for z = (double)phi
+template <bool PAIR>
+__global__ __launch_bounds__(NT) void k_dot_zq(uint32_t n, int nb, const float *__restrict__ phi,
+                                                const double *__restrict__ q, double *__restrict__ part) {
+  __shared__ double sh[NT / 32];
+  if constexpr (PAIR) {
+    const uint32_t i = 2u * (blockIdx.x * NT + threadIdx.x);
+    double2 zq = make_double2(0.0, 0.0);
+    if (i < n) {
+      const float2 z = *reinterpret_cast<const float2 *>(phi + i);
+      const double2 qv = ld2(q, i);
+      zq = make_double2((double)z.x * qv.x, (double)z.y * qv.y);
+    }
+    const double a = pair_sum(zq.x, zq.y, sh);
+    const int t = 2 * (int)blockIdx.x + (int)threadIdx.x;
+    if (threadIdx.x < 2 && t < nb) part[t] = a;
+  } else {
+    const uint32_t i = blockIdx.x * NT + threadIdx.x;
+    const double a = block_sum<NT>(i < n ? (double)phi[i] * q[i] : 0.0, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = a;
+  }
+}
+// An iteration moves p, q, r, x and z: with x += alpha p taken in the step of
+// p (which reads p anyway), z read as the V-cycle's FP32 phi and (float)r
+// written with r, 102 bytes a cell instead of 134: bonfire at 10 cm 151 -> 110
+// us an iteration in these kernels.
+// x += alpha p, then p = z + beta p with beta = -dev[3] / dev[0]; z = (double)phi, or z64
+template <bool PAIR, bool Z64>
+__global__ __launch_bounds__(NT) void k_step_p(uint32_t n, const double *__restrict__ dev,
+                                                const float *__restrict__ phi, const double *__restrict__ z64,
+                                                double *__restrict__ p, double *__restrict__ x) {
+  const double alpha = cg_alpha(dev), beta = dev[0] != 0.0 ? -dev[3] / dev[0] : 0.0;
+  if constexpr (PAIR) {
+    const uint32_t i = 2u * (blockIdx.x * NT + threadIdx.x);
+    if (i >= n) return;
+    const double2 pv = ld2(p, i), xv = ld2(x, i);
+    double2 z;
+    if (Z64) {
+      z = ld2(z64, i);
+    } else {
+      const float2 f = *reinterpret_cast<const float2 *>(phi + i);
+      z = make_double2((double)f.x, (double)f.y);
+    }
+    *reinterpret_cast<double2 *>(x + i) = make_double2(xv.x + alpha * pv.x, xv.y + alpha * pv.y);
+    *reinterpret_cast<double2 *>(p + i) = make_double2(z.x + beta * pv.x, z.y + beta * pv.y);
+  } else {
+    const uint32_t i = blockIdx.x * NT + threadIdx.x;
+    if (i >= n) return;
+    const double pv = p[i], z = Z64 ? z64[i] : (double)phi[i];
+    x[i] += alpha * pv;
+    p[i] = z + beta * pv;
+  }
+}
+// x += alpha p alone: the last iteration's
+__global__ __launch_bounds__(NT) void k_step_x(uint32_t n, const double *__restrict__ dev,
+                                                const double *__restrict__ p, double *__restrict__ x) {
+  const uint32_t i = blockIdx.x * NT + threadIdx.x;
+  if (i < n) x[i] += cg_alpha(dev) * p[i];
+}
+// preconditioner input: b32 = (float)r
 __global__ __launch_bounds__(NT) void k_to_f32_zero(uint32_t n, const double *__restrict__ r, float *__restrict__ b,
                                                      float *__restrict__ phi) {
   const uint32_t i = blockIdx.x * NT + threadIdx.x;
@@ -247,75 +443,85 @@ __global__ __launch_bounds__(NT) void k_to_f32_zero(uint32_t n, const double *__
     phi[i] = 0.0f;
   }
 }
-// z = (double)phi with partials of z.q
-__global__ __launch_bounds__(NT) void k_to_f64_dot(uint32_t n, const float *__restrict__ phi,
-                                                    const double *__restrict__ q, double *__restrict__ z,
-                                                    double *__restrict__ part) {
-  const uint32_t i = blockIdx.x * NT + threadIdx.x;
-  double zq = 0.0;
-  if (i < n) {
-    const double zi = (double)phi[i];
-    z[i] = zi;
-    zq = zi * q[i];
-  }
-  __shared__ double sh[NT / 64];
-  const double a = block_sum<NT>(zq, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = a;
-}
-// p = z + beta p with beta = -dev[3] / dev[0]
-__global__ __launch_bounds__(NT) void k_xpby_dev(uint32_t n, const double *__restrict__ z,
-                                                  const double *__restrict__ dev, double *__restrict__ p) {
-  const double beta = dev[0] != 0.0 ? -dev[3] / dev[0] : 0.0;
-  const uint32_t i = blockIdx.x * NT + threadIdx.x;
-  if (i < n) p[i] = z[i] + beta * p[i];
-}
 
-// r = b - A x with partials of r.r
+// partials of r.r for r = b - A x; r32 = (float)r where given
 __global__ __launch_bounds__(NT) void k_resid_rr(Op64 o, const uint8_t *__restrict__ nm, const uint8_t *__restrict__ nc,
                                                   const double *__restrict__ x, const double *__restrict__ b,
-                                                  double *__restrict__ r, double *__restrict__ part) {
+                                                  float *__restrict__ r32, double *__restrict__ part) {
   const uint32_t i = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
   double rr = 0.0;
   if (i < o.n) {
     const double ri = (nc[i] & 0x80) ? 0.0 : b[i] - apply_at(o, nm, nc, x, i);
-    r[i] = ri;
+    if (r32) r32[i] = (float)ri;
     rr = ri * ri;
   }
   __shared__ double sh[NT / 64];
   const double a = block_sum<NT>(rr, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = a;
 }
+__global__ __launch_bounds__(NT) void k_resid_rr_pair(Op64 o, int nb, const uint8_t *__restrict__ nm,
+                                                       const uint8_t *__restrict__ nc, const double *__restrict__ x,
+                                                       const double *__restrict__ b, float *__restrict__ r32,
+                                                       double *__restrict__ part) {
+  const int tile = xcd_tile(blockIdx.x, gridDim.x);
+  const uint32_t i = 2u * ((uint32_t)tile * NT + threadIdx.x);
+  double2 rr = make_double2(0.0, 0.0);
+  if (i < o.n) {
+    const double2 bv = ld2(b, i);
+    double2 c, y;
+    bool s0, s1;
+    apply_pair(o, nm, nc, x, i, c, y, s0, s1);
+    const double2 ri = make_double2(s0 ? 0.0 : bv.x - y.x, s1 ? 0.0 : bv.y - y.y);
+    if (r32) *reinterpret_cast<float2 *>(r32 + i) = make_float2((float)ri.x, (float)ri.y);
+    rr = make_double2(ri.x * ri.x, ri.y * ri.y);
+  }
+  __shared__ double sh[NT / 32];
+  const double a = pair_sum(rr.x, rr.y, sh);
+  const int t = 2 * tile + (int)threadIdx.x;
+  if (threadIdx.x < 2 && t < nb) part[xcd_block(t, nb)] = a;
+}
 
 uint32_t cg_part_blocks(uint32_t n) { return nblocks(n); }
-void launch_resid_rr(const MgLevel &L, const double *x, const double *b, double *r, double *part, double *dev,
+void launch_resid_rr(const MgLevel &L, const double *x, const double *b, float *r32, double *part, double *dev,
                      hipStream_t s) {
-  const unsigned nb = nblocks(L.n);
-  k_resid_rr<<<nb, NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, b, r, part);
-  k_sum_final<<<1, 1024, 0, s>>>(part, (int)nb, 1, dev, 2);
+  const int nb = nblocks(L.n);
+  if (pairs_of(L)) k_resid_rr_pair<<<nblocks2(L.n), NT, 0, s>>>(op64_of(L), nb, L.nm, L.nc, x, b, r32, part);
+  else k_resid_rr<<<nb, NT, 0, s>>>(op64_of(L), L.nm, L.nc, x, b, r32, part);
+  k_sum_final<<<1, 1024, 0, s>>>(part, nb, 1, dev, 2);
 }
 void launch_apply_dots(const MgLevel &L, const double *p, const double *r, double *q, double *part, double *dev,
                        hipStream_t s) {
-  const unsigned nb = nblocks(L.n);
-  k_apply_dots<<<nb, NT, 0, s>>>(op64_of(L), L.nm, L.nc, p, r, q, part);
-  k_sum_final<<<1, 1024, 0, s>>>(part, (int)nb, 2, dev, 0);
+  const int nb = nblocks(L.n);
+  if (pairs_of(L)) k_apply_dots_pair<<<nblocks2(L.n), NT, 0, s>>>(op64_of(L), nb, L.nm, L.nc, p, r, q, part);
+  else k_apply_dots<<<nb, NT, 0, s>>>(op64_of(L), L.nm, L.nc, p, r, q, part);
+  k_sum_final<<<1, 1024, 0, s>>>(part, nb, 2, dev, 0);
 }
-void launch_update_rr(uint32_t n, const double *dev, const double *p, const double *q, double *x, double *r,
-                      double *part, double *dev_out, hipStream_t s) {
-  const unsigned nb = nblocks(n);
-  k_update_rr<<<nb, NT, 0, s>>>(n, dev, p, q, x, r, part);
-  k_sum_final<<<1, 1024, 0, s>>>(part, (int)nb, 1, dev_out, 2);
+void launch_update_rr(uint32_t n, const double *q, double *r, float *b32, double *part, double *dev, hipStream_t s) {
+  const int nb = nblocks(n);
+  if (n % 2 == 0) k_update_rr<true><<<nblocks2(n), NT, 0, s>>>(n, nb, dev, q, r, b32, part);
+  else k_update_rr<false><<<nb, NT, 0, s>>>(n, nb, dev, q, r, b32, part);
+  k_sum_final<<<1, 1024, 0, s>>>(part, nb, 1, dev, 2);
 }
 void launch_to_f32_zero(uint32_t n, const double *r, float *b, float *phi, hipStream_t s) {
   k_to_f32_zero<<<nblocks(n), NT, 0, s>>>(n, r, b, phi);
 }
-void launch_to_f64_dot(uint32_t n, const float *phi, const double *q, double *z, double *part, double *dev,
-                       hipStream_t s) {
-  const unsigned nb = nblocks(n);
-  k_to_f64_dot<<<nb, NT, 0, s>>>(n, phi, q, z, part);
-  k_sum_final<<<1, 1024, 0, s>>>(part, (int)nb, 1, dev, 3);
+void launch_dot_zq(uint32_t n, const float *phi, const double *q, double *part, double *dev, hipStream_t s) {
+  const int nb = nblocks(n);
+  if (n % 2 == 0) k_dot_zq<true><<<nblocks2(n), NT, 0, s>>>(n, nb, phi, q, part);
+  else k_dot_zq<false><<<nb, NT, 0, s>>>(n, nb, phi, q, part);
+  k_sum_final<<<1, 1024, 0, s>>>(part, nb, 1, dev, 3);
 }
-void launch_xpby_dev(uint32_t n, const double *z, const double *dev, double *p, hipStream_t s) {
-  k_xpby_dev<<<nblocks(n), NT, 0, s>>>(n, z, dev, p);
+void launch_step_p(uint32_t n, const double *dev, const float *phi, const double *z64, double *p, double *x,
+                   hipStream_t s) {
+  const bool pair = n % 2 == 0;
+  const int nb = pair ? nblocks2(n) : nblocks(n);
+  if (pair && z64) k_step_p<true, true><<<nb, NT, 0, s>>>(n, dev, phi, z64, p, x);
+  else if (pair) k_step_p<true, false><<<nb, NT, 0, s>>>(n, dev, phi, z64, p, x);
+  else if (z64) k_step_p<false, true><<<nb, NT, 0, s>>>(n, dev, phi, z64, p, x);
+  else k_step_p<false, false><<<nb, NT, 0, s>>>(n, dev, phi, z64, p, x);
+}
+void launch_step_x(uint32_t n, const double *dev, const double *p, double *x, hipStream_t s) {
+  k_step_x<<<nblocks(n), NT, 0, s>>>(n, dev, p, x);
 }
 
 

@@ -93,7 +93,8 @@ int mg_resid_blocks(const MgLevel &L);
 void launch_copy(const float4 *src, float4 *dst, uint32_t n4, hipStream_t s);
 // V-cycle of sim.rs:451-491 over an arbitrary hierarchy (2 pre- and 2
 // post-sweeps per level, `coarse_iters` SOR iterations at omega = 1.6).
-void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s);
+// from_zero: level 0's phi is taken as 0 and not read.
+void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero = false);
 
 // FP64 solver kernels (k_solve.hip).
 void launch_resid64(const MgLevel &L, const double *x, const double *b, double *r, hipStream_t s);
@@ -114,13 +115,15 @@ void launch_zero64(uint32_t n, double *a, hipStream_t s);
 uint32_t cg_part_blocks(uint32_t n);
 void launch_apply_dots(const MgLevel &L, const double *p, const double *r, double *q, double *part, double *dev,
                        hipStream_t s);
-void launch_update_rr(uint32_t n, const double *dev, const double *p, const double *q, double *x, double *r,
-                      double *part, double *dev_out, hipStream_t s);
+// r -= alpha q, dev[2] = r.r, b32 = (float)r (may be null); alpha = dev[1] / dev[0]
+void launch_update_rr(uint32_t n, const double *q, double *r, float *b32, double *part, double *dev, hipStream_t s);
 void launch_to_f32_zero(uint32_t n, const double *r, float *b, float *phi, hipStream_t s);
-void launch_to_f64_dot(uint32_t n, const float *phi, const double *q, double *z, double *part, double *dev,
-                       hipStream_t s);
-void launch_xpby_dev(uint32_t n, const double *z, const double *dev, double *p, hipStream_t s);
-// r = b - A x, dev[2] = r.r
+// dev[3] = z.q for z = (double)phi
+void launch_dot_zq(uint32_t n, const float *phi, const double *q, double *part, double *dev, hipStream_t s);
+// x += alpha p, p = z + beta p with z = z64, or (double)phi where z64 is null; beta = -dev[3] / dev[0]
+void launch_step_p(uint32_t n, const double *dev, const float *phi, const double *z64, double *p, double *x,
+                   hipStream_t s);
+void launch_step_x(uint32_t n, const double *dev, const double *p, double *x, hipStream_t s);
 // Sealed fluid components (k_solve.hip): union-find labels with every
 // fluid cell's parent at its component's smallest index, open[root] = 1 for
 // components touching a side or the top; (root, cell) pairs of the sealed
@@ -130,7 +133,8 @@ void launch_cc_sealed(const MgLevel &L, const uint32_t *parent, const uint8_t *o
                       unsigned int *count, hipStream_t s);
 void launch_seal_project(uint32_t ncomp, const uint32_t *off, const uint32_t *idx, double *b, hipStream_t s);
 void launch_flags_changed(uint32_t n, const uint8_t *f, uint8_t *prev, unsigned int *changed, hipStream_t s);
-void launch_resid_rr(const MgLevel &L, const double *x, const double *b, double *r, double *part, double *dev,
+// dev[2] = r.r for r = b - A x; r32 = (float)r (may be null)
+void launch_resid_rr(const MgLevel &L, const double *x, const double *b, float *r32, double *part, double *dev,
                      hipStream_t s);
 
 // Debug / test: apply device math to an array (0 exp, 1 sqrt, 2 div by in2).

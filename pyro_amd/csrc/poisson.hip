@@ -106,8 +106,7 @@ int dots(PyroPoisson *P, std::initializer_list<std::pair<const double *, const d
 void precond(PyroPoisson *P, const double *r, double *z) {
   MgLevel &L0 = P->pc[0];
   launch_to_f32(P->n, r, L0.b, P->stream);
-  launch_zero32(P->n, L0.phi, P->stream);
-  enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream);
+  enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true);
   launch_to_f64(P->n, L0.phi, z, P->stream);
 }
 
@@ -440,7 +439,7 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
       launch_to_f64(n, L0.phi, P->x, P->stream);
       cycles++;
       it++;
-      launch_resid_rr(P->pc[0], P->x, P->b, P->r, P->cgpart, P->dev, P->stream);
+      launch_resid_rr(P->pc[0], P->x, P->b, nullptr, P->cgpart, P->dev, P->stream);
       double rr = 0.0;
       PCHK(hipMemcpyAsync(&rr, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
       rc = sync(P);
@@ -454,14 +453,14 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     rc = rel_resid(P, &rel, &bb);
     if (bb <= 0.0) bb = 1.0;
     if (!rc) watch(0);
+    MgLevel &L0 = P->pc[0];
+    if (!rc && !diverged && rel > tol) launch_to_f32(n, P->r, L0.b, P->stream);
     while (!rc && !diverged && rel > tol && it < max_iters) {
-      MgLevel &L0 = P->pc[0];
-      launch_to_f32_zero(n, P->r, L0.b, L0.phi, P->stream);
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true);
       launch_add_f32_to_f64(n, L0.phi, P->x, P->stream);
       cycles++;
       it++;
-      launch_resid_rr(L0, P->x, P->b, P->r, P->cgpart, P->dev, P->stream);
+      launch_resid_rr(L0, P->x, P->b, L0.b, P->cgpart, P->dev, P->stream);
       double rr = 0.0;
       PCHK(hipMemcpyAsync(&rr, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
       rc = sync(P);
@@ -478,13 +477,18 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     // host reads only r.r for the convergence test.
     bool use_net = method == PYRO_SOLVER_LEARNED;
     MgLevel &L0 = P->pc[0];
-    auto apply_m = [&](double rr_now, bool with_dot) -> int {
+    // z = M(r): in L0.phi (z64 null), or in P->z where the network had a part
+    // in it; L0.b holds (float)r when b32_ready.  dev[3] = z.q with_dot.
+    const double *z64 = nullptr;
+    auto apply_m = [&](double rr_now, bool with_dot, bool b32_ready) -> int {
+      z64 = nullptr;
       if (use_net) {
         bool ok = false;
         int e = learned_precond(P, P->r, rr_now, P->z, &ok);
         if (e) return e;
         if (ok) {
           if (P->learned_mode & 1) use_net = false;
+          z64 = P->z;
           if (with_dot) {
             const double *a[1] = {P->z}, *b[1] = {P->q};
             launch_dots(a, b, 1, n, P->part, P->dev + 3, P->stream);
@@ -493,26 +497,28 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         }
         use_net = false;
         fallbacks++;
+        b32_ready = false;
       }
-      launch_to_f32_zero(n, P->r, L0.b, L0.phi, P->stream);
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream);
-      if (with_dot)
-        launch_to_f64_dot(n, L0.phi, P->q, P->z, P->cgpart, P->dev, P->stream);
-      else
-        launch_to_f64(n, L0.phi, P->z, P->stream);
+      if (!b32_ready) launch_to_f32(n, P->r, L0.b, P->stream);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true);
+      if (with_dot) launch_dot_zq(n, L0.phi, P->q, P->cgpart, P->dev, P->stream);
       return 0;
     };
-    double bb = 0.0;
+    double bb = 0.0, bb_raw = 0.0;
     rc = rel_resid(P, &rel, &bb);  // r = b - A x
+    bb_raw = bb;
     if (bb <= 0.0) bb = 1.0;
     if (!rc) watch(0);
     if (!rc && !diverged && rel > tol) {
-      rc = apply_m(rel * rel * bb, false);
+      rc = apply_m(rel * rel * bb, false, false);
       cycles++;
-      if (!rc) PCHK(hipMemcpyAsync(P->p, P->z, n * sizeof(double), hipMemcpyDeviceToDevice, P->stream));
+      if (!rc && z64) PCHK(hipMemcpyAsync(P->p, z64, n * sizeof(double), hipMemcpyDeviceToDevice, P->stream));
+      if (!rc && !z64) launch_to_f64(n, L0.phi, P->p, P->stream);
+      bool pending = false;  // x has still to take alpha p of the last iteration
       while (!rc && it < max_iters) {
         launch_apply_dots(L0, P->p, P->r, P->q, P->cgpart, P->dev, P->stream);  // dev[0] p.q, dev[1] p.r
-        launch_update_rr(n, P->dev, P->p, P->q, P->x, P->r, P->cgpart, P->dev, P->stream);  // dev[2] r.r
+        launch_update_rr(n, P->q, P->r, use_net ? nullptr : L0.b, P->cgpart, P->dev, P->stream);  // dev[2] r.r
+        pending = true;
         it++;
         double rr = 0.0;
         PCHK(hipMemcpyAsync(&rr, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
@@ -520,12 +526,19 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         if (rc) break;
         rel = std::sqrt(rr / bb);
         if (watch(it) || rel <= tol) break;
-        rc = apply_m(rr, true);  // z, dev[3] z.q
+        rc = apply_m(rr, true, !use_net);  // z, dev[3] z.q
         if (rc) break;
         cycles++;
-        launch_xpby_dev(n, P->z, P->dev, P->p, P->stream);
+        launch_step_p(n, P->dev, L0.phi, z64, P->p, P->x, P->stream);
+        pending = false;
       }
-      if (!rc) rc = rel_resid(P, &rel, nullptr);  // true residual of the final x
+      if (pending) launch_step_x(n, P->dev, P->p, P->x, P->stream);
+      if (!rc) {  // true residual of the final x
+        launch_resid64(L0, P->x, P->b, P->r, P->stream);
+        double d[1];
+        rc = dots(P, {{P->r, P->r}}, d);
+        if (!rc) rel = bb_raw > 0.0 ? std::sqrt(d[0] / bb_raw) : std::sqrt(d[0]);
+      }
       if (!rc && !std::isfinite(rel)) rc = pfail(PYRO_E_NONFINITE, "non-finite residual of the final iterate");
     }
   }
