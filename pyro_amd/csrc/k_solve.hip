@@ -657,19 +657,4 @@ void launch_seal_project(uint32_t ncomp, const uint32_t *off, const uint32_t *id
   if (ncomp) k_seal_project<<<ncomp, NT, 0, s>>>(off, idx, b);
 }
 
-// changed |= (f != prev); prev = f
-__global__ __launch_bounds__(NT) void k_flags_changed(uint32_t n, const uint8_t *__restrict__ f, uint8_t *prev,
-                                                      unsigned int *changed) {
-  const uint32_t i = blockIdx.x * NT + threadIdx.x;
-  if (i >= n) return;
-  const uint8_t v = f[i];
-  if (prev[i] != v) {
-    prev[i] = v;
-    *changed = 1u;
-  }
-}
-void launch_flags_changed(uint32_t n, const uint8_t *f, uint8_t *prev, unsigned int *changed, hipStream_t s) {
-  k_flags_changed<<<nblocks(n), NT, 0, s>>>(n, f, prev, changed);
-}
-
 }  // namespace pyro

@@ -5,6 +5,7 @@
 #include "common.hpp"
 
 struct PyroShape;  // pyro_scene.h
+struct PyroSim;    // sim.hip
 
 namespace pyro {
 
@@ -127,18 +128,22 @@ void launch_step_x(uint32_t n, const double *dev, const double *p, double *x, hi
 // Sealed fluid components (k_solve.hip): union-find labels with every
 // fluid cell's parent at its component's smallest index, open[root] = 1 for
 // components touching a side or the top; (root, cell) pairs of the sealed
-// ones; b -= mean over each sealed component; a flag-change detector.
+// ones; b -= mean over each sealed component.
 void launch_cc_label(const MgLevel &L, uint32_t *parent, uint8_t *open, hipStream_t s);
 void launch_cc_sealed(const MgLevel &L, const uint32_t *parent, const uint8_t *open, uint2 *out,
                       unsigned int *count, hipStream_t s);
 void launch_seal_project(uint32_t ncomp, const uint32_t *off, const uint32_t *idx, double *b, hipStream_t s);
-void launch_flags_changed(uint32_t n, const uint8_t *f, uint8_t *prev, unsigned int *changed, hipStream_t s);
 // dev[2] = r.r for r = b - A x; r32 = (float)r (may be null)
 void launch_resid_rr(const MgLevel &L, const double *x, const double *b, float *r32, double *part, double *dev,
                      hipStream_t s);
 
 // Debug / test: apply device math to an array (0 exp, 1 sqrt, 2 div by in2).
 void launch_debug_math(int fn, const float *in, const float *in2, float *out, uint32_t n, hipStream_t s);
+
+// The stages of an open step up to the divergence in the step's fused launches
+// (sim.hip; 0 or a PYRO_E_* code), and the simulation's stream.
+int sim_run_to_divergence(::PyroSim *s);
+hipStream_t sim_stream(::PyroSim *s);
 
 inline int nblocks(uint32_t n) { return (int)((n + NT - 1) / NT); }
 

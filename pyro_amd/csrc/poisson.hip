@@ -55,6 +55,8 @@ struct PyroPoisson {
   double nfluid = 0.0;
   unsigned int *count = nullptr;  // device fluid-cell counter
   hipStream_t stream = nullptr;
+  // solve timing, and the order between a simulation's stream and this one
+  hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr, ev_sim = nullptr, ev_done = nullptr;
   std::vector<void *> allocs;
   int coarse_iters_pc = 80;
   PyroNet *net = nullptr;
@@ -119,11 +121,19 @@ int rel_resid(PyroPoisson *P, double *rel, double *bb_out) {
   if (bb_out) *bb_out = d[1];
   return 0;
 }
-// solid flags from a simulation's level-0 flags (1 solid; 0 and 2, burnt out, are fluid)
+// solid flags from a simulation's level-0 flags (1 solid; 0 and 2, burnt out,
+// are fluid), written with the labelling's copy only where they changed
 __global__ __launch_bounds__(256) void k_flags_from_sim(uint32_t n, const uint8_t *__restrict__ src,
-                                                        uint8_t *__restrict__ f) {
+                                                        uint8_t *__restrict__ f, uint8_t *__restrict__ prev,
+                                                        unsigned int *changed) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < n) f[i] = src[i] == 1 ? 1 : 0;
+  if (i >= n) return;
+  const uint8_t v = src[i] == 1 ? 1 : 0;
+  if (prev[i] != v || f[i] != v) {
+    prev[i] = v;
+    f[i] = v;
+    *changed = 1u;
+  }
 }
 
 // number of fluid cells: per-wave ballots summed in LDS, one integer atomic
@@ -256,20 +266,36 @@ int relabel(PyroPoisson *P) {
   return 0;
 }
 
+// The levels' codes, the fluid count and the labels follow the flags and are
+// formed again only when those changed (fourteen launches otherwise spent on
+// every solved step).
 int set_flags_device(PyroPoisson *P, const uint8_t *sim_flags) {
-  k_flags_from_sim<<<nblocks(P->n), 256, 0, P->stream>>>(P->n, sim_flags, P->pc[0].f);
-  launch_mg_setup(P->pc, P->nl_pc, P->stream);
   PCHK(hipMemsetAsync(P->count, 0, 2 * sizeof(unsigned int), P->stream));
-  k_count_fluid<<<COUNT_BLOCKS, 256, 0, P->stream>>>(P->n, P->pc[0].f, P->count);
-  launch_flags_changed(P->n, P->pc[0].f, P->fprev, P->count + 1, P->stream);
+  k_flags_from_sim<<<nblocks(P->n), 256, 0, P->stream>>>(P->n, sim_flags, P->pc[0].f, P->fprev, P->count + 1);
   unsigned int c[2] = {0, 0};
   PCHK(hipMemcpyAsync(c, P->count, sizeof(c), hipMemcpyDeviceToHost, P->stream));
   int rc = sync(P);
   if (rc) return rc;
+  if (!c[1] && P->labelled) return 0;
+  P->labelled = false;  // until the labels below are complete
+  launch_mg_setup(P->pc, P->nl_pc, P->stream);
+  k_count_fluid<<<COUNT_BLOCKS, 256, 0, P->stream>>>(P->n, P->pc[0].f, P->count);
+  PCHK(hipMemcpyAsync(c, P->count, sizeof(unsigned int), hipMemcpyDeviceToHost, P->stream));
+  rc = sync(P);
+  if (rc) return rc;
   P->nfluid = (double)c[0];
   P->nfluid1 = -1.0;
-  if (c[1] || !P->labelled) return relabel(P);
-  return 0;
+  return relabel(P);
+}
+
+// b = the simulation's level-0 right-hand side, x = its level-0 phi (warm) or 0
+void take_problem(PyroPoisson *P, const float *b, const float *phi, bool warm) {
+  launch_to_f64(P->n, b, P->b, P->stream);
+  P->b_fresh = true;
+  if (warm)
+    launch_to_f64(P->n, phi, P->x, P->stream);
+  else
+    launch_zero64(P->n, P->x, P->stream);
 }
 
 bool projects(const PyroPoisson *P, int method) {
@@ -293,6 +319,10 @@ int pyro_poisson_create(uint32_t nx, uint32_t ny, uint32_t nz, float h, const ui
   P->n = nx * ny * nz;
   if (hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(pfail(PYRO_E_HIP, "hipStreamCreate failed"));
+  if (hipEventCreate(&P->ev_t0) != hipSuccess || hipEventCreate(&P->ev_t1) != hipSuccess ||
+      hipEventCreateWithFlags(&P->ev_sim, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&P->ev_done, hipEventDisableTiming) != hipSuccess)
+    return bail(pfail(PYRO_E_HIP, "hipEventCreate failed"));
   int d[3] = {(int)nx, (int)ny, (int)nz};
   float hl = h;
   int rc = 0;
@@ -364,6 +394,8 @@ int pyro_poisson_destroy(PyroPoisson *P) {
   for (void *v : P->allocs) (void)hipFree(v);
   if (P->seal_idx) (void)hipFree(P->seal_idx);
   if (P->seal_off) (void)hipFree(P->seal_off);
+  for (hipEvent_t e : {P->ev_t0, P->ev_t1, P->ev_sim, P->ev_done})
+    if (e) (void)hipEventDestroy(e);
   if (P->stream) (void)hipStreamDestroy(P->stream);
   delete P;
   return 0;
@@ -401,10 +433,7 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
   if (!P || max_iters < 1 || !(tol >= 0.0)) return pfail(PYRO_E_INVALID, "bad argument");
   if (method < PYRO_SOLVER_VCYCLE || method > PYRO_SOLVER_LEARNED) return pfail(PYRO_E_INVALID, "unknown method");
   if (method == PYRO_SOLVER_LEARNED && !P->net) return pfail(PYRO_E_STATE, "no network attached");
-  hipEvent_t e0, e1;
-  PCHK(hipEventCreate(&e0));
-  PCHK(hipEventCreate(&e1));
-  PCHK(hipEventRecord(e0, P->stream));
+  PCHK(hipEventRecord(P->ev_t0, P->stream));
   if (P->b_fresh && P->seal_comp && projects(P, method)) {
     launch_seal_project(P->seal_comp, P->seal_off, P->seal_idx, P->b, P->stream);
     P->b_fresh = false;
@@ -542,12 +571,10 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
       if (!rc && !std::isfinite(rel)) rc = pfail(PYRO_E_NONFINITE, "non-finite residual of the final iterate");
     }
   }
-  PCHK(hipEventRecord(e1, P->stream));
-  PCHK(hipEventSynchronize(e1));
+  PCHK(hipEventRecord(P->ev_t1, P->stream));
+  PCHK(hipEventSynchronize(P->ev_t1));
   float ms = 0.0f;
-  PCHK(hipEventElapsedTime(&ms, e0, e1));
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  PCHK(hipEventElapsedTime(&ms, P->ev_t0, P->ev_t1));
   if (rc) return rc;
   if (info) {
     info->iterations = it;
@@ -607,12 +634,7 @@ int pyro_poisson_set_from_sim(PyroPoisson *P, PyroSim *sim, int warm) {
       pyro_sim_device_ptr(sim, PYRO_FIELD_LEVEL_BASE + 0, &pp, &npb))
     return pfail(PYRO_E_INVALID, std::string("simulation: ") + pyro_last_error());
   if (nb != (size_t)P->n * 4) return pfail(PYRO_E_INVALID, "grid mismatch");
-  launch_to_f64(P->n, static_cast<const float *>(bp), P->b, P->stream);
-  P->b_fresh = true;
-  if (warm)
-    launch_to_f64(P->n, static_cast<const float *>(pp), P->x, P->stream);
-  else
-    launch_zero64(P->n, P->x, P->stream);
+  take_problem(P, static_cast<const float *>(bp), static_cast<const float *>(pp), warm != 0);
   return sync(P);
 }
 
@@ -644,10 +666,23 @@ int pyro_sim_step_solve(PyroSim *sim, PyroPoisson *P, int method, double tol, in
   auto simfail = [&]() {
     return abort_with(pfail(PYRO_E_STATE, std::string("simulation: ") + pyro_last_error()));
   };
-  for (int st = PYRO_STAGE_SOLID; st <= PYRO_STAGE_DIVERGENCE; st++)
-    if (pyro_sim_run_stage(sim, st)) return simfail();
-  int rc = pyro_poisson_set_flags_from_sim(P, sim);
-  if (!rc) rc = pyro_poisson_set_from_sim(P, sim, 1);
+  if (sim_run_to_divergence(sim)) return simfail();
+  void *fp = nullptr, *bp = nullptr, *pp = nullptr;
+  if (pyro_sim_device_ptr(sim, PYRO_FIELD_LEVEL_BASE + 2, &fp, nullptr) ||
+      pyro_sim_device_ptr(sim, PYRO_FIELD_LEVEL_BASE + 1, &bp, nullptr) ||
+      pyro_sim_device_ptr(sim, PYRO_FIELD_LEVEL_BASE + 0, &pp, nullptr))
+    return simfail();
+  // the solve's stream follows the simulation's, and the projection below the
+  // solve's, by events: the host waits only where it reads a value
+  const hipStream_t ss = sim_stream(sim);
+  auto follow = [&](hipEvent_t ev, hipStream_t from, hipStream_t to) -> int {
+    PCHK(hipEventRecord(ev, from));
+    PCHK(hipStreamWaitEvent(to, ev, 0));
+    return 0;
+  };
+  int rc = follow(P->ev_sim, ss, P->stream);
+  if (!rc) rc = set_flags_device(P, static_cast<const uint8_t *>(fp));
+  if (!rc) take_problem(P, static_cast<const float *>(bp), static_cast<const float *>(pp), true);
   PyroSolveInfo si{};
   if (!rc) rc = pyro_poisson_solve(P, method, tol, max_iters, &si);
   if (rc) return abort_with(rc);
@@ -657,11 +692,9 @@ int pyro_sim_step_solve(PyroSim *sim, PyroPoisson *P, int method, double tol, in
                                                  std::to_string(si.rel_resid) + " after " +
                                                  std::to_string(si.iterations) + " iterations"));
   }
-  void *pp = nullptr;
-  size_t nb = 0;
-  if (pyro_sim_device_ptr(sim, PYRO_FIELD_LEVEL_BASE + 0, &pp, &nb)) return simfail();
   launch_to_f32(P->n, P->x, static_cast<float *>(pp), P->stream);
-  rc = sync(P);
+  rc = follow(P->ev_done, P->stream, ss);
+  if (!rc && hipGetLastError() != hipSuccess) rc = pfail(PYRO_E_HIP, "kernel launch failed");
   if (rc) return abort_with(rc);
   if (want_stats && pyro_sim_run_stage(sim, PYRO_STAGE_RESID)) return simfail();
   if (pyro_sim_run_stage(sim, PYRO_STAGE_PROJECT)) return simfail();

@@ -134,26 +134,22 @@ void enqueue_stage(PyroSim *s, int stage, bool stats, hipStream_t st) {
   }
 }
 
-// sim.rs:394-414, plus the FP64 stats combination on stats steps.  Solid and
-// curl run as one launch, and the four advection stages as two (adv_vel1 with
-// adv_s1, then adv_vel2 with adv_s2): in each group no stage reads what
-// another writes, so the outputs are those of the reference's order.
+// sim.rs:394-403: solid to divergence.  Solid and curl run as one launch, and
+// the four advection stages as two (adv_vel1 with adv_s1, then adv_vel2 with
+// adv_s2): in each group no stage reads what another writes, so the outputs
+// are those of the reference's order.
+void enqueue_to_divergence(PyroSim *s, bool stats, hipStream_t st) {
+  const Fields f = fields_of(s);
+  launch_solid_curl(f, stats ? &s->st : nullptr, st);
+  launch_adv_pass1(f, st);
+  launch_adv_pass2(f, st);
+  for (int k : {PYRO_STAGE_REACT, PYRO_STAGE_FORCES, PYRO_STAGE_DIVERGENCE}) enqueue_stage(s, k, stats, st);
+}
+
+// sim.rs:394-414, plus the FP64 stats combination on stats steps.
 void enqueue_step_body(PyroSim *s, bool stats, hipStream_t st) {
-  for (int k = PYRO_STAGE_SOLID; k <= PYRO_STAGE_VCYCLES; k++) {
-    if (k == PYRO_STAGE_SOLID) {
-      launch_solid_curl(fields_of(s), stats ? &s->st : nullptr, st);
-      k = PYRO_STAGE_CURL;
-      continue;
-    }
-    if (k == PYRO_STAGE_ADV_VEL1) {
-      const Fields f = fields_of(s);
-      launch_adv_pass1(f, st);
-      launch_adv_pass2(f, st);
-      k = PYRO_STAGE_ADV_S2;
-      continue;
-    }
-    enqueue_stage(s, k, stats, st);
-  }
+  enqueue_to_divergence(s, stats, st);
+  enqueue_stage(s, PYRO_STAGE_VCYCLES, stats, st);
   if (stats) enqueue_stage(s, PYRO_STAGE_RESID, true, st);
   enqueue_stage(s, PYRO_STAGE_PROJECT, stats, st);
   if (stats) launch_stats_finalize(s->g, s->st, STATS_RAN_ALL, st);
@@ -688,6 +684,20 @@ int pyro_sim_run_stage(PyroSim *s, int stage) {
   if (e != hipSuccess) return fail(PYRO_E_HIP, std::string("launch: ") + hipGetErrorString(e));
   return 0;
 }
+
+}  // extern "C"
+namespace pyro {
+int sim_run_to_divergence(PyroSim *s) {
+  if (!s->in_step) return fail(PYRO_E_STATE, "run_stage outside begin_step/end_step");
+  enqueue_to_divergence(s, s->step_stats, s->stream);
+  s->stats_ran |= STATS_RAN_SOLID | STATS_RAN_CURL | STATS_RAN_REACT;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(PYRO_E_HIP, std::string("launch: ") + hipGetErrorString(e));
+  return 0;
+}
+hipStream_t sim_stream(PyroSim *s) { return s->stream; }
+}  // namespace pyro
+extern "C" {
 
 int pyro_sim_end_step(PyroSim *s) {
   if (!s) return fail(PYRO_E_INVALID, "null sim");
