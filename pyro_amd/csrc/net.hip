@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "hostcopy.hpp"
 #include "kernels.hpp"
 #include "net.hpp"
 #include "pyro_hip.h"
@@ -57,6 +58,7 @@ struct Sample {
 }  // namespace
 
 struct PyroNet {
+  HostCopyUse host;  // large host arrays go through the pinned slots
   hipStream_t stream = nullptr;
   size_t np = 0;
   float *params = nullptr, *grads = nullptr, *am = nullptr, *av = nullptr;
@@ -409,11 +411,11 @@ int pyro_net_forward(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, const fl
   float *tmp = N->inf.y;  // host x0 staged through y (n floats) twice
   const size_t n = g.n();
   for (int half = 0; half < 2; half++) {
-    NCHK(hipMemcpyAsync(tmp, x0 + half * n, n * sizeof(float), hipMemcpyHostToDevice, N->stream));
+    NCHK(copy_in(tmp, x0 + half * n, n * sizeof(float), N->stream, true));
     launch_f32_to_bf16((uint32_t)n, tmp, N->inf.x0 + half * n, N->stream);
   }
   forward(N, N->inf, N->inf.x0);
-  NCHK(hipMemcpyAsync(y, N->inf.y, n * sizeof(float), hipMemcpyDeviceToHost, N->stream));
+  NCHK(copy_out(y, N->inf.y, n * sizeof(float), N->stream));
   return nsync(N);
 }
 
@@ -426,11 +428,11 @@ int pyro_net_backward(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, const f
   if (rc) return rc;
   const size_t n = g.n();
   for (int half = 0; half < 2; half++) {
-    NCHK(hipMemcpyAsync(N->tr.gy, x0 + half * n, n * sizeof(float), hipMemcpyHostToDevice, N->stream));
+    NCHK(copy_in(N->tr.gy, x0 + half * n, n * sizeof(float), N->stream, true));
     launch_f32_to_bf16((uint32_t)n, N->tr.gy, N->tr.x0 + half * n, N->stream);
   }
   forward(N, N->tr, N->tr.x0);
-  NCHK(hipMemcpyAsync(N->tr.gy, gy, n * sizeof(float), hipMemcpyHostToDevice, N->stream));
+  NCHK(copy_in(N->tr.gy, gy, n * sizeof(float), N->stream, true));
   backward(N, N->tr, N->tr.x0);
   return nsync(N);
 }

@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "hostcopy.hpp"
 #include "kernels.hpp"
 #include "net.hpp"
 #include "pyro_hip.h"
@@ -41,6 +42,7 @@ int pfail(int code, const std::string &m) {
 }  // namespace
 
 struct PyroPoisson {
+  HostCopyUse host;  // large right-hand sides and solutions go through the pinned slots
   int d[3] = {0, 0, 0};
   float h = 0.0f;
   uint32_t n = 0;
@@ -410,9 +412,9 @@ int pyro_poisson_levels(const PyroPoisson *P, int *ref_levels, int *pc_levels) {
 
 int pyro_poisson_set(PyroPoisson *P, const double *b, const double *phi) {
   if (!P) return pfail(PYRO_E_INVALID, "null handle");
-  if (b) PCHK(hipMemcpy(P->b, b, P->n * sizeof(double), hipMemcpyHostToDevice));
+  if (b) PCHK(copy_in(P->b, b, P->n * sizeof(double), P->stream));
   if (b) P->b_fresh = true;
-  if (phi) PCHK(hipMemcpy(P->x, phi, P->n * sizeof(double), hipMemcpyHostToDevice));
+  if (phi) PCHK(copy_in(P->x, phi, P->n * sizeof(double), P->stream));
   return 0;
 }
 
@@ -420,7 +422,7 @@ int pyro_poisson_get(PyroPoisson *P, double *phi) {
   if (!P || !phi) return pfail(PYRO_E_INVALID, "null argument");
   int rc = sync(P);
   if (rc) return rc;
-  PCHK(hipMemcpy(phi, P->x, P->n * sizeof(double), hipMemcpyDeviceToHost));
+  PCHK(copy_out(phi, P->x, P->n * sizeof(double), P->stream));
   return 0;
 }
 
@@ -603,7 +605,7 @@ int pyro_poisson_sealed_info(const PyroPoisson *P, uint32_t *components, uint32_
 int pyro_poisson_get_rhs(PyroPoisson *P, double *b) {
   if (!P || !b) return pfail(PYRO_E_INVALID, "null argument");
   PCHK(hipStreamSynchronize(P->stream));
-  PCHK(hipMemcpy(b, P->b, P->n * sizeof(double), hipMemcpyDeviceToHost));
+  PCHK(copy_out(b, P->b, P->n * sizeof(double), P->stream));
   return 0;
 }
 
