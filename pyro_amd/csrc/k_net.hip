@@ -304,6 +304,152 @@ __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
   }
 }
 
+// 16 output channels from 16-channel chunks (CA/16 of the upsampled `a`, then
+// `b`).  With one 16-row output block an MFMA of k_conv3 uses its B fragment
+// once, and the LDS (128 B a clock, 8 clocks a fragment) feeds four matrix
+// cores at half their rate.  Here a wave computes 16 x 4 x 4 voxels and keeps
+// a plane's fragments in registers: a group's two taps are an x pair of one
+// row (P: kx 0, 1; R: kx 1, 2), kx 2 with the next row's kx 0 (Q), the step
+// to the next plane (X) or the 27th tap (L), so on one plane the rows' P, Q
+// and R serve all nine (ky, kz) offsets: 26 reads for 56 products instead of
+// 56.  The planes ascend and each voxel's groups stay in order, so every sum
+// is k_conv3's.  Block: 16 x 8 x 8 voxels, footprint 18 x 10 x 10.
+// Every piece of the footprint is loaded without a branch, so that a thread's
+// fifteen are in flight together; with a branch around each the compiler
+// waits for one before the next (160x320x160, forward pass: 1526 us, now 1256).
+// Launches at 160x320x160 with k_conv3 and with this: 48 -> 16 channels 736 us
+// and 363, 16 -> 16 332 and 188; at 80x160x80 95 and 46, 39 and 26.
+constexpr int CS_Y = 8, CS_Z = 8, CS_FY = CS_Y + 2, CS_FZ = CS_Z + 2, CS_FN = CV_FX * CS_FY * CS_FZ;
+template <int CA, bool RELU>
+__global__ __launch_bounds__(256, 2) void k_conv3_16(ConvArgs p) {
+  constexpr int NCH = CA / 16 + 1;
+  constexpr int ROW = CV_FX * 16, PLANE = CS_FY * ROW;  // elements
+  __shared__ __align__(16) bf16 lds[CS_FN * 16];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int j = lane >> 4, col = lane & 15, up = j >> 1;
+  const int ntx = (p.nx + CV_TX - 1) / CV_TX, nty = (p.ny + CS_Y - 1) / CS_Y;
+  const int bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int tx = bid % ntx, rr = bid / ntx, ty = rr % nty, tz = rr / nty;
+  const int x0 = tx * CV_TX, y0 = ty * CS_Y, z0 = tz * CS_Z;
+  f32x4 acc[4][4];  // [z][y]
+#pragma unroll
+  for (int z = 0; z < 4; z++)
+#pragma unroll
+    for (int y = 0; y < 4; y++) acc[z][y] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const int wy = 4 * (w & 1), wz = 4 * (w >> 1);
+  // a lane's eight channels of footprint voxel fx of a row: the two halves of
+  // a voxel change places where bit 3 of fx is set, so that sixteen voxels
+  // (32 bytes apart) touch every bank once
+  auto at = [&](int fx) __attribute__((always_inline)) {
+    return lds + wz * PLANE + wy * ROW + fx * 16 + ((j ^ (fx >> 3)) & 1) * 8;
+  };
+  const bf16 *bP = at(col + up), *bR = at(col + 1 + up), *bL = at(col + 2) + 2 * ROW;
+  const bf16 *bQ = at(up ? col : col + 2) + (up ? ROW : 0), *bX = at(up ? col : col + 2) + (up ? PLANE : 2 * ROW);
+  // staging: a thread loads one 16-byte half of voxel sx of the rows sr + 7 k
+  constexpr int PIECES = 2 * CV_FX, SROWS = 256 / PIECES, NROWS = CS_FY * CS_FZ;
+  constexpr int NPT = (NROWS + SROWS - 1) / SROWS;
+  const int sp = threadIdx.x % PIECES, sr = threadIdx.x / PIECES, sx = sp >> 1;
+  const int sgx = x0 + sx - 1;
+  const int cgx = min(max(sgx, 0), p.nx - 1);
+  bf16 *sdst = lds + sx * 16 + ((sp ^ (sx >> 3)) & 1) * 8;
+#pragma unroll 1
+  for (int q = 0; q < NCH; q++) {
+    const bool from_a = q < NCH - 1;
+    const int sh = from_a ? 1 : 0;
+    const size_t snx = (size_t)(from_a ? p.anx : p.nx), sny = (size_t)(from_a ? p.any : p.ny), sc = from_a ? CA : 16;
+    const bf16 *src = (from_a ? p.a + 16 * q : p.b) + 8 * (sp & 1);
+    const bf16 *wp = p.wp + (size_t)q * 14 * 16 * 32 + col * 32 + 8 * j;
+    __syncthreads();
+    bf16x8 A[14];
+#pragma unroll
+    for (int g = 0; g < 14; g++) A[g] = *reinterpret_cast<const bf16x8 *>(wp + (size_t)g * 16 * 32);
+    {
+      // every piece is loaded, from the nearest voxel inside the grid, and
+      // zeroed afterwards where it lies outside: no branches, so that all of
+      // a thread's loads are in flight together
+      uint4 val[NPT];
+#pragma unroll
+      for (int k = 0; k < NPT; k++) {
+        const int row = min(sr + SROWS * k, NROWS - 1);
+        const int gy = min(max(y0 + row % CS_FY - 1, 0), p.ny - 1), gz = min(max(z0 + row / CS_FY - 1, 0), p.nz - 1);
+        const size_t v = (size_t)(cgx >> sh) + snx * ((size_t)(gy >> sh) + sny * (size_t)(gz >> sh));
+        val[k] = *reinterpret_cast<const uint4 *>(src + v * sc);
+      }
+#pragma unroll
+      for (int k = 0; k < NPT; k++) {
+        const int row = sr + SROWS * k, fy = row % CS_FY, fz = row / CS_FY;
+        const int gy = y0 + fy - 1, gz = z0 + fz - 1;
+        const bool in = sgx == cgx && gy >= 0 && gy < p.ny && gz >= 0 && gz < p.nz;
+        if (sr < SROWS && row < NROWS)
+          *reinterpret_cast<uint4 *>(sdst + row * ROW) = in ? val[k] : make_uint4(0u, 0u, 0u, 0u);
+      }
+    }
+    __syncthreads();
+    auto rd = [&](const bf16 *b, int plane, int row) __attribute__((always_inline)) {
+      return *reinterpret_cast<const bf16x8 *>(b + plane * PLANE + row * ROW);
+    };
+#pragma unroll
+    for (int pl = 0; pl < 6; pl++) {
+      bf16x8 P[6], R[6], Q[5];
+#pragma unroll
+      for (int r = 0; r < 6; r++) {
+        P[r] = rd(bP, pl, r);
+        R[r] = rd(bR, pl, r);
+        if (r < 5) Q[r] = rd(bQ, pl, r);
+      }
+      bf16x8 X[4], L[4];
+#pragma unroll
+      for (int y = 0; y < 4; y++) {
+        if (pl >= 1 && pl <= 4) X[y] = rd(bX, pl - 1, y);
+        if (pl >= 2) L[y] = rd(bL, pl, y);
+      }
+      // one product of every (plane offset, row) in turn: twelve sums in flight
+#pragma unroll
+      for (int st = 0; st < 5; st++) {
+#pragma unroll
+        for (int y = 0; y < 4; y++) {
+          if (pl <= 3 && st < 4) {  // kz = 0: groups 0..3
+            const bf16x8 &B = st == 0 ? P[y] : st == 1 ? Q[y] : st == 2 ? R[y + 1] : P[y + 2];
+            acc[pl < 4 ? pl : 0][y] = mfma16x16x32(A[st], B, acc[pl < 4 ? pl : 0][y]);
+          }
+          if (pl >= 1 && pl <= 4) {  // the step to kz = 1, then groups 5..8
+            const bf16x8 &B = st == 0 ? X[y] : st == 1 ? R[y] : st == 2 ? P[y + 1] : st == 3 ? Q[y + 1] : R[y + 2];
+            const int z = pl >= 1 && pl <= 4 ? pl - 1 : 0;
+            acc[z][y] = mfma16x16x32(A[4 + st], B, acc[z][y]);
+          }
+          if (pl >= 2) {  // kz = 2: groups 9..13
+            const bf16x8 &B = st == 0 ? P[y] : st == 1 ? Q[y] : st == 2 ? R[y + 1] : st == 3 ? P[y + 2] : L[y];
+            const int z = pl >= 2 ? pl - 2 : 0;
+            acc[z][y] = mfma16x16x32(A[9 + st], B, acc[z][y]);
+          }
+        }
+      }
+    }
+  }
+  const int gx = x0 + col;
+  if (gx >= p.nx) return;
+  float bias[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) bias[i] = p.bias ? p.bias[4 * j + i] : 0.0f;
+#pragma unroll
+  for (int z = 0; z < 4; z++) {
+#pragma unroll
+    for (int y = 0; y < 4; y++) {
+      const int gy = y0 + wy + y, gz = z0 + wz + z;
+      if (gy >= p.ny || gz >= p.nz) continue;
+      const size_t v = (size_t)gx + (size_t)p.nx * ((size_t)gy + (size_t)p.ny * (size_t)gz);
+      bf16x4 o;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        float t = acc[z][y][i] + bias[i];
+        if (RELU) t = t > 0.0f ? t : 0.0f;
+        o[i] = tobf(t);
+      }
+      *reinterpret_cast<bf16x4 *>(p.out + v * 16 + 4 * j) = o;
+    }
+  }
+}
+
 bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *b, int cb, const bf16 *wp,
                   const float *bias, int cout, bool relu, bf16 *out, hipStream_t s) {
   ConvArgs p;
@@ -312,19 +458,37 @@ bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *
   p.a = a; p.b = b; p.wp = wp; p.bias = bias; p.out = out;
   const unsigned nb = (unsigned)(((g.nx + CV_TX - 1) / CV_TX) * ((g.ny + CV_TY - 1) / CV_TY) *
                                  ((g.nz + CV_TZ - 1) / CV_TZ));
+  const unsigned nb16 = (unsigned)(((g.nx + CV_TX - 1) / CV_TX) * ((g.ny + CS_Y - 1) / CS_Y) *
+                                   ((g.nz + CS_Z - 1) / CS_Z));
 #define PYRO_CONV(CA_, CB_, CO_, R_)                                          \
   if (ca == CA_ && cb == CB_ && cout == CO_ && relu == R_) {                  \
     k_conv3<CA_, CB_, CO_, R_><<<nb, 256, 0, s>>>(p);                         \
     return true;                                                              \
   }
-  PYRO_CONV(0, 16, 16, true)
+#define PYRO_CONV16(CA_, R_)                                      \
+  if (ca == CA_ && cb == 16 && cout == 16 && relu == R_) {        \
+    k_conv3_16<CA_, R_><<<nb16, 256, 0, s>>>(p);                  \
+    return true;                                                  \
+  }
+  // Small grids: the small tiles give four times the workgroups, and while
+  // all of them are resident at once (two to a compute unit) a launch lasts as
+  // long as one of them.  The forward pass with either kernel for these
+  // layers: 24x40x24 (120 small tiles) 126 us against 130, 40x64x40 (480) 137
+  // against 138; 48x80x48 (720) 166 against 164, 64x64x64 (1024) 175 against 167.
+  if (nb <= 512) {
+    PYRO_CONV(0, 16, 16, true)
+    PYRO_CONV(32, 16, 16, true)
+    PYRO_CONV(0, 16, 16, false)
+  }
+  PYRO_CONV16(0, true)
+  PYRO_CONV16(32, true)
+  PYRO_CONV16(0, false)
+#undef PYRO_CONV16
   PYRO_CONV(0, 16, 32, true)
   PYRO_CONV(0, 32, 32, true)
   PYRO_CONV(0, 32, 64, true)
   PYRO_CONV(0, 64, 64, true)
   PYRO_CONV(64, 32, 32, true)
-  PYRO_CONV(32, 16, 16, true)
-  PYRO_CONV(0, 16, 16, false)
   PYRO_CONV(0, 32, 16, false)
   PYRO_CONV(0, 32, 32, false)
   PYRO_CONV(0, 64, 32, false)
