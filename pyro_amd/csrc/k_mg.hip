@@ -779,6 +779,338 @@ void launch_mg_sweep(const MgLevel &L, const float *pin, float *pout, float omeg
   }
 }
 
+// ---------------------------------------------------------------- two sweeps
+// Both red-black sweeps of a smoothing step in one launch, for levels where a
+// sweep is bound by its launch and its load latency and not by its bytes.  A
+// block of 512 threads takes 16 x 8 x 8 cells; phi, h^2 b and the codes of the
+// tile and a ring of 4 sit in LDS, and the four colour passes run on rings of
+// 3, 2, 1 and 0.  The arrays are split by colour: entry k of row (y, z) of
+// colour c is the cell lx = 2 k + par, par = (c + ly + lz) & 1 (tile origins are
+// multiples of four), so the lanes
+// of a pass touch consecutive words, and the neighbours of an entry of one
+// colour are entries of the other: k and k + 1 (par = 1) or k - 1 (par = 0) of
+// its row, k of the rows y +- 1 and z +- 1.  Arithmetic and order are those of
+// k_mg_sweep (the two x neighbours may change places in the first addition).
+constexpr int S2_NT = 512, S2_TX = 16, S2_TY = 8, S2_TZ = 8;
+constexpr int S2_K = (S2_TX + 8) / 2, S2_Y = S2_TY + 8, S2_Z = S2_TZ + 8, S2_E = S2_K * S2_Y * S2_Z;
+
+struct S2Lds {
+  float p[2][S2_E], hb[2][S2_E];
+  uint8_t c[2][S2_E];
+  float2 ct[64];
+};
+
+// One colour pass on the tile and a ring of R.  OUT: the pass's cells are not
+// stored but returned in *v (one a thread, with its entry in *e).
+template <int C, int R, bool ICNT, bool OUT>
+__device__ __forceinline__ void s2_pass(S2Lds &L, float omega, float wdir, float *v, int *e) {
+  constexpr int KN = S2_TX / 2 + R, RY = S2_TY + 2 * R, RZ = S2_TZ + 2 * R, PER = KN * RY, ZS = S2_NT / PER;
+  constexpr int N = (RZ + ZS - 1) / ZS;
+  static_assert(!OUT || (N == 1 && R == 0), "one output cell a thread");
+  const int t = threadIdx.x, zi = t / PER, r = t - zi * PER, yy = r / KN, kk = r - yy * KN;
+  const int ly = yy + 4 - R;
+  float *own = L.p[C];
+  const float *oth = L.p[1 - C];
+  uint32_t code[N];
+  float nb[N][6], cen[N], hb[N];
+  int id[N];
+  bool act[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    const int lz = zi + 4 - R + ZS * q;
+    act[q] = zi < ZS && (RZ % ZS == 0 || lz < 4 + S2_TZ + R);
+    const int par = (ly + lz + C) & 1;
+    const int i = (lz * S2_Y + ly) * S2_K + kk + ((5 - R - par) >> 1);
+    id[q] = act[q] ? i : S2_K * S2_Y + S2_K + 1;  // any interior entry
+    const int p = id[q];
+    code[q] = L.c[C][p];
+    nb[q][0] = oth[p];
+    nb[q][1] = oth[p + 2 * par - 1];
+    nb[q][2] = oth[p + S2_K];
+    nb[q][3] = oth[p - S2_K];
+    nb[q][4] = oth[p + S2_K * S2_Y];
+    nb[q][5] = oth[p - S2_K * S2_Y];
+    cen[q] = own[p];
+    hb[q] = L.hb[C][p];
+  }
+  float xs[N], qs[N];
+  bool redo = false;
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    float sum = nb[q][0];
+#pragma unroll
+    for (int k = 1; k < 6; k++) sum += nb[q][k];
+    xs[q] = sum - hb[q];
+    if (ICNT) {
+      const float2 cr = L.ct[code[q] & 63u];
+      const float q0 = xs[q] * cr.y;
+      const float er = __builtin_fmaf(-q0, cr.x, xs[q]);
+      qs[q] = __builtin_fmaf(er, cr.y, q0);
+      redo |= __builtin_amdgcn_classf(qs[q], 0x90);  // -subnormal | +subnormal
+    } else {
+      qs[q] = xs[q] / nc_count(code[q], wdir);
+    }
+  }
+  if (ICNT && redo) {
+#pragma unroll
+    for (int q = 0; q < N; q++)
+      if (__builtin_amdgcn_classf(qs[q], 0x90)) {
+        float x = xs[q];
+        asm volatile("" : "+v"(x));
+        qs[q] = x / L.ct[code[q] & 63u].x;
+      }
+  }
+#pragma unroll
+  for (int q = 0; q < N; q++) {
+    const float nv = mixf_(cen[q], qs[q], omega);
+    const float o = (code[q] & (NC_SOLID | NC_NONE)) ? cen[q] : nv;
+    if (OUT) {
+      *v = o;
+      *e = id[q];
+    } else if (act[q]) {
+      own[id[q]] = o;
+    }
+  }
+}
+
+// The four elements from `over` on (0 beyond the fourth).
+__device__ __forceinline__ float4 s2_shift(float4 v, int over) {
+  if (over == 1) return make_float4(v.y, v.z, v.w, 0.0f);
+  if (over == 2) return make_float4(v.z, v.w, 0.0f, 0.0f);
+  if (over == 3) return make_float4(v.w, 0.0f, 0.0f, 0.0f);
+  return v;
+}
+// The coarse level that a fused prolongation (PRO) reads: 14 x 10 x 10 cells
+// around the footprint, indices clamped to the level as in k_mg_prolong.
+constexpr int S2_CX = S2_K + 2, S2_CY = S2_Y / 2 + 2, S2_CZ = S2_Z / 2 + 2, S2_CN = S2_CX * S2_CY * S2_CZ;
+struct S2Coarse {
+  int c0, c1, c2;
+  const float *p;
+  const uint8_t *f;
+};
+template <bool PRO>
+struct S2CLds {
+  float p[S2_CN];
+  uint8_t f[S2_CN];
+};
+template <>
+struct S2CLds<false> {};
+
+// v[0..3] plus the masked, renormalised trilinear correction of mg.wgsl:97-120
+// (k_mg_prolong, whose weights and order of sums these are) for the four cells
+// from footprint x = 4 q at (ly, lz).  keep: cells that take no correction.
+__device__ __forceinline__ void s2_prolong(const S2CLds<true> &C, bool solid, int q, int ly, int lz, uint32_t keep,
+                                           float *v) {
+  // cells 2 m and 2 m + 1 lie between the coarse cells m - 1, m and m, m + 1
+  // with fractions 0.75 and 0.25; footprint cell 0 is even, and its m - 1 is
+  // entry 0 of the staged cells
+  const int base = (((lz + 1) >> 1) * S2_CY + ((ly + 1) >> 1)) * S2_CX + 2 * q;
+  const float fy = (ly & 1) ? 0.25f : 0.75f, fz = (lz & 1) ? 0.25f : 0.75f;
+  float pc[4][4], wyz[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {  // j = y offset + 2 z offset
+    const int e = base + ((j >> 1) * S2_CY + (j & 1)) * S2_CX;
+    wyz[j] = ((j & 1) ? fy : 1.0f - fy) * ((j >> 1) ? fz : 1.0f - fz);
+#pragma unroll
+    for (int k = 0; k < 4; k++) pc[j][k] = C.p[e + k];
+  }
+  // all weights are multiples of 1/64, so their products are exact in any order
+  if (!solid) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const float fx = (i & 1) ? 0.25f : 0.75f;
+      float acc = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 8; k++) acc += (((k & 1) ? fx : 1.0f - fx) * wyz[k >> 1]) * pc[k >> 1][(i + 1) / 2 + (k & 1)];
+      if (!((keep >> i) & 1u)) v[i] = v[i] + acc;
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float fx = (i & 1) ? 0.25f : 0.75f;
+    float acc = 0.0f, ws = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int j = k >> 1, m = (i + 1) / 2 + (k & 1);
+      const bool sol = C.f[base + ((j >> 1) * S2_CY + (j & 1)) * S2_CX + m] == 1;
+      const float w = sol ? 0.0f : ((k & 1) ? fx : 1.0f - fx) * wyz[j];
+      acc += w * pc[j][m];
+      ws += w;
+    }
+    float corr = acc;
+    if (ws != 1.0f) {
+      float x = acc;
+      asm volatile("" : "+v"(x));
+      corr = x / ws;
+    }
+    if (!((keep >> i) & 1u) && ws > 1e-4f) v[i] = v[i] + corr;
+  }
+}
+
+// ALN: the level's x-size is a multiple of 4 (whole float4 and code words);
+// otherwise the last group of a row is loaded from where it ends with the row
+// and shifted, its elements past the row are masked, and codes are loaded as
+// bytes.  The level has at most S2_MAX_ODD cells (32-bit offsets) and rows of
+// at least four (sweep2_fits).
+template <bool ALN, bool ICNT, bool PRO>
+__global__ __launch_bounds__(S2_NT) void k_mg_sweep2(LvArgs a, int ntx, int nty, const float *__restrict__ b,
+                                                      const uint8_t *__restrict__ nc, const float *__restrict__ pin,
+                                                      float *__restrict__ pout, float omega, S2Coarse co) {
+  __shared__ __align__(16) S2Lds L;
+  __shared__ S2CLds<PRO> LC;
+  const int t = threadIdx.x;
+  if (ICNT && t < 64) {
+    const uint32_t cnt = (t & 7u) + ((t >> 3) & 7u);
+    L.ct[t] = make_float2((float)cnt, cnt ? 1.0f / (float)cnt : 0.0f);
+  }
+  const int bid = xcd_tile(blockIdx.x, gridDim.x);
+  const int tx = bid % ntx, rr = bid / ntx, ty = rr % nty, tz = rr / nty;
+  const int x0 = tx * S2_TX - 4, y0 = ty * S2_TY - 4, z0 = tz * S2_TZ - 4;
+  const RB rp = rb_of(pin, pin ? a.n * 4u : 0u), rbb = rb_of(b, a.n * 4u), rcd = rb_of(nc, a.n);
+  constexpr int Q = S2_K / 2, NG = Q * S2_Y * S2_Z / S2_NT;
+  static_assert(Q * S2_Y * S2_Z == NG * S2_NT, "whole staging rounds");
+  float4 pv[NG], bv[NG];
+  uint32_t cv[NG];
+#pragma unroll
+  for (int i = 0; i < NG; i++) {
+    const int g = t + S2_NT * i, q = g % Q, row = g / Q, ly = row % S2_Y, lz = row / S2_Y;
+    const int gx = x0 + 4 * q, gy = y0 + ly, gz = z0 + lz;
+    const bool ok = (uint32_t)gx < (uint32_t)a.d0 && (uint32_t)gy < (uint32_t)a.d1 && (uint32_t)gz < (uint32_t)a.d2;
+    const uint32_t n = (uint32_t)gx + (uint32_t)a.d0 * ((uint32_t)gy + (uint32_t)a.d1 * (uint32_t)gz);
+    const int over = !ALN && gx + 4 > a.d0 ? gx + 4 - a.d0 : 0;  // elements past the row's end
+    pv[i] = rb_ld4(rp, ok ? 4u * (n - over) : RB_OOB);
+    bv[i] = rb_ld4(rbb, ok ? 4u * (n - over) : RB_OOB);
+    if (ALN) {
+      const uint32_t c = rb_ld32(rcd, ok ? n : RB_OOB);
+      cv[i] = ok ? c : 0x40404040u;
+    } else {
+      uint32_t c = 0u;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const bool okj = ok && gx + j < a.d0;
+        const uint32_t cj = __builtin_amdgcn_raw_buffer_load_b8(rcd.r, okj ? n + j : RB_OOB, 0, 0);
+        c |= (okj ? cj : (uint32_t)NC_NONE) << (8 * j);
+      }
+      cv[i] = c;
+    }
+  }
+  bool solid = false;
+  if constexpr (PRO) {
+#pragma unroll
+    for (int i = 0; i < (S2_CN + S2_NT - 1) / S2_NT; i++) {
+      const int g = min(t + S2_NT * i, S2_CN - 1), u = g % S2_CX, r = g / S2_CX;
+      const int cx = clampi(x0 / 2 - 1 + u, 0, co.c0 - 1), cy = clampi(y0 / 2 - 1 + r % S2_CY, 0, co.c1 - 1);
+      const int cz = clampi(z0 / 2 - 1 + r / S2_CY, 0, co.c2 - 1);
+      const uint32_t j = (uint32_t)cx + (uint32_t)co.c0 * ((uint32_t)cy + (uint32_t)co.c1 * (uint32_t)cz);
+      LC.p[g] = co.p[j];
+      const uint8_t fl = co.f[j];
+      LC.f[g] = fl;
+      solid |= fl == 1;
+    }
+    solid = __syncthreads_or(solid);
+  }
+#pragma unroll
+  for (int i = 0; i < NG; i++) {
+    const int g = t + S2_NT * i, q = g % Q, row = g / Q, ly = row % S2_Y, lz = row / S2_Y;
+    float4 v = pv[i], w = bv[i];
+    const uint32_t c = cv[i];
+    if (!ALN) {
+      const int over = x0 + 4 * q + 4 - a.d0;
+      v = s2_shift(v, over);
+      w = s2_shift(w, over);
+    }
+    if constexpr (PRO) {
+      const int gx = x0 + 4 * q, gy = y0 + ly, gz = z0 + lz;
+      if ((uint32_t)gx < (uint32_t)a.d0 && (uint32_t)gy < (uint32_t)a.d1 && (uint32_t)gz < (uint32_t)a.d2) {
+        float vv[4] = {v.x, v.y, v.z, v.w};
+        const uint32_t keep = ALN || gx + 4 <= a.d0 ? 0u : (0xfu << (a.d0 - gx));  // past the row's end
+        s2_prolong(LC, solid, q, ly, lz, keep, vv);
+        v = make_float4(vv[0], vv[1], vv[2], vv[3]);
+      }
+    }
+    if (c & 0x80808080u) {  // solids read 0 in the neighbour sums
+      if (c & 0x80u) v.x = 0.0f;
+      if (c & 0x8000u) v.y = 0.0f;
+      if (c & 0x800000u) v.z = 0.0f;
+      if (c & 0x80000000u) v.w = 0.0f;
+    }
+    const int e = row * S2_K + 2 * q, o = (ly + lz) & 1;  // o: colour of the group's even cells
+    *reinterpret_cast<float2 *>(L.p[o] + e) = make_float2(v.x, v.z);
+    *reinterpret_cast<float2 *>(L.p[1 - o] + e) = make_float2(v.y, v.w);
+    *reinterpret_cast<float2 *>(L.hb[o] + e) = make_float2(a.hh * w.x, a.hh * w.z);
+    *reinterpret_cast<float2 *>(L.hb[1 - o] + e) = make_float2(a.hh * w.y, a.hh * w.w);
+    *reinterpret_cast<uint16_t *>(L.c[o] + e) = (uint16_t)((c & 0xffu) | ((c >> 8) & 0xff00u));
+    *reinterpret_cast<uint16_t *>(L.c[1 - o] + e) = (uint16_t)(((c >> 8) & 0xffu) | ((c >> 16) & 0xff00u));
+  }
+  __syncthreads();
+  s2_pass<0, 3, ICNT, false>(L, omega, a.wdir, nullptr, nullptr);
+  __syncthreads();
+  s2_pass<1, 2, ICNT, false>(L, omega, a.wdir, nullptr, nullptr);
+  __syncthreads();
+  s2_pass<0, 1, ICNT, false>(L, omega, a.wdir, nullptr, nullptr);
+  __syncthreads();
+  float v1;
+  int e;
+  s2_pass<1, 0, ICNT, true>(L, omega, a.wdir, &v1, &e);
+  // the thread's colour-1 cell and its pair's colour-0 cell
+  const int row = e / S2_K, k = e - row * S2_K, ly = row % S2_Y, lz = row / S2_Y;
+  const int gx = x0 + 2 * k, gy = y0 + ly, gz = z0 + lz;
+  if (gx >= a.d0 || gy >= a.d1 || gz >= a.d2) return;
+  const int o = (ly + lz) & 1;  // colour of the pair's even cell
+  const float v0 = L.p[0][e];
+  float lo = o ? v1 : v0, hi = o ? v0 : v1;
+  const uint32_t n = (uint32_t)gx + (uint32_t)a.d0 * ((uint32_t)gy + (uint32_t)a.d1 * (uint32_t)gz);
+  const bool second = ALN || gx + 1 < a.d0;
+  if (pin) {  // solid cells keep their phi (zeroed only in LDS)
+    if (L.c[o][e] & NC_SOLID) lo = pin[n];
+    if (second && (L.c[1 - o][e] & NC_SOLID)) hi = pin[n + 1];
+  }
+  if (ALN) {
+    *reinterpret_cast<float2 *>(pout + n) = make_float2(lo, hi);
+  } else {
+    pout[n] = lo;
+    if (second) pout[n + 1] = hi;
+  }
+}
+
+// Levels that take both sweeps in one launch.  The tile's rings cost 2.4
+// updates a cell and sweep against 1.5, so the launch saved (two, with the
+// prolongation) has to be worth more than the work: four V-cycles with and
+// without it for the level of n cells:
+//   40x80x40 (128 k)   514 us before, 467 now     48x32x48 (74 k)  299, 278
+//   80x120x80 (768 k)  1312 (its finer level apart), 1300
+//   80x160x80 (1.02 M) 467 without, 479 with      160x320x160      1498, 1844
+//   a solve at 96^3 (885 k)  2960 us without, 2893 with; 128^3 (2.1 M) 4453, 4727
+// Rows that are no multiple of four cells take k_mg_sweep one element at a
+// time, and there the line lies higher: a solve at 97x61x118 5594 us before,
+// 4101 now; 129^3 (2.1 M) 9721 without, 9325 with; 193x121x235 (5.5 M) 17.45
+// ms, 17.38; 255^3 30.8, 31.9.
+constexpr uint32_t S2_MAX = 900000u, S2_MAX_ODD = 4000000u;
+static bool sweep2_fits(const MgLevel &L) { return L.d[0] >= 4 && L.n <= (L.d[0] % 4 ? S2_MAX_ODD : S2_MAX); }
+// C: the level whose correction is added first, or null
+static void launch_mg_sweep2(const MgLevel &L, const MgLevel *C, const float *pin, float *pout, float omega,
+                             hipStream_t s) {
+  const LvArgs a = lv_args(L);
+  const int ntx = (L.d[0] + S2_TX - 1) / S2_TX, nty = (L.d[1] + S2_TY - 1) / S2_TY, ntz = (L.d[2] + S2_TZ - 1) / S2_TZ;
+  const int nb = ntx * nty * ntz;
+  const S2Coarse co = C ? S2Coarse{C->d[0], C->d[1], C->d[2], C->phi, C->f} : S2Coarse{};
+#define PYRO_SWEEP2(A_, I_, P_) \
+  k_mg_sweep2<A_, I_, P_><<<nb, S2_NT, 0, s>>>(a, ntx, nty, L.b, L.nc, pin, pout, omega, co)
+  const int k = (L.d[0] % 4 == 0 ? 4 : 0) + (L.wdir == 1.0f ? 2 : 0) + (C ? 1 : 0);
+  switch (k) {
+    case 0: PYRO_SWEEP2(false, false, false); break;
+    case 1: PYRO_SWEEP2(false, false, true); break;
+    case 2: PYRO_SWEEP2(false, true, false); break;
+    case 3: PYRO_SWEEP2(false, true, true); break;
+    case 4: PYRO_SWEEP2(true, false, false); break;
+    case 5: PYRO_SWEEP2(true, false, true); break;
+    case 6: PYRO_SWEEP2(true, true, false); break;
+    default: PYRO_SWEEP2(true, true, true); break;
+  }
+#undef PYRO_SWEEP2
+}
+
 // ---------------------------------------------------------------- coarse
 // All red-black SOR iterations of the coarsest level in one workgroup
 // (sim.rs:472-473: 80 iterations, omega = 1.6).  phi lives in a zero-padded
@@ -1785,23 +2117,35 @@ void launch_mg_resid(const MgLevel &L, StatParts *st, hipStream_t s) {
 
 // ---------------------------------------------------------------- V-cycle
 void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero) {
-  auto sweeps = [&](const MgLevel &L, bool fine, bool zero = false) {
-    launch_mg_sweep(L, zero ? nullptr : L.phi, L.tmp, 1.0f, s, fine);
-    launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, fine);
-  };
   // the levels from t on run in one launch where they fit
   int t = nl - 1;
   while (t > 0 && tail_fits(lv, t - 1, nl)) t--;
   if (from_zero && t == 0) launch_zero32(lv[0].n, lv[0].phi, s);  // the tail reads phi
+  // smoothing: two sweeps phi -> tmp -> phi, or both in one launch, phi ->
+  // tmp before the coarser level and tmp -> phi, with the prolongation, after it
   for (int l = 0; l < t; l++) {
-    sweeps(lv[l], l == 0, from_zero && l == 0);
-    launch_mg_restrict(lv[l], lv[l + 1], s);
+    MgLevel L = lv[l];
+    const float *pin = (l > 0 || from_zero) ? nullptr : L.phi;  // a restricted level starts from 0
+    if (sweep2_fits(L)) {
+      launch_mg_sweep2(L, nullptr, pin, L.tmp, 1.0f, s);
+      L.phi = L.tmp;
+    } else {
+      launch_mg_sweep(L, pin, L.tmp, 1.0f, s, l == 0);
+      launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, l == 0);
+    }
+    launch_mg_restrict(L, lv[l + 1], s);
   }
   if (t < nl - 1) launch_mg_tail(lv, t, nl, coarse_iters, 1.6f, s);
   else launch_mg_coarse(lv[t], coarse_iters, 1.6f, s);
   for (int l = t - 1; l >= 0; l--) {
-    launch_mg_prolong(lv[l + 1], lv[l], s);
-    sweeps(lv[l], l == 0);
+    MgLevel L = lv[l];
+    if (sweep2_fits(L)) {
+      launch_mg_sweep2(L, &lv[l + 1], L.tmp, L.phi, 1.0f, s);
+    } else {
+      launch_mg_prolong(lv[l + 1], L, s);
+      launch_mg_sweep(L, L.phi, L.tmp, 1.0f, s, l == 0);
+      launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, l == 0);
+    }
   }
 }
 
