@@ -8,8 +8,8 @@
 //
 // The reference dispatches the coarsest level's 80 red-black SOR iterations
 // as 160 separate passes; here they run in one workgroup with phi, b and the
-// solid mask resident in LDS (160 KB per CU on gfx950), one barrier per
-// colour pass.
+// solid mask on chip (160 KB of LDS per CU on gfx950), one barrier per colour
+// pass, or, where a level is too large for that, as 40 launches.
 #include "kernels.hpp"
 
 namespace pyro {
@@ -1112,107 +1112,13 @@ static void launch_mg_sweep2(const MgLevel &L, const MgLevel *C, const float *pi
 }
 
 // ---------------------------------------------------------------- coarse
-// All red-black SOR iterations of the coarsest level in one workgroup
-// (sim.rs:472-473: 80 iterations, omega = 1.6).  phi lives in a zero-padded
-// LDS grid (the ghost ring is the Dirichlet phi = 0 of mg.wgsl:29, solids are
-// zeroed as in the sweep); each thread owns up to CO_K cells per colour and
-// keeps their LDS index, count and h^2 b in registers.  Within one colour
-// pass no cell reads a cell of its own colour, so the loads of a chunk of
-// CO_C cells are issued together before any store.
-constexpr int CO_NT = 1024, CO_K = 8, CO_C = 2;
-constexpr int CO_PAD_MAX = 36000;  // padded cells: 144 KB of LDS (< 65536: 16-bit index)
+// All red-black SOR iterations of the coarsest level (sim.rs:472-473: 80
+// iterations, omega = 1.6): in the tail's workgroup up to about 12 k cells, in
+// one workgroup with a thread per column (below), or else as sweep launches.
+constexpr int CO_NT = 1024;
+constexpr int CO_PAD_MAX = 36000;  // floats of the column solve's LDS (144 KB)
 
-__global__ __launch_bounds__(CO_NT) void k_mg_coarse(LvArgs a, const float *__restrict__ b,
-                                                      const uint8_t *__restrict__ f, const uint8_t *__restrict__ nc,
-                                                      float *__restrict__ p, int iters, float omega) {
-  __shared__ float sp[CO_PAD_MAX];
-  const int P0 = a.d0 + 2, P1 = a.d1 + 2, P2 = a.d2 + 2;
-  const int PN = P0 * P1 * P2;
-  const uint32_t sy = (uint32_t)a.d0, sz = (uint32_t)a.d0 * (uint32_t)a.d1;
-  const int nt = (int)blockDim.x;  // whole waves covering a colour's cells
-  for (int i = threadIdx.x; i < PN; i += nt) {
-    int lx = i % P0, t = i / P0, ly = t % P1, lz = t / P1;
-    int gx = lx - 1, gy = ly - 1, gz = lz - 1;
-    float v = 0.0f;
-    if (gx >= 0 && gy >= 0 && gz >= 0 && gx < a.d0 && gy < a.d1 && gz < a.d2) {
-      uint32_t g = (uint32_t)gx + sy * (uint32_t)gy + sz * (uint32_t)gz;
-      v = f[g] == 1 ? 0.0f : p[g];
-    }
-    sp[i] = v;
-  }
-  // per owned cell: LDS index (bits 0-15) | fluid (16-18) | outside (19-21) | active (31);
-  // an inactive slot points at grid cell (0, 0, 0), whose six neighbours
-  // are inside the padded array, and is never stored
-  const uint32_t idle = (uint32_t)(1 + P0 + P0 * P1);
-  uint32_t pk[2][CO_K];
-  float hb[2][CO_K];
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-#pragma unroll
-    for (int j = 0; j < CO_K; j++) {
-      pk[c][j] = idle;
-      hb[c][j] = 0.0f;
-      uint32_t t = threadIdx.x + (uint32_t)j * (uint32_t)nt;
-      if (t >= a.nhalf) continue;
-      uint32_t r = fdiv(t, a.dhx);
-      int gxh = (int)(t - r * a.dhx.d);
-      uint32_t zq = fdiv(r, a.dny);
-      int y = (int)(r - zq * (uint32_t)a.d1), z = (int)zq;
-      int x = 2 * gxh + ((y + z + c) & 1);
-      if (x >= a.d0) continue;
-      uint32_t g = (uint32_t)x + sy * (uint32_t)y + sz * (uint32_t)z;
-      uint8_t code = nc[g];
-      if (code & (NC_SOLID | NC_NONE)) continue;
-      uint32_t li = (uint32_t)(((z + 1) * P1 + (y + 1)) * P0 + (x + 1));
-      pk[c][j] = li | ((uint32_t)(code & 63u) << 16) | 0x80000000u;
-      hb[c][j] = a.hh * b[g];
-    }
-  }
-  __syncthreads();
-  const int o1 = 1, o2 = P0, o3 = P0 * P1;
-  for (int it = 0; it < iters; it++) {
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-#pragma unroll
-      for (int j0 = 0; j0 < CO_K; j0 += CO_C) {
-        if ((uint32_t)j0 * (uint32_t)nt >= a.nhalf) break;  // no thread owns a cell here (uniform)
-        float nb[CO_C][7];
-#pragma unroll
-        for (int q = 0; q < CO_C; q++) {
-          const int i = (int)(pk[c][j0 + q] & 0xffffu);
-          nb[q][0] = sp[i + o1]; nb[q][1] = sp[i - o1]; nb[q][2] = sp[i + o2];
-          nb[q][3] = sp[i - o2]; nb[q][4] = sp[i + o3]; nb[q][5] = sp[i - o3];
-          nb[q][6] = sp[i];
-        }
-#pragma unroll
-        for (int q = 0; q < CO_C; q++) {
-          const uint32_t w = pk[c][j0 + q];
-          float sum = 0.0f;
-          sum += nb[q][0];
-          sum += nb[q][1];
-          sum += nb[q][2];
-          sum += nb[q][3];
-          sum += nb[q][4];
-          sum += nb[q][5];
-          const float cnt = nc_count(w >> 16, a.wdir);
-          const float nv = mixf_(nb[q][6], (sum - hb[c][j0 + q]) / cnt, omega);
-          if (w & 0x80000000u) sp[(int)(w & 0xffffu)] = nv;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int i = threadIdx.x; i < PN; i += nt) {
-    int lx = i % P0, t = i / P0, ly = t % P1, lz = t / P1;
-    int gx = lx - 1, gy = ly - 1, gz = lz - 1;
-    if (gx >= 0 && gy >= 0 && gz >= 0 && gx < a.d0 && gy < a.d1 && gz < a.d2) {
-      uint32_t g = (uint32_t)gx + sy * (uint32_t)gy + sz * (uint32_t)gz;
-      if (f[g] != 1) p[g] = sp[i];
-    }
-  }
-}
-
-// The same solve with one thread per (x, y) column and the column's phi in
+// The solve with one thread per (x, y) column and the column's phi in
 // registers, for an outside weight of 1 (integer counts 1..6, div_count).
 // LDS holds phi plane-major: plane z + 1 (z = -1 .. ZJ - 1) of CZ_PLANE
 // floats, the cell of column c = x + d0 * y at offset c.  CZ_PLANE is a
@@ -2020,12 +1926,6 @@ static void launch_mg_tail(const MgLevel *lv, int t, int nl, int iters, float om
   }
 }
 
-bool mg_coarse_fits_lds(const MgLevel &L) {
-  uint32_t pad = (uint32_t)(L.d[0] + 2) * (uint32_t)(L.d[1] + 2) * (uint32_t)(L.d[2] + 2);
-  uint32_t half = (uint32_t)((L.d[0] + 1) / 2) * (uint32_t)L.d[1] * (uint32_t)L.d[2];
-  return pad <= (uint32_t)CO_PAD_MAX && half <= (uint32_t)(CO_NT * CO_K);
-}
-
 void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
   LvArgs a = lv_args(L);
   const int ncol = L.d[0] * L.d[1];
@@ -2070,17 +1970,19 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
     }
     return;
   }
-  if (mg_coarse_fits_lds(L)) {
-    // one cell of a colour per thread where that fits, whole waves only
-    // (the level fits: nhalf <= CO_NT * CO_K)
-    const uint32_t nt = a.nhalf >= (uint32_t)CO_NT ? (uint32_t)CO_NT : ((a.nhalf + 63u) / 64u) * 64u;
-    k_mg_coarse<<<1, nt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
-  }
-  else {
-    for (int it = 0; it < iters; it += 2) {
-      launch_mg_sweep(L, L.phi, L.tmp, omega, s, false);
-      launch_mg_sweep(L, L.tmp, L.phi, omega, s, false);
+  // Two iterations a launch.  22x32x22 (15.5 k cells) 330 us in one workgroup
+  // with phi in LDS, 259 now; at one iteration a launch 26x38x26 took 778 us
+  // (rows that are no multiple of four), now 260, and 40x60x40 319, now 241.
+  // The column solve above takes 165 us for 20x40x20.
+  int it = 0;
+  if (sweep2_fits(L))
+    for (; it + 4 <= iters; it += 4) {
+      launch_mg_sweep2(L, nullptr, L.phi, L.tmp, omega, s);
+      launch_mg_sweep2(L, nullptr, L.tmp, L.phi, omega, s);
     }
+  for (; it < iters; it += 2) {
+    launch_mg_sweep(L, L.phi, L.tmp, omega, s, false);
+    launch_mg_sweep(L, L.tmp, L.phi, omega, s, false);
   }
 }
 

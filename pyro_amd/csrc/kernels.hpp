@@ -85,9 +85,8 @@ void launch_mg_setup(const MgLevel *L, int nl, hipStream_t s);
 void launch_mg_sweep(const MgLevel &L, const float *pin, float *pout, float omega, hipStream_t s, bool fine);
 void launch_mg_restrict(const MgLevel &F, const MgLevel &C, hipStream_t s);
 void launch_mg_prolong(const MgLevel &C, const MgLevel &F, hipStream_t s);
-// All `iters` red-black sweeps of the coarsest level in one launch.
+// All `iters` (even) red-black sweeps of the coarsest level.
 void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s);
-bool mg_coarse_fits_lds(const MgLevel &L);
 void launch_mg_resid(const MgLevel &L, StatParts *st, hipStream_t s);
 int mg_resid_blocks(const MgLevel &L);
 

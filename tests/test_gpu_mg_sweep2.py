@@ -1,5 +1,5 @@
 """Levels whose two sweeps run in one launch (k_mg_sweep2, 16 x 8 x 8 tiles),
-with the prolongation before them: sizes around the tile, rows of every
+with the prolongation before them or as the coarsest level's solve: sizes around the tile, rows of every
 remainder of four, the smallest row it takes and one below it, and both sides
 of the size where single sweeps take over.  Random solid blocks."""
 import pytest
@@ -19,6 +19,9 @@ pytestmark = pytest.mark.gpu
     ((35, 16, 200), 2),
     ((96, 96, 96), 4),    # the last size of whole rows
     ((100, 96, 96), 4),   # single sweeps on level 0
+    ((23, 45, 15), 1),    # a coarsest level solved by sweeps, odd rows
+    ((24, 46, 15), 1),    # and whole rows
+    ((48, 72, 15), 1),
 ])
 def test_two_sweeps_bitwise_equal_oracle(dims, levels):
     _vcycles_match_oracle(dims, levels, blocks=5)
