@@ -190,6 +190,12 @@ __device__ __forceinline__ int xcd_tile(int bid, int nb) {
   return (bid & 7) * q + (bid >> 3);
 }
 
+// The block of a launch of nb blocks that xcd_tile gives tile t.
+__device__ __forceinline__ int xcd_block(int t, int nb) {
+  const int q = nb >> 3;
+  return t >= (q << 3) ? t : (t % q) * 8 + t / q;
+}
+
 // Deterministic block reductions (fixed pairing order) for FP64 stats.
 // v[first] + v[first + step] + ... (count terms), added in that order from
 // 0 with eight loads in flight: the bits of the plain loop, without a load

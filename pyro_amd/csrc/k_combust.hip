@@ -28,9 +28,15 @@ __device__ __forceinline__ bool isSolidS(const Params *__restrict__ P, float4 s)
   return s.y + s.z > P->burnout;
 }
 
+// The same with the kinds of the eight slots in LDS: a lane's slot is its own,
+// and out of Params it is a load from memory for every cell tested.
+__device__ __forceinline__ bool isSolidK(const Params *__restrict__ P, const uint32_t *kinds, float4 s) {
+  return kinds[slotOf(s)] == 2u ? s.y > 0.5f : s.y + s.z > P->burnout;
+}
+
 // Radiative transfer along one ray of 10 strided steps (combust.wgsl:18-39).
 __device__ __forceinline__ float rayIrr(const Params *__restrict__ P, const Geo &g, const float4 *__restrict__ solIn,
-                        const float4 *__restrict__ s0, int px, int py, int pz, int dx_, int dy_, int dz_) {
+                        const float4 *__restrict__ s0, const uint32_t *kinds, int px, int py, int pz, int dx_, int dy_, int dz_) {
   // strides 1,1,1,2,2,3,4,5,7,9 packed one per nibble (no private array)
   const uint64_t strides = 0x9754322111ull;
   // The sample points do not depend on the marching, so each half of the ray
@@ -56,22 +62,27 @@ __device__ __forceinline__ float rayIrr(const Params *__restrict__ P, const Geo 
       py += dy_ * sd;
       pz += dz_ * sd;
     }
+    // what a sample contributes does not depend on the march either
+    float e[5], src[5];
 #pragma unroll
     for (int u = 0; u < 5; u++) {
-      const int st = 5 * h + u;
+      const int sd = (int)((strides >> (4 * (5 * h + u))) & 15u);
+      const float T = q[u].x, len = (float)sd * dl;
+      const bool sol = isSolidK(P, kinds, so[u]);
+      e[u] = sol ? 2.0f : 1.0f - pexp(-kapP(P, T, q[u].z, q[u].w) * len);  // 2: a solid cell
+      src[u] = pow4(sol ? so[u].w : T);
+    }
+#pragma unroll
+    for (int u = 0; u < 5; u++) {
       if (done || !in[u]) { done = true; break; }
-      if (isSolidS(P, so[u])) {
-        acc += tr * pow4(so[u].w);
+      if (e[u] == 2.0f) {
+        acc += tr * src[u];
         tr = 0.0f;
         done = true;
         break;
       }
-      const float T = q[u].x;
-      const int sd = (int)((strides >> (4 * st)) & 15u);
-      const float len = (float)sd * dl;
-      const float e = 1.0f - pexp(-kapP(P, T, q[u].z, q[u].w) * len);
-      acc += tr * e * pow4(T);
-      tr *= 1.0f - e;
+      acc += tr * e[u] * src[u];
+      tr *= 1.0f - e[u];
     }
     if (done) break;
   }
@@ -97,29 +108,40 @@ __device__ __forceinline__ void rayDir(int k, int r, int &dx_, int &dy_, int &dz
   dy_ += s * (second ? t2y : t1y);
   dz_ += s * (second ? t2z : t1z);
 }
-// Faces of a solid cell whose irradiance the cell needs (combust.wgsl:60-75):
-// bit k set for a neighbour in direction k (dirOf) that is inside the grid,
-// not below the ground and not solid.  Inert cells (kind 2) need none.
-__device__ __forceinline__ uint32_t ray_faces(const Params *__restrict__ P, const Geo &g,
-                                              const float4 *__restrict__ solIn, int x, int y, int z, float4 so) {
-  if (kindOf(P, so) == 2u) return 0u;
-  uint32_t mask = 0u;
+// The six neighbours of a solid cell (combust.wgsl:60-75), loaded together (one
+// outside the grid at the cell itself): the direction's bit in `in` if it is
+// inside the grid, in `solid` if it is solid as well, and its temperature.
+struct Nbrs {
+  uint32_t in, solid;
+  float T[6];
+};
+__device__ __forceinline__ Nbrs solid_nbrs(const Params *__restrict__ P, const Geo &g,
+                                           const float4 *__restrict__ solIn, const uint32_t *kinds, uint32_t i, int x,
+                                           int y, int z) {
+  Nbrs n;
+  n.in = n.solid = 0u;
+  float4 s[6];
 #pragma unroll
   for (int k = 0; k < 6; k++) {
     int dx_, dy_, dz_;
     dirOf(k, dx_, dy_, dz_);
-    const int nx_ = x + dx_, ny_ = y + dy_, nz_ = z + dz_;
-    if (ny_ < 0 || !inb(g, nx_, ny_, nz_)) continue;
-    if (!isSolidS(P, solIn[sidx(g, nx_, ny_, nz_)])) mask |= 1u << k;
+    const bool in = inb(g, x + dx_, y + dy_, z + dz_);
+    s[k] = solIn[in ? sidx(g, x + dx_, y + dy_, z + dz_) : i];
+    n.in |= in ? 1u << k : 0u;
   }
-  return mask;
+#pragma unroll
+  for (int k = 0; k < 6; k++) {
+    n.T[k] = s[k].w;
+    n.solid |= isSolidK(P, kinds, s[k]) ? n.in & (1u << k) : 0u;
+  }
+  return n;
 }
 
 // Surface energy balance and pyrolysis of one solid cell (combust.wgsl:60-128).
-// The irradiance of the cell's ray faces (ray_faces) is given: face k at
-// irr[popc(mask & ((1 << k) - 1))].
-__device__ __forceinline__ void solid_cell(const Params *__restrict__ P, const Geo &g, const float4 *__restrict__ solIn,
-                                        const float4 *__restrict__ s0, int x, int y, int z, float4 so,
+// The irradiance of the cell's ray faces (the neighbours inside the grid that
+// are not solid: mask) is given: face k at irr[popc(mask & ((1 << k) - 1))].
+__device__ __forceinline__ void solid_cell(const Params *__restrict__ P, const Geo &g, const Nbrs &nb,
+                                        const float4 *__restrict__ s0, uint32_t i, int x, int y, int z, float4 so,
                                         const float *irr, uint32_t mask, float4 &o, float4 &po, uint32_t &fl,
                                         float &stPyro, float &stMass, float &stArea) {
   fl = 1;
@@ -128,24 +150,24 @@ __device__ __forceinline__ void solid_cell(const Params *__restrict__ P, const G
   float fuel = so.y, chr = so.z, Ts = so.w;
   if (kind != 2u) {
     float nF = 0.0f, Tg = 0.0f, Yo = 0.0f, qin = 0.0f, qcond = 0.0f;
+    float4 q[6];
+#pragma unroll
     for (int k = 0; k < 6; k++) {
       int dx_, dy_, dz_;
       dirOf(k, dx_, dy_, dz_);
-      int nx_ = x + dx_, ny_ = y + dy_, nz_ = z + dz_;
-      if (ny_ < 0) continue;
-      bool nin = inb(g, nx_, ny_, nz_);
-      if (nin) {
-        float4 sn = solIn[sidx(g, nx_, ny_, nz_)];
-        if (isSolidS(P, sn)) {
-          qcond += m.b[3] / P->dx * (sn.w - Ts);
-          continue;
-        }
+      q[k] = s0[(nb.in >> k) & 1u ? sidx(g, x + dx_, y + dy_, z + dz_) : i];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+      if (k == 3 && y == 0) continue;  // the ground
+      if ((nb.solid >> k) & 1u) {
+        qcond += m.b[3] / P->dx * (nb.T[k] - Ts);
+        continue;
       }
       nF += 1.0f;
-      if (nin) {
-        float4 q = s0[sidx(g, nx_, ny_, nz_)];
-        Tg += q.x;
-        Yo += q.z;
+      if ((nb.in >> k) & 1u) {
+        Tg += q[k].x;
+        Yo += q[k].z;
         qin += irr[__popc(mask & ((1u << k) - 1u))];
       } else {
         Tg += P->t0;
@@ -220,65 +242,70 @@ constexpr uint8_t FLAG_BURNT = 2;
 // its own slot, so the listing order does not matter.  (One thread per cell
 // marched up to 6 faces in turn, and its wave every face any of its cells
 // needed.)
+struct SolidLds {
+  uint16_t fm[6 * NT];  // listed face: thread << 3 | k
+  float fi[6 * NT];     // its irradiance
+  float ray[5 * NT];    // the rays of a batch of NT faces
+  uint32_t kinds[8];    // kindOf each slot
+  int nf;
+};
+// The pass over the NT cells from c0 (a block's tile), their flags given; `p`
+// is the tile's place among the partials.  A tile without solid or burnt cells
+// has nothing to do (its statistics partials are +0).
 template <bool STATS>
-__device__ __forceinline__ void solid_block(const Params *__restrict__ P, const Geo &g,
-                                            const float4 *__restrict__ solIn, float4 *__restrict__ solOut,
-                                            float4 *__restrict__ pyr, uint8_t *__restrict__ flags,
-                                            const float4 *__restrict__ s0, double *__restrict__ part) {
-  __shared__ uint16_t sfm[6 * NT];  // listed face: thread << 3 | k
-  __shared__ float sfi[6 * NT];     // its irradiance
-  __shared__ float sray[5 * NT];    // the rays of a batch of NT faces
-  __shared__ int snf;
-  const uint32_t c0 = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT;
+__device__ __forceinline__ void solid_tile(const Params *__restrict__ P, const Geo &g, SolidLds &L,
+                                           const float4 *__restrict__ solIn, float4 *__restrict__ solOut,
+                                           float4 *__restrict__ pyr, uint8_t *__restrict__ flags,
+                                           const float4 *__restrict__ s0, double *__restrict__ part, uint32_t c0,
+                                           uint32_t p, uint8_t fprev) {
   const uint32_t i = c0 + threadIdx.x;
   float stPyro = 0.0f, stMass = 0.0f, stArea = 0.0f;
-  if (threadIdx.x == 0) snf = 0;
-  const uint8_t fprev = i < g.n ? flags[i] : 0;
-  int x = 0, y = 0, z = 0;
-  float4 so = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  uint32_t mask = 0u;
-  if (fprev == 1) {
-    so = solIn[i];
-    decode_cell(g, i, x, y, z);
-    mask = ray_faces(P, g, solIn, x, y, z, so);
-  }
-  // snf = 0 is visible after this barrier; a block without solid or burnt
-  // cells has nothing to do (its statistics partials are +0)
+  if (threadIdx.x == 0) L.nf = 0;  // visible after the barrier
   if (!__syncthreads_or(fprev != 0)) {
     if (STATS && threadIdx.x == 0) {
-      part[blockIdx.x * 3 + 0] = 0.0;
-      part[blockIdx.x * 3 + 1] = 0.0;
-      part[blockIdx.x * 3 + 2] = 0.0;
+      part[p * 3 + 0] = 0.0;
+      part[p * 3 + 1] = 0.0;
+      part[p * 3 + 2] = 0.0;
     }
     return;
   }
+  int x = 0, y = 0, z = 0;
+  float4 so = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  Nbrs nb = {};
+  uint32_t mask = 0u;  // faces whose irradiance the cell needs (inert cells: none)
+  if (fprev == 1) {
+    so = solIn[i];
+    decode_cell(g, i, x, y, z);
+    nb = solid_nbrs(P, g, solIn, L.kinds, i, x, y, z);
+    if (L.kinds[slotOf(so)] != 2u) mask = nb.in & ~nb.solid;
+  }
   int base = 0;
   if (mask) {
-    base = atomicAdd(&snf, __popc(mask));
+    base = atomicAdd(&L.nf, __popc(mask));
     int s = base;
 #pragma unroll
     for (int k = 0; k < 6; k++)
-      if (mask & (1u << k)) sfm[s++] = (uint16_t)((threadIdx.x << 3) | k);
+      if (mask & (1u << k)) L.fm[s++] = (uint16_t)((threadIdx.x << 3) | k);
   }
   __syncthreads();
   // the listed faces in batches of NT: the batch's rays one per thread, then
   // each face's five rays summed in faceIrr's order
-  const int nf = snf;
+  const int nf = L.nf;
   for (int f0 = 0; f0 < nf; f0 += NT) {
     const int nr = 5 * (nf - f0 < NT ? nf - f0 : NT);
     for (int j = threadIdx.x; j < nr; j += NT) {
       const int f = f0 + j / 5, r = j - 5 * (j / 5);
-      const int owner = sfm[f] >> 3, k = sfm[f] & 7;
+      const int owner = L.fm[f] >> 3, k = L.fm[f] & 7;
       int ox, oy, oz, nx_, ny_, nz_, dx_, dy_, dz_;
       decode_cell(g, c0 + (uint32_t)owner, ox, oy, oz);
       dirOf(k, nx_, ny_, nz_);
       rayDir(k, r, dx_, dy_, dz_);
-      sray[j] = rayIrr(P, g, solIn, s0, ox + nx_, oy + ny_, oz + nz_, dx_, dy_, dz_);
+      L.ray[j] = rayIrr(P, g, solIn, s0, L.kinds, ox + nx_, oy + ny_, oz + nz_, dx_, dy_, dz_);
     }
     __syncthreads();
     for (int j = threadIdx.x; j < nr / 5; j += NT) {
-      const float *q = sray + 5 * j;
-      sfi[f0 + j] = 0.2f * ((((q[0] + q[1]) + q[2]) + q[3]) + q[4]);
+      const float *q = L.ray + 5 * j;
+      L.fi[f0 + j] = 0.2f * ((((q[0] + q[1]) + q[2]) + q[3]) + q[4]);
     }
     __syncthreads();
   }
@@ -290,7 +317,7 @@ __device__ __forceinline__ void solid_block(const Params *__restrict__ P, const 
     } else if (fprev == 1) {
       float4 o = so, po = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       uint32_t fl = 0;
-      solid_cell(P, g, solIn, s0, x, y, z, so, sfi + base, mask, o, po, fl, stPyro, stMass, stArea);
+      solid_cell(P, g, nb, s0, i, x, y, z, so, L.fi + base, mask, o, po, fl, stPyro, stMass, stArea);
       solOut[i] = o;
       pyr[i] = po;
       flags[i] = fl ? 1 : FLAG_BURNT;
@@ -302,11 +329,15 @@ __device__ __forceinline__ void solid_block(const Params *__restrict__ P, const 
     double b = block_sum<NT>((double)stMass, sh);
     double c = block_sum<NT>((double)stArea, sh);
     if (threadIdx.x == 0) {
-      part[blockIdx.x * 3 + 0] = a;
-      part[blockIdx.x * 3 + 1] = b;
-      part[blockIdx.x * 3 + 2] = c;
+      part[p * 3 + 0] = a;
+      part[p * 3 + 1] = b;
+      part[p * 3 + 2] = c;
     }
   }
+}
+
+__device__ __forceinline__ void solid_kinds(const Params *__restrict__ P, SolidLds &L) {
+  if (threadIdx.x < 8) L.kinds[threadIdx.x] = (uint32_t)(P->mats[threadIdx.x].a[3] + 0.5f);
 }
 
 template <bool STATS>
@@ -314,40 +345,77 @@ __global__ __launch_bounds__(NT) void k_solid(const Params *__restrict__ P, Geo 
                                                float4 *__restrict__ solOut, float4 *__restrict__ pyr,
                                                uint8_t *__restrict__ flags, const float4 *__restrict__ s0,
                                                double *__restrict__ part) {
-  solid_block<STATS>(P, g, solIn, solOut, pyr, flags, s0, part);
+  __shared__ SolidLds L;
+  solid_kinds(P, L);
+  const uint32_t c0 = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT, i = c0 + threadIdx.x;
+  solid_tile<STATS>(P, g, L, solIn, solOut, pyr, flags, s0, part, c0, blockIdx.x, i < g.n ? flags[i] : 0);
 }
 
-// The step's solid and curl stages in one launch (the same block and cell
-// mapping): curl reads only the velocity and writes only curl, which solid
-// neither reads nor writes, so each block computes its cells' vorticity and
-// then runs the solid pass; the dense, memory-bound curl fills the CUs that
-// wait on the few blocks with ray marches.
+// The step's solid and curl stages in one launch: curl reads only the velocity
+// and writes only curl, which solid neither reads nor writes.  The first ns
+// blocks take the solid tiles, tile j, j + ns, ... each, and the rest the
+// curl, so the few tiles with ray marches, which lie together in the grid,
+// start first, on different CUs and XCDs, and the dense, memory-bound curl
+// fills the CUs meanwhile.  Eight tiles' flags are loaded at once: nearly all
+// tiles are empty.  (One block for both stages of a tile left the ray marches
+// to the XCD whose part of the grid holds them, at the end of its part:
+// 160x240x160 88 us, 50 now; 160x320x160 79, 56; 320x480x320 720, 541.  512
+// or 2048 blocks, 16 tiles at once or fewer registers are slower.)
+constexpr int SOLID_BLOCKS = 1024, SOLID_BATCH = 8;
 template <bool STATS>
-__global__ __launch_bounds__(NT) void k_solid_curl(const Params *__restrict__ P, Geo g,
+__global__ __launch_bounds__(NT) void k_solid_curl(const Params *__restrict__ P, Geo g, int ns,
                                                     const float4 *__restrict__ solIn, float4 *__restrict__ solOut,
                                                     float4 *__restrict__ pyr, uint8_t *__restrict__ flags,
                                                     const float4 *__restrict__ s0, double *__restrict__ part,
                                                     const float *__restrict__ U, const float *__restrict__ V,
                                                     const float *__restrict__ W, float4 *__restrict__ curl,
                                                     float *__restrict__ cpart) {
-  const uint32_t i = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
-  float spd = 0.0f;
-  if (i < g.n) spd = curl_cell<STATS>(P, g, U, V, W, curl, i);
-  if (STATS) {
-    __shared__ float sh[NT / 64];
-    const float m = block_max<NT>(spd, sh);
-    if (threadIdx.x == 0) cpart[blockIdx.x] = m;
+  const int nt = (int)((g.n + NT - 1) / NT);
+  if ((int)blockIdx.x >= ns) {
+    const int blk = (int)blockIdx.x - ns;
+    const uint32_t i = (uint32_t)xcd_tile(blk, nt) * NT + threadIdx.x;
+    float spd = 0.0f;
+    if (i < g.n) spd = curl_cell<STATS>(P, g, U, V, W, curl, i);
+    if (STATS) {
+      __shared__ float sh[NT / 64];
+      const float m = block_max<NT>(spd, sh);
+      if (threadIdx.x == 0) cpart[blk] = m;
+    }
+    return;
   }
-  solid_block<STATS>(P, g, solIn, solOut, pyr, flags, s0, part);
+  __shared__ SolidLds L;
+  solid_kinds(P, L);
+  for (int t0 = (int)blockIdx.x; t0 < nt; t0 += SOLID_BATCH * ns) {
+    uint8_t f[SOLID_BATCH];
+    bool any = STATS;
+#pragma unroll
+    for (int u = 0; u < SOLID_BATCH; u++) {
+      const uint32_t t = (uint32_t)t0 + (uint32_t)(ns * u), i = t * NT + threadIdx.x;
+      f[u] = (int)t < nt && i < g.n ? flags[i] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < SOLID_BATCH; u++) any |= f[u] != 0;
+    if (!__syncthreads_or(any)) continue;
+#pragma unroll 1
+    for (int u = 0; u < SOLID_BATCH; u++) {
+      const int t = t0 + ns * u;
+      if (t >= nt) break;
+      solid_tile<STATS>(P, g, L, solIn, solOut, pyr, flags, s0, part, (uint32_t)t * NT, (uint32_t)xcd_block(t, nt), f[0]);
+#pragma unroll
+      for (int v = 0; v + 1 < SOLID_BATCH; v++) f[v] = f[v + 1];  // f[0]: the next tile's
+    }
+  }
 }
 void launch_solid_curl(const Fields &f, StatParts *st, hipStream_t s) {
-  const int nb = nblocks(f.g.n);
+  const int nt = nblocks(f.g.n);
+  // a multiple of 8 leaves the curl blocks on the XCDs that xcd_tile means
+  const int ns = nt < SOLID_BLOCKS ? (nt + 7) / 8 * 8 : SOLID_BLOCKS;
   if (st)
-    k_solid_curl<true><<<nb, NT, 0, s>>>(f.P, f.g, f.sol_in, f.sol_out, f.pyr, f.flags, f.s0, st->solid, f.va[0],
-                                         f.va[1], f.va[2], f.curl, st->curl);
+    k_solid_curl<true><<<ns + nt, NT, 0, s>>>(f.P, f.g, ns, f.sol_in, f.sol_out, f.pyr, f.flags, f.s0, st->solid,
+                                              f.va[0], f.va[1], f.va[2], f.curl, st->curl);
   else
-    k_solid_curl<false><<<nb, NT, 0, s>>>(f.P, f.g, f.sol_in, f.sol_out, f.pyr, f.flags, f.s0, nullptr, f.va[0],
-                                          f.va[1], f.va[2], f.curl, nullptr);
+    k_solid_curl<false><<<ns + nt, NT, 0, s>>>(f.P, f.g, ns, f.sol_in, f.sol_out, f.pyr, f.flags, f.s0, nullptr,
+                                               f.va[0], f.va[1], f.va[2], f.curl, nullptr);
 }
 
 void launch_solid(const Fields &f, StatParts *st, hipStream_t s) {

@@ -285,12 +285,6 @@ __device__ __forceinline__ double pair_sum(double v0, double v1, double *sh) {
     for (int q = 0; q < 4; q++) r += sh[4 * threadIdx.x + q];
   return r;
 }
-// The block of a launch of nb blocks that xcd_tile gives tile t.
-__device__ __forceinline__ int xcd_block(int t, int nb) {
-  const int q = nb >> 3;
-  return t >= (q << 3) ? t : (t % q) * 8 + t / q;
-}
-
 // q = A p with partials of p.q and p.r
 __global__ __launch_bounds__(NT) void k_apply_dots(Op64 o, const uint8_t *__restrict__ nm, const uint8_t *__restrict__ nc,
                                                     const double *__restrict__ p, const double *__restrict__ r,
