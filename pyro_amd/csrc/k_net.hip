@@ -259,10 +259,11 @@ __device__ __forceinline__ void conv_chunk(const bf16 *__restrict__ wp, const bf
   }
 }
 
-template <int CA, int CB, int COUT, bool RELU>
+// MS: blocks (blockIdx.y) that share a tile's output channels.
+template <int CA, int CB, int COUT, bool RELU, int MS>
 __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
-  constexpr int MB = COUT / 16;
-  constexpr int CCA = MB == 1 ? 16 : 32;  // conv_a_chunk
+  constexpr int MB = COUT / 16 / MS;
+  constexpr int CCA = COUT == 16 ? 16 : 32;  // conv_a_chunk
   constexpr int NCA = CA / CCA;
   constexpr int NCB = CB == 16 ? 1 : CB / 32;
   constexpr int CCB = CB == 16 ? 16 : 32;
@@ -279,7 +280,8 @@ __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
   for (int m = 0; m < MB; m++)
 #pragma unroll
     for (int nb = 0; nb < 4; nb++) acc[m][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const bf16 *wp = p.wp;
+  const int c0 = MS > 1 ? (int)blockIdx.y * MB * 16 : 0;  // the block's first output channel
+  const bf16 *wp = p.wp + c0 * 32;
 #pragma unroll 1
   for (int q = 0; q < NCA; q++) {
     __syncthreads();
@@ -305,7 +307,7 @@ __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
     const size_t v = (size_t)gx + (size_t)p.nx * ((size_t)gy + (size_t)p.ny * (size_t)gz);
 #pragma unroll
     for (int m = 0; m < MB; m++) {
-      const int co = m * 16 + 4 * j;
+      const int co = c0 + m * 16 + 4 * j;
       bf16x4 o;
 #pragma unroll
       for (int i = 0; i < 4; i++) {
@@ -474,10 +476,21 @@ bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *
                                  ((g.nz + CV_TZ - 1) / CV_TZ));
   const unsigned nb16 = (unsigned)(((g.nx + CV_TX - 1) / CV_TX) * ((g.ny + CS_Y - 1) / CS_Y) *
                                    ((g.nz + CS_Z - 1) / CS_Z));
-#define PYRO_CONV(CA_, CB_, CO_, R_)                                          \
-  if (ca == CA_ && cb == CB_ && cout == CO_ && relu == R_) {                  \
-    k_conv3<CA_, CB_, CO_, R_><<<nb, 256, 0, s>>>(p);                         \
-    return true;                                                              \
+  // A layer on a coarse grid has fewer tiles than the chip has compute units.
+  // Its output channels are then split over MS blocks a tile, as far as all
+  // blocks are resident at once (three to a compute unit, 768).  In us, one
+  // block a tile and split: 64 -> 64 at 6 tiles 23 and 12, at 100 32 and 17, at
+  // 192 44 and 23; 96 -> 32 at 15 tiles 23 and 20, at 120 34 and 23, at 384 37
+  // and 34, at 512 38 and 53; 32 -> 96 at 120 tiles 24 and 14, at 256 31 and 22
+  // (two blocks; 25 with six), at 600 41 and 45.
+  constexpr unsigned RESIDENT = 768;
+#define PYRO_CONV(CA_, CB_, CO_, R_)                                                                        \
+  if (ca == CA_ && cb == CB_ && cout == CO_ && relu == R_) {                                                \
+    constexpr int S1 = CO_ / 16, S2 = CO_ == 64 || CO_ == 96 ? 2 : 1;                                       \
+    if (nb * S1 <= RESIDENT) k_conv3<CA_, CB_, CO_, R_, S1><<<dim3(nb, S1), 256, 0, s>>>(p);                \
+    else if (nb * S2 <= RESIDENT) k_conv3<CA_, CB_, CO_, R_, S2><<<dim3(nb, S2), 256, 0, s>>>(p);           \
+    else k_conv3<CA_, CB_, CO_, R_, 1><<<nb, 256, 0, s>>>(p);                                               \
+    return true;                                                                                            \
   }
 #define PYRO_CONV16(CA_, R_)                                      \
   if (ca == CA_ && cb == 16 && cout == 16 && relu == R_) {        \
