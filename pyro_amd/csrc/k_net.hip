@@ -195,9 +195,7 @@ __device__ __forceinline__ void conv_stage(const ConvArgs &p, int c0, int x0, in
 }
 
 // MFMAs of one staged chunk: NG K32 groups (27 taps of 32 channels, or 14
-// tap pairs of 16 channels).  With one 16-row output block (MB = 1) every
-// weight fragment of the chunk is loaded into registers up front and the
-// group loop is fully unrolled, so the loop body is LDS reads and MFMAs only.
+// tap pairs of 16 channels).
 template <int CC, int MB, int COUT>
 __device__ __forceinline__ void conv_chunk(const bf16 *__restrict__ wp, const bf16 *lds, f32x4 (&acc)[MB][4], int w,
                                            int j, int col) {
@@ -225,8 +223,9 @@ __device__ __forceinline__ void conv_chunk(const bf16 *__restrict__ wp, const bf
   };
   if constexpr (MB == 1) {
     // batches of BS groups, the next batch's weight fragments loaded while
-    // the current batch computes
-    constexpr int BS = CC == 32 ? 9 : 7, NBATCH = NG / BS;
+    // the current batch computes.  Short batches: with nine and seven the
+    // forward pass at 24x40x24 took 87 us, now 78 (64x64x64 109, 102.5).
+    constexpr int BS = CC == 32 ? 3 : 2, NBATCH = NG / BS;
     static_assert(NBATCH * BS == NG, "group batches");
     bf16x8 Acur[BS][1], Anext[BS][1];
 #pragma unroll
