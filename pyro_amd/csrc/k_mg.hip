@@ -95,6 +95,15 @@ __device__ __forceinline__ float div_count(float x, float c, float r) {
   return q;
 }
 
+// The same without the division: a subnormal quotient is noted in `redo`.
+__device__ __forceinline__ float quot_count(float x, float c, float r, bool &redo) {
+  const float q0 = x * r;
+  const float e = __builtin_fmaf(-q0, c, x);
+  const float q = __builtin_fmaf(e, r, q0);
+  redo |= __builtin_amdgcn_classf(q, 0x90);  // -subnormal | +subnormal
+  return q;
+}
+
 // Residual + average over fluid children, coarse phi = 0 (mg.wgsl:67-81).
 // The coarse flags (mg.wgsl:82) are produced once per step by the setup pass.
 // A block takes 16 x 4 x 4 coarse cells (one per thread); the fine φ and
@@ -1543,7 +1552,15 @@ __global__ __launch_bounds__(EX ? CZ_EX_NT : CO_NT) void k_mg_coarse_z(LvArgs a,
       } else {
         // Long columns: many waves share each SIMD and hide the latency;
         // registers are the limit (no per-pass arrays).  The next slot's
-        // four reads are issued before this slot's arithmetic.
+        // four reads are issued before this slot's arithmetic.  A quotient
+        // that came out subnormal is only noted: LDS still holds the pass's
+        // old values, from which the rare lane recomputes its slots with the
+        // IEEE division.  The scheduling barriers keep the reads one slot
+        // ahead: left to itself the compiler gathers all of a pass's reads,
+        // and the waves then wait on the LDS together.  20x40x20: 165 us with
+        // a branch a slot, 183 without the barriers, 155 now; 18x28x18 145,
+        // 165 and 121; the counts kept as floats (21 more registers) 157.
+        bool redo = false;
         float nb[4] = {sxp[c * CZ_PLANE], sxm[c * CZ_PLANE], syp[c * CZ_PLANE], sym[c * CZ_PLANE]};
 #pragma unroll
         for (int j = c; j < ZJ; j += 2) {
@@ -1554,6 +1571,7 @@ __global__ __launch_bounds__(EX ? CZ_EX_NT : CO_NT) void k_mg_coarse_z(LvArgs a,
             nx[2] = syp[(j + 2) * CZ_PLANE];
             nx[3] = sym[(j + 2) * CZ_PLANE];
           }
+          __builtin_amdgcn_sched_barrier(0);
           const float cn = (float)((cp[j >> 2] >> (8 * (j & 3))) & 0xffu);
           float sum = nb[0];
           sum += nb[1];
@@ -1561,9 +1579,23 @@ __global__ __launch_bounds__(EX ? CZ_EX_NT : CO_NT) void k_mg_coarse_z(LvArgs a,
           sum += nb[3];
           sum += ph[j + 2];
           sum += ph[j];
-          ph[j + 1] = mixf_(ph[j + 1], div_count(sum - hb[j], cn, rc[j]), omega);
+          ph[j + 1] = mixf_(ph[j + 1], quot_count(sum - hb[j], cn, rc[j], redo), omega);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
           for (int k = 0; k < 4; k++) nb[k] = nx[k];
+        }
+        if (redo) {
+#pragma unroll
+          for (int j = c; j < ZJ; j += 2) {
+            const float cn = (float)((cp[j >> 2] >> (8 * (j & 3))) & 0xffu);
+            float sum = sxp[j * CZ_PLANE];
+            sum += sxm[j * CZ_PLANE];
+            sum += syp[j * CZ_PLANE];
+            sum += sym[j * CZ_PLANE];
+            sum += ph[j + 2];
+            sum += ph[j];
+            ph[j + 1] = mixf_(sp[B + j * CZ_PLANE], div_count(sum - hb[j], cn, rc[j]), omega);
+          }
         }
       }
 #pragma unroll
