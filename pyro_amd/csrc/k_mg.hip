@@ -372,13 +372,31 @@ void launch_mg_prolong(const MgLevel &C, const MgLevel &F, hipStream_t s) {
 //   or the top.  cnt of mg.wgsl:25-33 = fluid + wdir * outside; with
 //   wdir = 1 it is the same small integer, exactly.
 
-__global__ __launch_bounds__(NT) void k_mg_counts(LvArgs a, FastDiv d0, const uint8_t *__restrict__ f,
-                                                   uint8_t *__restrict__ nc, uint8_t *__restrict__ nm) {
-  uint32_t i = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
-  if (i >= a.n) return;
-  uint32_t r = fdiv(i, d0);
+// All levels go in one launch, and the coarse flags of three levels in another:
+// a launch a level and kind took 4 to 5 us each, seven of them in every step.
+// The levels' blocks follow one another; the table is indexed where it lies,
+// in the kernel arguments (a copy would be indexed in scratch memory).
+constexpr int SU_MAX = 12;
+typedef const __attribute__((address_space(1))) uint8_t *gcu8;
+typedef __attribute__((address_space(1))) uint8_t *gu8;
+struct SetupLevel {
+  int d0, d1, d2;
+  uint32_t n, block0;  // cells, first block
+  FastDiv q0, q1;      // d0, d1
+  gu8 f, nc, nm;
+};
+struct SetupArgs {
+  int nl, first;  // levels, first level written (coarse flags)
+  SetupLevel l[SU_MAX];
+};
+
+// The codes of a cell, or of four cells along x at once.
+__device__ __forceinline__ void counts_cell(const SetupLevel &a, uint32_t i) {
+  gcu8 f = a.f;
+  const gu8 nc = a.nc, nm = a.nm;
+  uint32_t r = fdiv(i, a.q0);
   int x = (int)(i - r * (uint32_t)a.d0);
-  uint32_t zq = fdiv(r, a.dny);
+  uint32_t zq = fdiv(r, a.q1);
   int y = (int)(r - zq * (uint32_t)a.d1), z = (int)zq;
   const uint32_t sy = (uint32_t)a.d0, sz = (uint32_t)a.d0 * (uint32_t)a.d1;
   const bool hxp = x + 1 < a.d0, hxm = x > 0, hyp = y + 1 < a.d1, hym = y > 0, hzp = z + 1 < a.d2, hzm = z > 0;
@@ -406,19 +424,19 @@ __global__ __launch_bounds__(NT) void k_mg_counts(LvArgs a, FastDiv d0, const ui
 // 4): a thread reads the flag words of its cells and of their y and z
 // neighbours and the two bytes beside them in x, and writes one code word.
 __device__ __forceinline__ uint32_t byte_of(uint32_t w, int j) { return (w >> (8 * j)) & 0xffu; }
-__global__ __launch_bounds__(NT) void k_mg_counts4(LvArgs a, FastDiv d0, const uint8_t *__restrict__ f,
-                                                    uint8_t *__restrict__ nc, uint8_t *__restrict__ nm) {
-  const uint32_t w = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;  // word index
-  if (w >= a.n / 4u) return;
+__device__ __forceinline__ void counts_cells4(const SetupLevel &a, uint32_t w) {  // w: word index
+  typedef const __attribute__((address_space(1))) uint32_t *gcu32;
+  typedef __attribute__((address_space(1))) uint32_t *gu32;
+  gcu8 f = a.f;
   const uint32_t i = 4u * w;
-  uint32_t r = fdiv(i, d0);
+  uint32_t r = fdiv(i, a.q0);
   const int x0 = (int)(i - r * (uint32_t)a.d0);
-  uint32_t zq = fdiv(r, a.dny);
+  uint32_t zq = fdiv(r, a.q1);
   const int y = (int)(r - zq * (uint32_t)a.d1), z = (int)zq;
   const uint32_t sy = (uint32_t)a.d0, sz = (uint32_t)a.d0 * (uint32_t)a.d1;
   const bool hyp = y + 1 < a.d1, hym = y > 0, hzp = z + 1 < a.d2, hzm = z > 0;
   const bool hx0 = x0 > 0, hx3 = x0 + 4 < a.d0;
-  const uint32_t *f4 = reinterpret_cast<const uint32_t *>(f);
+  gcu32 f4 = (gcu32)f;
   // a neighbour outside the level reads the cell's own word or byte and is not used
   const uint32_t C = f4[w];
   const uint32_t YP = f4[hyp ? w + sy / 4u : w], YM = f4[hym ? w - sy / 4u : w];
@@ -446,43 +464,87 @@ __global__ __launch_bounds__(NT) void k_mg_counts4(LvArgs a, FastDiv d0, const u
     codes |= code << (8 * j);
     masks |= m << (8 * j);
   }
-  reinterpret_cast<uint32_t *>(nc)[w] = codes;
-  if (nm) reinterpret_cast<uint32_t *>(nm)[w] = masks;
+  ((gu32)a.nc)[w] = codes;
+  if (a.nm) ((gu32)a.nm)[w] = masks;
 }
 
-// Coarse cell is solid iff every child inside the fine box is solid (mg.wgsl:74-82).
-__global__ __launch_bounds__(NT) void k_mg_coarse_flags(LvArgs F, const uint8_t *__restrict__ ff, int c0, int c1,
-                                                         int c2, FastDiv dc0, FastDiv dc1, uint8_t *__restrict__ fc) {
-  uint32_t i = (uint32_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
-  if (i >= (uint32_t)c0 * (uint32_t)c1 * (uint32_t)c2) return;
-  uint32_t r = fdiv(i, dc0);
-  int x = (int)(i - r * (uint32_t)c0);
-  uint32_t zq = fdiv(r, dc1);
-  int y = (int)(r - zq * (uint32_t)c1), z = (int)zq;
-  int nfl = 0;
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    int a = 2 * x + (k & 1), bb = 2 * y + ((k >> 1) & 1), c = 2 * z + ((k >> 2) & 1);
-    if (a >= F.d0 || bb >= F.d1 || c >= F.d2) continue;
-    nfl += ff[(uint32_t)a + (uint32_t)F.d0 * ((uint32_t)bb + (uint32_t)F.d1 * (uint32_t)c)] != 1;
+__global__ __launch_bounds__(NT) void k_mg_counts(SetupArgs) {
+  const SetupArgs &a = *(const SetupArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t blk = (uint32_t)xcd_tile(blockIdx.x, gridDim.x);
+  int l = 0;
+  while (l + 1 < a.nl && blk >= a.l[l + 1].block0) l++;
+  const SetupLevel &L = a.l[l];
+  const uint32_t i = (blk - L.block0) * NT + threadIdx.x;
+  if (L.d0 % 4 == 0) {
+    if (i < L.n / 4u) counts_cells4(L, i);
+  } else if (i < L.n) {
+    counts_cell(L, i);
   }
-  fc[i] = nfl > 0 ? 0 : 1;
+}
+
+// Coarse cell is solid iff every child inside the fine box is solid
+// (mg.wgsl:74-82), so iff every cell of a finer level is that lies in it.  A
+// thread takes a cell of the level K above the one read, a plane of its 8^K
+// cells at a time (one beyond the box is read as the last inside it), and
+// stops at the first plane that is not solid: nearly always the first.
+template <int K>
+__device__ __forceinline__ uint8_t all_solid(const SetupLevel &F, int x, int y, int z) {
+  constexpr int S = 1 << K;
+  for (int zz = 0; zz < S; zz++) {
+    const int c = (z << K) + zz;
+    if (c >= F.d2) break;
+    bool solid = true;
+#pragma unroll
+    for (int k = 0; k < S * S; k++) {
+      const int a = min((x << K) + k % S, F.d0 - 1), b = min((y << K) + k / S, F.d1 - 1);
+      solid &= F.f[(uint32_t)a + (uint32_t)F.d0 * ((uint32_t)b + (uint32_t)F.d1 * (uint32_t)c)] == 1;
+    }
+    if (!solid) return 0;
+  }
+  return 1;
+}
+__global__ __launch_bounds__(NT) void k_mg_coarse_flags(SetupArgs) {
+  const SetupArgs &a = *(const SetupArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t blk = blockIdx.x;
+  int l = a.first;
+  while (l + 1 < a.nl && blk >= a.l[l + 1].block0) l++;
+  const SetupLevel &C = a.l[l], &F = a.l[a.first - 1];
+  const uint32_t i = (blk - C.block0) * NT + threadIdx.x;
+  if (i >= C.n) return;
+  const uint32_t r = fdiv(i, C.q0), zq = fdiv(r, C.q1);
+  const int x = (int)(i - r * (uint32_t)C.d0), y = (int)(r - zq * (uint32_t)C.d1), z = (int)zq;
+  const int k = l - a.first + 1;
+  C.f[i] = k == 1 ? all_solid<1>(F, x, y, z) : k == 2 ? all_solid<2>(F, x, y, z) : all_solid<3>(F, x, y, z);
 }
 
 void launch_mg_setup(const MgLevel *L, int nl, hipStream_t s) {
+  SetupArgs a = {};
+  a.nl = nl;
   for (int l = 0; l < nl; l++) {
-    if (l > 0) {
-      const MgLevel &F = L[l - 1], &C = L[l];
-      k_mg_coarse_flags<<<nblocks(C.n), NT, 0, s>>>(lv_args(F), F.f, C.d[0], C.d[1], C.d[2],
-                                                   make_fastdiv((uint32_t)C.d[0]), make_fastdiv((uint32_t)C.d[1]), C.f);
-    }
-    if (L[l].d[0] % 4 == 0)
-      k_mg_counts4<<<nblocks(L[l].n / 4u), NT, 0, s>>>(lv_args(L[l]), make_fastdiv((uint32_t)L[l].d[0]), L[l].f,
-                                                        L[l].nc, L[l].nm);
-    else
-      k_mg_counts<<<nblocks(L[l].n), NT, 0, s>>>(lv_args(L[l]), make_fastdiv((uint32_t)L[l].d[0]), L[l].f, L[l].nc,
-                                                 L[l].nm);
+    SetupLevel &S = a.l[l];
+    S.d0 = L[l].d[0]; S.d1 = L[l].d[1]; S.d2 = L[l].d[2];
+    S.n = L[l].n;
+    S.q0 = make_fastdiv((uint32_t)L[l].d[0]);
+    S.q1 = make_fastdiv((uint32_t)L[l].d[1]);
+    S.f = (gu8)L[l].f; S.nc = (gu8)L[l].nc; S.nm = (gu8)L[l].nm;
   }
+  SetupArgs c = a;
+  for (int f = 1; f < nl; f += 3) {
+    uint32_t blocks = 0;
+    c.first = f;
+    c.nl = f + 3 < nl ? f + 3 : nl;
+    for (int l = f; l < c.nl; l++) {
+      c.l[l].block0 = blocks;
+      blocks += (uint32_t)nblocks(L[l].n);
+    }
+    k_mg_coarse_flags<<<blocks, NT, 0, s>>>(c);
+  }
+  uint32_t blocks = 0;
+  for (int l = 0; l < nl; l++) {
+    a.l[l].block0 = blocks;
+    blocks += (uint32_t)nblocks(L[l].d[0] % 4 == 0 ? L[l].n / 4u : L[l].n);
+  }
+  k_mg_counts<<<blocks, NT, 0, s>>>(a);
 }
 
 // ---------------------------------------------------------------- sweep
