@@ -104,6 +104,14 @@ __device__ __forceinline__ float quot_count(float x, float c, float r, bool &red
   return q;
 }
 
+// The four elements from `over` on (0 beyond the fourth).
+__device__ __forceinline__ float4 shift4(float4 v, int over) {
+  if (over == 1) return make_float4(v.y, v.z, v.w, 0.0f);
+  if (over == 2) return make_float4(v.z, v.w, 0.0f, 0.0f);
+  if (over == 3) return make_float4(v.w, 0.0f, 0.0f, 0.0f);
+  return v;
+}
+
 // Residual + average over fluid children, coarse phi = 0 (mg.wgsl:67-81).
 // The coarse flags (mg.wgsl:82) are produced once per step by the setup pass.
 // A block takes 16 x 4 x 4 coarse cells (one per thread); the fine φ and
@@ -118,14 +126,19 @@ constexpr int RS_FN = RS_FX * RS_FY * RS_FZ;
 // range is widened to 16-byte alignment, [2 x0 - 4, 2 x0 + 36), and staged
 // as whole float4 / uchar4 groups: thread t < 250 loads group t % 10 of the
 // rows t / 10 + 25 it, it = 0..3 (a group lies entirely inside or outside
-// the level; outside reads 0 and codes 0x40).
+// the level; outside reads 0 and codes 0x40).  ODD (any other x-size from four
+// up): the same with the last group of a row loaded from where it ends with
+// the row and shifted, and codes loaded as bytes; one element at a time the
+// launch took 8.4 us on the levels of a 97x61x118 grid, 5.2 now.
 constexpr int RS_VX = 2 * RS_TX + 8, RS_VQ = RS_VX / 4, RS_VN = RS_VX * RS_FY * RS_FZ;
 static_assert(RS_VQ * 25 == 250 && RS_FY * RS_FZ == 100, "restriction staging map");
-template <bool VEC>
+enum { ROWS_ANY = 0, ROWS_ODD = 1, ROWS_VEC = 2 };
+template <int R>
 __global__ __launch_bounds__(NT) void k_mg_restrict(LvArgs F, int ntx, int nty, const float *__restrict__ pf,
                                                      const float *__restrict__ bf, const uint8_t *__restrict__ ncf,
                                                      int c0, int c1, int c2, float *__restrict__ bc,
                                                      float *__restrict__ pc) {
+  constexpr bool VEC = R != ROWS_ANY;
   constexpr int FX = VEC ? RS_VX : RS_FX;
   __shared__ __align__(16) float sp[VEC ? RS_VN : RS_FN];
   __shared__ __align__(16) uint8_t sc[VEC ? RS_VN : RS_FN];
@@ -159,14 +172,25 @@ __global__ __launch_bounds__(NT) void k_mg_restrict(LvArgs F, int ntx, int nty, 
       const bool ok = t < 250 && (uint32_t)gx < (uint32_t)F.d0 && (uint32_t)gy < (uint32_t)F.d1 &&
                       (uint32_t)gz < (uint32_t)F.d2;
       const uint32_t g = (uint32_t)gx + (uint32_t)sy * (uint32_t)gy + (uint32_t)sz * (uint32_t)gz;
-      pv[it] = rb_ld4(rp, ok ? 4u * g : RB_OOB);
-      const uint32_t c = rb_ld32(rcd, ok ? g : RB_OOB);
-      cv[it] = ok ? c : 0x40404040u;
+      const int over = R == ROWS_ODD && gx + 4 > F.d0 ? gx + 4 - F.d0 : 0;  // elements past the row's end
+      pv[it] = rb_ld4(rp, ok ? 4u * (g - (uint32_t)over) : RB_OOB);
+      if (R == ROWS_VEC) {
+        const uint32_t c = rb_ld32(rcd, ok ? g : RB_OOB);
+        cv[it] = ok ? c : 0x40404040u;
+      } else {
+        cv[it] = 0u;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const bool okj = ok && gx + j < F.d0;
+          const uint32_t cj = __builtin_amdgcn_raw_buffer_load_b8(rcd.r, okj ? g + j : RB_OOB, 0, 0);
+          cv[it] |= (okj ? cj : (uint32_t)NC_NONE) << (8 * j);
+        }
+      }
     }
     if (t < 250) {
 #pragma unroll
       for (int it = 0; it < 4; it++) {
-        float4 v = pv[it];
+        float4 v = R == ROWS_ODD ? shift4(pv[it], gx + 4 - F.d0) : pv[it];
         const uint32_t c = cv[it];
         if (c & 0x80808080u) {  // solids read 0 in the neighbour sums
           if (c & 0x80u) v.x = 0.0f;
@@ -226,13 +250,14 @@ __global__ __launch_bounds__(NT) void k_mg_restrict(LvArgs F, int ntx, int nty, 
 void launch_mg_restrict(const MgLevel &Fl, const MgLevel &C, hipStream_t s) {
   LvArgs F = lv_args(Fl);
   const int ntx = (C.d[0] + RS_TX - 1) / RS_TX, nty = (C.d[1] + RS_TY - 1) / RS_TY, ntz = (C.d[2] + RS_TZ - 1) / RS_TZ;
-  const bool vec = (Fl.d[0] % 4) == 0 && (uint64_t)Fl.n * 4u < (1ull << 31);
-  if (vec)
-    k_mg_restrict<true><<<ntx * nty * ntz, NT, 0, s>>>(F, ntx, nty, Fl.phi, Fl.b, Fl.nc, C.d[0], C.d[1], C.d[2], C.b,
-                                                       C.phi);
-  else
-    k_mg_restrict<false><<<ntx * nty * ntz, NT, 0, s>>>(F, ntx, nty, Fl.phi, Fl.b, Fl.nc, C.d[0], C.d[1], C.d[2],
-                                                        C.b, C.phi);
+  const bool buf = (uint64_t)Fl.n * 4u < (1ull << 31);
+#define PYRO_RESTRICT(R_)                                                                                       \
+  k_mg_restrict<R_><<<ntx * nty * ntz, NT, 0, s>>>(F, ntx, nty, Fl.phi, Fl.b, Fl.nc, C.d[0], C.d[1], C.d[2], C.b, \
+                                                   C.phi)
+  if (buf && Fl.d[0] % 4 == 0) PYRO_RESTRICT(ROWS_VEC);
+  else if (buf && Fl.d[0] > 4) PYRO_RESTRICT(ROWS_ODD);
+  else PYRO_RESTRICT(ROWS_ANY);
+#undef PYRO_RESTRICT
 }
 
 // Masked, renormalised trilinear correction (mg.wgsl:97-120).  A block takes
@@ -1172,13 +1197,6 @@ __device__ __forceinline__ void s2_pass(S2Lds &L, float omega, float wdir, float
   }
 }
 
-// The four elements from `over` on (0 beyond the fourth).
-__device__ __forceinline__ float4 s2_shift(float4 v, int over) {
-  if (over == 1) return make_float4(v.y, v.z, v.w, 0.0f);
-  if (over == 2) return make_float4(v.z, v.w, 0.0f, 0.0f);
-  if (over == 3) return make_float4(v.w, 0.0f, 0.0f, 0.0f);
-  return v;
-}
 // The coarse level that a fused prolongation (PRO) reads: 14 x 10 x 10 cells
 // around the footprint, indices clamped to the level as in k_mg_prolong.
 constexpr int S2_CX = S2_K + 2, S2_CY = S2_Y / 2 + 2, S2_CZ = S2_Z / 2 + 2, S2_CN = S2_CX * S2_CY * S2_CZ;
@@ -1316,8 +1334,8 @@ __global__ __launch_bounds__(S2_NT) void k_mg_sweep2(LvArgs a, int ntx, int nty,
     const uint32_t c = cv[i];
     if (!ALN) {
       const int over = x0 + 4 * q + 4 - a.d0;
-      v = s2_shift(v, over);
-      w = s2_shift(w, over);
+      v = shift4(v, over);
+      w = shift4(w, over);
     }
     if constexpr (PRO) {
       const int gx = x0 + 4 * q, gy = y0 + ly, gz = z0 + lz;
