@@ -1404,6 +1404,12 @@ __global__ __launch_bounds__(S2_NT) void k_mg_sweep2(LvArgs a, int ntx, int nty,
 // 4101 now; 129^3 (2.1 M) 9721 without, 9325 with; 193x121x235 (5.5 M) 17.45
 // ms, 17.38; 255^3 30.8, 31.9.
 constexpr uint32_t S2_MAX = 900000u, S2_MAX_ODD = 4000000u;
+// The prolongation joins them up to here: every cell of the rings is prolonged
+// too (3.75 times the tile).  A solve at 97x61x118 (its 698 k cells) 3.93 ms
+// with it in the launch, 3.78 without; 129^3 9.07 and 8.44; 96^3 2.84 and
+// 2.77; with a line of 50 k instead, four V-cycles at 80x160x80 (128 k) 465 us
+// against 458.
+constexpr uint32_t S2_PROLONG_MAX = 500000u;
 static bool sweep2_fits(const MgLevel &L) { return L.d[0] >= 4 && L.n <= (L.d[0] % 4 ? S2_MAX_ODD : S2_MAX); }
 // C: the level whose correction is added first, or null
 static void launch_mg_sweep2(const MgLevel &L, const MgLevel *C, const float *pin, float *pout, float omega,
@@ -2364,7 +2370,7 @@ void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, 
   while (t > 0 && tail_fits(lv, t - 1, nl)) t--;
   if (from_zero && t == 0) launch_zero32(lv[0].n, lv[0].phi, s);  // the tail reads phi
   // smoothing: two sweeps phi -> tmp -> phi, or both in one launch, phi ->
-  // tmp before the coarser level and tmp -> phi, with the prolongation, after it
+  // tmp before the coarser level and tmp -> phi after it
   for (int l = 0; l < t; l++) {
     MgLevel L = lv[l];
     const float *pin = (l > 0 || from_zero) ? nullptr : L.phi;  // a restricted level starts from 0
@@ -2382,7 +2388,13 @@ void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, 
   for (int l = t - 1; l >= 0; l--) {
     MgLevel L = lv[l];
     if (sweep2_fits(L)) {
-      launch_mg_sweep2(L, &lv[l + 1], L.tmp, L.phi, 1.0f, s);
+      const bool fuse = L.n <= S2_PROLONG_MAX;
+      if (!fuse) {
+        MgLevel T = L;
+        T.phi = T.tmp;
+        launch_mg_prolong(lv[l + 1], T, s);
+      }
+      launch_mg_sweep2(L, fuse ? &lv[l + 1] : nullptr, L.tmp, L.phi, 1.0f, s);
     } else {
       launch_mg_prolong(lv[l + 1], L, s);
       launch_mg_sweep(L, L.phi, L.tmp, 1.0f, s, l == 0);
