@@ -2364,25 +2364,30 @@ void launch_mg_resid(const MgLevel &L, StatParts *st, hipStream_t s) {
 }
 
 // ---------------------------------------------------------------- V-cycle
-void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero) {
+void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero, VPart part) {
   // the levels from t on run in one launch where they fit
   int t = nl - 1;
   while (t > 0 && tail_fits(lv, t - 1, nl)) t--;
-  if (from_zero && t == 0) launch_zero32(lv[0].n, lv[0].phi, s);  // the tail reads phi
+  if (from_zero && t == 0 && part != VPart::Rest) launch_zero32(lv[0].n, lv[0].phi, s);  // the tail reads phi
   // smoothing: two sweeps phi -> tmp -> phi, or both in one launch, phi ->
   // tmp before the coarser level and tmp -> phi after it
   for (int l = 0; l < t; l++) {
     MgLevel L = lv[l];
     const float *pin = (l > 0 || from_zero) ? nullptr : L.phi;  // a restricted level starts from 0
-    if (sweep2_fits(L)) {
-      launch_mg_sweep2(L, nullptr, pin, L.tmp, 1.0f, s);
-      L.phi = L.tmp;
-    } else {
-      launch_mg_sweep(L, pin, L.tmp, 1.0f, s, l == 0);
-      launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, l == 0);
+    const bool two = sweep2_fits(L);
+    if (l > 0 || part != VPart::Rest) {
+      if (two) {
+        launch_mg_sweep2(L, nullptr, pin, L.tmp, 1.0f, s);
+      } else {
+        launch_mg_sweep(L, pin, L.tmp, 1.0f, s, l == 0);
+        launch_mg_sweep(L, L.tmp, L.phi, 1.0f, s, l == 0);
+      }
     }
+    if (part == VPart::Head) return;
+    if (two) L.phi = L.tmp;
     launch_mg_restrict(L, lv[l + 1], s);
   }
+  if (part == VPart::Head) return;
   if (t < nl - 1) launch_mg_tail(lv, t, nl, coarse_iters, 1.6f, s);
   else launch_mg_coarse(lv[t], coarse_iters, 1.6f, s);
   for (int l = t - 1; l >= 0; l--) {

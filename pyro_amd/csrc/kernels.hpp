@@ -93,8 +93,11 @@ int mg_resid_blocks(const MgLevel &L);
 void launch_copy(const float4 *src, float4 *dst, uint32_t n4, hipStream_t s);
 // V-cycle of sim.rs:451-491 over an arbitrary hierarchy (2 pre- and 2
 // post-sweeps per level, `coarse_iters` SOR iterations at omega = 1.6).
-// from_zero: level 0's phi is taken as 0 and not read.
-void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero = false);
+// from_zero: level 0's phi is taken as 0 and not read.  Head: only what comes
+// before the first restriction; Rest: what follows it.
+enum class VPart { All, Head, Rest };
+void enqueue_vcycle(const MgLevel *lv, int nl, int coarse_iters, hipStream_t s, bool from_zero = false,
+                    VPart part = VPart::All);
 
 // FP64 solver kernels (k_solve.hip).
 void launch_resid64(const MgLevel &L, const double *x, const double *b, double *r, hipStream_t s);

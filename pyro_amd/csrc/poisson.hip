@@ -53,6 +53,8 @@ struct PyroPoisson {
   double *x = nullptr, *b = nullptr, *r = nullptr, *p = nullptr, *q = nullptr, *z = nullptr;
   double *w = nullptr, *t = nullptr;  // learned preconditioner: N(r) and the residual after it
   double *part = nullptr, *dots = nullptr;
+  double *rr_host = nullptr;       // pinned: r.r of the last iteration
+  hipEvent_t ev_rr = nullptr;      // its copy
   double *cgpart = nullptr, *dev = nullptr;  // fused-CG partial sums and the iteration's scalars
   double nfluid = 0.0;
   unsigned int *count = nullptr;  // device fluid-cell counter
@@ -93,6 +95,19 @@ int palloc(PyroPoisson *P, T **ptr, size_t count) {
 int sync(PyroPoisson *P) {
   PCHK(hipStreamSynchronize(P->stream));
   PCHK(hipGetLastError());
+  return 0;
+}
+// r.r of the iteration just enqueued, read by the host.  While it waits, the
+// card goes on with the next V-cycle's first sweeps (head), whose right-hand
+// side is there already; if the iteration was the last one they are not used.
+// Waiting with nothing enqueued left the card idle for some 20 us an iteration.
+int read_rr(PyroPoisson *P, bool head, double *rr) {
+  PCHK(hipMemcpyAsync(P->rr_host, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
+  PCHK(hipEventRecord(P->ev_rr, P->stream));
+  if (head) enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, VPart::Head);
+  PCHK(hipEventSynchronize(P->ev_rr));
+  PCHK(hipGetLastError());
+  *rr = *P->rr_host;
   return 0;
 }
 
@@ -323,6 +338,8 @@ int pyro_poisson_create(uint32_t nx, uint32_t ny, uint32_t nz, float h, const ui
     return bail(pfail(PYRO_E_HIP, "hipStreamCreate failed"));
   if (hipEventCreate(&P->ev_t0) != hipSuccess || hipEventCreate(&P->ev_t1) != hipSuccess ||
       hipEventCreateWithFlags(&P->ev_sim, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&P->ev_rr, hipEventDisableTiming) != hipSuccess ||
+      hipHostMalloc(reinterpret_cast<void **>(&P->rr_host), sizeof(double), hipHostMallocDefault) != hipSuccess ||
       hipEventCreateWithFlags(&P->ev_done, hipEventDisableTiming) != hipSuccess)
     return bail(pfail(PYRO_E_HIP, "hipEventCreate failed"));
   int d[3] = {(int)nx, (int)ny, (int)nz};
@@ -396,8 +413,9 @@ int pyro_poisson_destroy(PyroPoisson *P) {
   for (void *v : P->allocs) (void)hipFree(v);
   if (P->seal_idx) (void)hipFree(P->seal_idx);
   if (P->seal_off) (void)hipFree(P->seal_off);
-  for (hipEvent_t e : {P->ev_t0, P->ev_t1, P->ev_sim, P->ev_done})
+  for (hipEvent_t e : {P->ev_t0, P->ev_t1, P->ev_sim, P->ev_rr, P->ev_done})
     if (e) (void)hipEventDestroy(e);
+  if (P->rr_host) (void)hipHostFree(P->rr_host);
   if (P->stream) (void)hipStreamDestroy(P->stream);
   delete P;
   return 0;
@@ -487,14 +505,13 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     MgLevel &L0 = P->pc[0];
     if (!rc && !diverged && rel > tol) launch_to_f32(n, P->r, L0.b, P->stream);
     while (!rc && !diverged && rel > tol && it < max_iters) {
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, it ? VPart::Rest : VPart::All);
       launch_add_f32_to_f64(n, L0.phi, P->x, P->stream);
       cycles++;
       it++;
       launch_resid_rr(L0, P->x, P->b, L0.b, P->cgpart, P->dev, P->stream);
       double rr = 0.0;
-      PCHK(hipMemcpyAsync(&rr, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
-      rc = sync(P);
+      rc = read_rr(P, true, &rr);
       if (rc) break;
       rel = std::sqrt(rr / bb);
       if (watch(it)) break;
@@ -530,8 +547,9 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         fallbacks++;
         b32_ready = false;
       }
+      // b32_ready: the V-cycle's head is under way (read_rr)
       if (!b32_ready) launch_to_f32(n, P->r, L0.b, P->stream);
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, b32_ready ? VPart::Rest : VPart::All);
       if (with_dot) launch_dot_zq(n, L0.phi, P->q, P->cgpart, P->dev, P->stream);
       return 0;
     };
@@ -552,8 +570,7 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         pending = true;
         it++;
         double rr = 0.0;
-        PCHK(hipMemcpyAsync(&rr, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
-        rc = sync(P);
+        rc = read_rr(P, !use_net, &rr);
         if (rc) break;
         rel = std::sqrt(rr / bb);
         if (watch(it) || rel <= tol) break;
