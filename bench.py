@@ -90,9 +90,9 @@ COARSE_ITERS = 80
 COARSE_BYTES_PER_CELL_ITER = 24.0
 # The coarse solve's own bound is the VALU issue rate of its one CU (one
 # wave64 VALU instruction per cycle at 2.4 GHz): the counter run of
-# profiles/pool_2cm_kernel_counters.md reads 25,550 VALU instructions per wave
+# profiles/pool_2cm_kernel_counters.md reads 25,545 VALU instructions per wave
 # over 12 waves for the 20x40x20 level of the pool at 2 cm.
-COARSE_VALU_PER_WAVE, COARSE_WAVES, CU_CLOCK_HZ = 25550, 12, 2.4e9
+COARSE_VALU_PER_WAVE, COARSE_WAVES, CU_CLOCK_HZ = 25545, 12, 2.4e9
 # U-Net FLOPs per level-0 voxel: 2*27*cin*cout per conv at its level's
 # resolution (1/8 per halving) plus the 1x1x1 head: level 0 2*27*(2*16 + 16*16
 # + 48*16) + 2*16, level 1 2*27*(16*32 + 32*32 + 96*32)/8, level 2
@@ -258,9 +258,9 @@ def kernel_rooflines(scene, ck, args):
         if stg.startswith("adv_") or stg in ("solid", "curl"):
             continue  # in the fused launches above
         add(kname, f"stage {stg}, {bpc:g} B per cell", bpc * cells, stage_ms[stg], 1)
-    add("k_mg_sweep<true, true, true>", "level-0 red-black sweep, both colours, 24 B per cell", 24.0 * cells,
-        sweep, 16)
-    add("k_mg_restrict<true>" if nx % 4 == 0 else "k_mg_restrict<false>", "level 0 -> 1, 13.5 B per fine cell",
+    add("k_mg_sweep_z" if cells >= 12e6 else "k_mg_sweep<true, true, true>",
+        "level-0 red-black sweep, both colours, 24 B per cell", 24.0 * cells, sweep, 16)
+    add("k_mg_restrict<2>" if nx % 4 == 0 else "k_mg_restrict<1>", "level 0 -> 1, 13.5 B per fine cell",
         RESTRICT_BYTES_PER_FINE_CELL * cells, restrict0, 4)
     add("k_mg_prolong", "level 1 -> 0, 13 B per fine cell", PROLONG_BYTES_PER_FINE_CELL * cells, prolong0, 4)
     coarse_name = next((k for k in traffic if k.startswith("k_mg_coarse_z")), "k_mg_coarse_z")
