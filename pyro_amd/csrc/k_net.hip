@@ -821,29 +821,64 @@ size_t dw_part_elems(const G3 &g, const ConvSpec &c) {
 // XT of the concatenated conv input [up(a) (ca ch), b (cb ch)] (cb = 2: the
 // network input, rows 2..15 zero) in the first xgroups rows of blocks, GT in
 // the rest: a row takes eight channels, a thread two x of them, one 4-byte
-// store per channel.
+// store per channel.  The bias gradient's blocks come before them: a launch of
+// its own, one block a CU, waits on its loads most of the time (eight layers at
+// 80x160x80 182 + 72 us a step, together 198).
 struct TransArgs {
-  int nx, ny, nz, P, anx, any, ca, cb, cout, xgroups;
+  int nx, ny, nz, P, anx, any, ca, cb, xgroups;
   const bf16 *a, *b, *g;
   bf16 *xt, *gt;
   uint32_t x_items, g_items;  // per group of eight channels
   FastDiv dxp, dxy, dgp, dgy;  // (P + 16) / 2, ny + 2; P / 2, ny
+  uint32_t n;                  // voxels
+  float *bpart;
+  FastDiv dnb;  // blocks a row
 };
+// bias gradient: partials of db[c] = sum_v g[v][c], sixteen loads in flight
+template <int C>
+__device__ __forceinline__ void bias_grad(uint32_t n, const bf16 *__restrict__ g, float *__restrict__ part) {
+  constexpr uint32_t VL = 256 / C, STEP = BG_BLOCKS * VL, U = 16;
+  const uint32_t c = threadIdx.x % C, vl = threadIdx.x / C;
+  float s = 0.0f;
+  uint32_t v = blockIdx.x * VL + vl;
+  for (; (uint64_t)v + (U - 1) * STEP < n; v += U * STEP) {
+    bf16 x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) x[u] = g[(size_t)(v + u * STEP) * C + c];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) s += bf(x[u]);
+  }
+  for (; v < n; v += STEP) s += bf(g[(size_t)v * C + c]);
+  __shared__ float sh[256];
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (vl == 0) {
+    float t = 0.0f;
+    for (uint32_t k = 0; k < VL; k++) t += sh[k * C + c];
+    part[blockIdx.x * C + c] = t;
+  }
+}
 __device__ __forceinline__ uint32_t pair_of(bf16 lo, bf16 hi) {
   return (uint32_t)__builtin_bit_cast(uint16_t, lo) | ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
 }
+template <int COUT>
 __global__ __launch_bounds__(256) void k_to_t(TransArgs p) {
-  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+  if (blockIdx.x < BG_BLOCKS) {
+    bias_grad<COUT>(p.n, p.g, p.bpart);
+    return;
+  }
+  const uint32_t id = blockIdx.x - BG_BLOCKS, row = fdiv(id, p.dnb);
+  const uint32_t t = (id - row * p.dnb.d) * 256u + threadIdx.x;
   bf16x8 v[2];
 #pragma unroll
   for (int e = 0; e < 2; e++)
 #pragma unroll
     for (int i = 0; i < 8; i++) v[e][i] = tobf(0.0f);
-  if ((int)blockIdx.y < p.xgroups) {
+  if ((int)row < p.xgroups) {
     if (t >= p.x_items) return;
     const uint32_t hp = p.dxp.d, h2 = p.dxy.d, r = fdiv(t, p.dxp), zz = fdiv(r, p.dxy), yy = r - zz * h2;
     const int xp = 2 * (int)(t - r * hp);
-    const int y = (int)yy - 1, z = (int)zz - 1, c = 8 * (int)blockIdx.y;
+    const int y = (int)yy - 1, z = (int)zz - 1, c = 8 * (int)row;
     if (y >= 0 && y < p.ny && z >= 0 && z < p.nz) {
 #pragma unroll
       for (int e = 0; e < 2; e++) {
@@ -872,12 +907,12 @@ __global__ __launch_bounds__(256) void k_to_t(TransArgs p) {
   }
   if (t >= p.g_items) return;
   const uint32_t r = fdiv(t, p.dgp), z = fdiv(r, p.dgy), y = r - z * p.dgy.d;
-  const int xp = 2 * (int)(t - r * p.dgp.d), c = 8 * ((int)blockIdx.y - p.xgroups);
+  const int xp = 2 * (int)(t - r * p.dgp.d), c = 8 * ((int)row - p.xgroups);
 #pragma unroll
   for (int e = 0; e < 2; e++) {
     if (xp + e >= p.nx) continue;
     const size_t w = (size_t)(xp + e) + (size_t)p.nx * ((size_t)y + (size_t)p.ny * (size_t)z);
-    v[e] = *reinterpret_cast<const bf16x8 *>(p.g + w * p.cout + c);
+    v[e] = *reinterpret_cast<const bf16x8 *>(p.g + w * COUT + c);
   }
   const size_t plane = 2 * (size_t)p.g_items;
   const size_t base = (size_t)c * plane + 2 * (size_t)t;
@@ -1102,31 +1137,6 @@ __global__ __launch_bounds__(256) void k_dw_reduce(int cout, int cin, int rows_x
   float *o = dW + ((size_t)co * cin + ci) * 27 + t;
   *o = accumulate ? *o + s : s;
 }
-// bias gradient: partials of db[c] = sum_v g[v][c], sixteen loads in flight
-template <int C>
-__global__ __launch_bounds__(256) void k_bias_grad(uint32_t n, const bf16 *__restrict__ g, float *__restrict__ part) {
-  constexpr uint32_t VL = 256 / C, STEP = BG_BLOCKS * VL, U = 16;
-  const uint32_t c = threadIdx.x % C, vl = threadIdx.x / C;
-  float s = 0.0f;
-  uint32_t v = blockIdx.x * VL + vl;
-  for (; (uint64_t)v + (U - 1) * STEP < n; v += U * STEP) {
-    bf16 x[U];
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) x[u] = g[(size_t)(v + u * STEP) * C + c];
-#pragma unroll
-    for (uint32_t u = 0; u < U; u++) s += bf(x[u]);
-  }
-  for (; v < n; v += STEP) s += bf(g[(size_t)v * C + c]);
-  __shared__ float sh[256];
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  if (vl == 0) {
-    float t = 0.0f;
-    for (uint32_t k = 0; k < VL; k++) t += sh[k * C + c];
-    part[blockIdx.x * C + c] = t;
-  }
-}
-
 template <int COUT>
 static void launch_dw(unsigned nb, const G3 &g, const DwPlan &d, const bf16 *gt, const bf16 *xt, float *part,
                       hipStream_t s) {
@@ -1151,7 +1161,7 @@ static void launch_dw_layer(const G3 &g, const ConvSpec &c, const bf16 *a, const
   p.nx = g.nx; p.ny = g.ny; p.nz = g.nz;
   p.P = d.P;
   p.anx = ga.nx; p.any = ga.ny;
-  p.ca = c.ca; p.cb = c.cb; p.cout = c.cout;
+  p.ca = c.ca; p.cb = c.cb;
   p.a = a; p.b = b; p.g = gpre;
   p.xt = xt; p.gt = gt;
   p.xgroups = d.rows_x / 8;
@@ -1161,20 +1171,22 @@ static void launch_dw_layer(const G3 &g, const ConvSpec &c, const bf16 *a, const
   p.dgy = make_fastdiv((uint32_t)g.ny);
   p.x_items = (uint32_t)(g.nz + 2) * (uint32_t)(g.ny + 2) * p.dxp.d;
   p.g_items = (uint32_t)g.nz * (uint32_t)g.ny * p.dgp.d;
-  k_to_t<<<dim3(nblk(p.x_items > p.g_items ? p.x_items : p.g_items), p.xgroups + c.cout / 8), 256, 0, s>>>(p);
+  p.n = g.n();
+  p.bpart = part + dw_bias_at(d, c.cout);
+  p.dnb = make_fastdiv(nblk(p.x_items > p.g_items ? p.x_items : p.g_items));
+  const unsigned tb = BG_BLOCKS + p.dnb.d * (unsigned)(p.xgroups + c.cout / 8);
   const unsigned nb = (unsigned)(3 * (d.rows_x / 16) * d.S);
-  float *bpart = part + dw_bias_at(d, c.cout);
   if (c.cout == 16) {
+    k_to_t<16><<<tb, 256, 0, s>>>(p);
     launch_dw<16>(nb, g, d, gt, xt, part, s);
-    k_bias_grad<16><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
   } else if (c.cout == 32) {
+    k_to_t<32><<<tb, 256, 0, s>>>(p);
     launch_dw<32>(nb, g, d, gt, xt, part, s);
-    k_bias_grad<32><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
   } else {
+    k_to_t<64><<<tb, 256, 0, s>>>(p);
     launch_dw<64>(nb, g, d, gt, xt, part, s);
-    k_bias_grad<64><<<BG_BLOCKS, 256, 0, s>>>(g.n(), gpre, bpart);
   }
-  k_dw_reduce<<<nblk((uint64_t)c.cout * c.cin() * 27) + 1, 256, 0, s>>>(c.cout, c.cin(), d.rows_x, d.S, part, bpart, dW,
+  k_dw_reduce<<<nblk((uint64_t)c.cout * c.cin() * 27) + 1, 256, 0, s>>>(c.cout, c.cin(), d.rows_x, d.S, part, p.bpart, dW,
                                                                         db, accumulate ? 1 : 0);
 }
 void launch_conv_dw(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre,
