@@ -734,6 +734,7 @@ void launch_skip_grad(const G3 &g, const bf16 *gcat, int ctot, int off, const G3
 
 // head backward: gd0 and per-block partial sums of dwh (16) and dbh (1)
 constexpr int HB_BLOCKS = 512;
+static_assert(HB_BLOCKS * 17 == HEAD_PART);
 __global__ __launch_bounds__(256) void k_head_bwd(uint32_t n, const bf16 *__restrict__ d0, const float *__restrict__ gy,
                                                   const float *__restrict__ wh, bf16 *__restrict__ gd0,
                                                   float *__restrict__ part) {
@@ -768,19 +769,12 @@ __global__ __launch_bounds__(256) void k_head_bwd(uint32_t n, const bf16 *__rest
     __syncthreads();
   }
 }
-__global__ __launch_bounds__(32) void k_head_bwd_reduce(const float *__restrict__ part, float *__restrict__ dwh,
-                                                        float *__restrict__ dbh, int accumulate) {
-  const int c = threadIdx.x;
-  if (c >= 17) return;
-  float s = 0.0f;
-  for (int b = 0; b < HB_BLOCKS; b++) s += part[b * 17 + c];
-  float *o = c < 16 ? dwh + c : dbh;
-  *o = accumulate ? *o + s : s;
-}
 void launch_head_bwd(const G3 &g, const bf16 *d0, const float *gy, const float *wh, bf16 *gd0, float *part,
-                     float *dwh, float *dbh, bool accumulate, hipStream_t s) {
+                     float *dwh, float *dbh, DwSums &sums, hipStream_t s) {
   k_head_bwd<<<HB_BLOCKS, 256, 0, s>>>(g.n(), d0, gy, wh, gd0, part);
-  k_head_bwd_reduce<<<1, 32, 0, s>>>(part, dwh, dbh, accumulate ? 1 : 0);
+  sums.hpart = part;
+  sums.dwh = dwh;
+  sums.dbh = dbh;
 }
 
 // ------------------------------------------------------------ weight gradients
@@ -1105,8 +1099,10 @@ __global__ __launch_bounds__(256) void k_dw(int ny, int nz, int P, int rows_x, i
   }
 }
 // a[first] + a[first + step] + ... (count terms) in that order, U loads in flight
+typedef const float __attribute__((address_space(1))) *gf32c;
+typedef float __attribute__((address_space(1))) *gf32;
 template <int U>
-__device__ __forceinline__ float seq_sum32(const float *__restrict__ a, int count, size_t first, size_t step) {
+__device__ __forceinline__ float seq_sum32(gf32c a, int count, size_t first, size_t step) {
   float s = 0.0f;
   for (int k0 = 0; k0 < count; k0 += U) {
     float x[U];
@@ -1118,25 +1114,42 @@ __device__ __forceinline__ float seq_sum32(const float *__restrict__ a, int coun
   }
   return s;
 }
-// dW from the row splits' partials (input channel fastest, as they lie), and
-// in the last block the bias gradient from its partials
-__global__ __launch_bounds__(256) void k_dw_reduce(int cout, int cin, int rows_x, int S, const float *__restrict__ part,
-                                                   const float *__restrict__ bpart, float *__restrict__ dW,
-                                                   float *__restrict__ db, int accumulate) {
-  if (blockIdx.x == gridDim.x - 1) {
+// Every layer's dW from its row splits' partials (input channel fastest, as
+// they lie), in a layer's last block the bias gradient from its partials, and
+// in the launch's last the head's.  A launch a layer is bound by the round
+// trips of one sum (6 us, and 10 for the head's): eight layers and the head
+// 59 us a training step at 80x160x80, 17 in one launch.
+__global__ __launch_bounds__(256) void k_dw_reduce(DwSums) {
+  // indexed by block where the arguments lie
+  const DwSums &a = *(const DwSums *)__builtin_amdgcn_kernarg_segment_ptr();
+  if (a.hpart && blockIdx.x == a.blocks) {
     const int c = threadIdx.x;
-    if (c >= cout) return;
-    const float s = seq_sum32<32>(bpart, BG_BLOCKS, (size_t)c, (size_t)cout);
-    db[c] = accumulate ? db[c] + s : s;
+    if (c >= 17) return;
+    const float s = seq_sum32<32>((gf32c)a.hpart, HB_BLOCKS, (size_t)c, 17);
+    *(c < 16 ? (gf32)a.dwh + c : (gf32)a.dbh) = s;
     return;
   }
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e >= cout * cin * 27) return;
-  const int ci = e % cin, co = (e / cin) % cout, t = e / (cin * cout);
-  const float s = seq_sum32<16>(part, S, ((size_t)t * cout + co) * rows_x + ci, (size_t)27 * cout * rows_x);
-  float *o = dW + ((size_t)co * cin + ci) * 27 + t;
-  *o = accumulate ? *o + s : s;
+  int k = 0;
+  while (k + 1 < a.n && blockIdx.x >= a.e[k + 1].block0) k++;
+  const DwSums::Entry &p = a.e[k];
+  const int e = (int)(blockIdx.x - p.block0) * 256 + threadIdx.x, total = p.cout * p.cin * 27;
+  const int nb = (total + 255) / 256;
+  if ((int)(blockIdx.x - p.block0) == nb) {
+    const int c = threadIdx.x;
+    if (c >= p.cout) return;
+    ((gf32)p.db)[c] = seq_sum32<32>((gf32c)p.bpart, BG_BLOCKS, (size_t)c, (size_t)p.cout);
+    return;
+  }
+  if (e >= total) return;
+  const int ci = e % p.cin, co = (e / p.cin) % p.cout, t = e / (p.cin * p.cout);
+  const float s = seq_sum32<16>((gf32c)p.part, p.S, ((size_t)t * p.cout + co) * p.rows_x + ci,
+                                (size_t)27 * p.cout * p.rows_x);
+  ((gf32)p.dW)[((size_t)co * p.cin + ci) * 27 + t] = s;
 }
+void launch_dw_reduce(const DwSums &sums, hipStream_t s) {
+  k_dw_reduce<<<sums.blocks + (sums.hpart ? 1 : 0), 256, 0, s>>>(sums);
+}
+
 template <int COUT>
 static void launch_dw(unsigned nb, const G3 &g, const DwPlan &d, const bf16 *gt, const bf16 *xt, float *part,
                       hipStream_t s) {
@@ -1154,7 +1167,7 @@ static void launch_dw(unsigned nb, const G3 &g, const DwPlan &d, const bf16 *gt,
 }
 // weight and bias gradients of one layer (cb = 2: the first)
 static void launch_dw_layer(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b,
-                            const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW, float *db, bool accumulate,
+                            const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW, float *db, DwSums &sums,
                             hipStream_t s) {
   const DwPlan d = dw_plan(g, c);
   TransArgs p;
@@ -1186,16 +1199,17 @@ static void launch_dw_layer(const G3 &g, const ConvSpec &c, const bf16 *a, const
     k_to_t<64><<<tb, 256, 0, s>>>(p);
     launch_dw<64>(nb, g, d, gt, xt, part, s);
   }
-  k_dw_reduce<<<nblk((uint64_t)c.cout * c.cin() * 27) + 1, 256, 0, s>>>(c.cout, c.cin(), d.rows_x, d.S, part, p.bpart, dW,
-                                                                        db, accumulate ? 1 : 0);
+  DwSums::Entry &e = sums.e[sums.n++];
+  e = {part, p.bpart, dW, db, c.cout, c.cin(), d.rows_x, d.S, sums.blocks};
+  sums.blocks += (uint32_t)nblk((uint64_t)c.cout * c.cin() * 27) + 1;
 }
 void launch_conv_dw(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre,
-                    bf16 *xt, bf16 *gt, float *part, float *dW, float *db, bool accumulate, hipStream_t s) {
-  launch_dw_layer(g, c, a, ga, b, gpre, xt, gt, part, dW, db, accumulate, s);
+                    bf16 *xt, bf16 *gt, float *part, float *dW, float *db, DwSums &sums, hipStream_t s) {
+  launch_dw_layer(g, c, a, ga, b, gpre, xt, gt, part, dW, db, sums, s);
 }
 void launch_conv_in_dw(const G3 &g, const bf16 *x0, const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW,
-                       float *db, bool accumulate, hipStream_t s) {
-  launch_dw_layer(g, ConvSpec{0, 2, 16}, nullptr, g, x0, gpre, xt, gt, part, dW, db, accumulate, s);
+                       float *db, DwSums &sums, hipStream_t s) {
+  launch_dw_layer(g, ConvSpec{0, 2, 16}, nullptr, g, x0, gpre, xt, gt, part, dW, db, sums, s);
 }
 
 // ------------------------------------------------------------ solver transforms

@@ -129,16 +129,15 @@ int work_alloc(Work &W, const G3 &g, bool train) {
     if (!rc) rc |= dalloc(L, &W.gp1, n1 * 16);
     if (!rc) rc |= dalloc(L, &W.gs0, n0 * 16);
     if (!rc) rc |= dalloc(L, &W.ga0, n0 * 16);
-    // weight-gradient scratch: the largest layer at each level
+    // weight-gradient scratch: operands of the largest layer, partials of all
     const G3 lg[NCONV] = {W.g0, W.g1, W.g1, W.g2, W.g2, W.g1, W.g0};
     size_t xt = dw_xt_elems(W.g0, ConvSpec{0, 2, 16}), gt = dw_gt_elems(W.g0, ConvSpec{0, 2, 16});
-    size_t part = dw_part_elems(W.g0, ConvSpec{0, 2, 16});
+    size_t part = HEAD_PART + dw_part_elems(W.g0, ConvSpec{0, 2, 16});
     for (int l = 0; l < NCONV; l++) {
       xt = std::max(xt, dw_xt_elems(lg[l], kSpec[l]));
       gt = std::max(gt, dw_gt_elems(lg[l], kSpec[l]));
-      part = std::max(part, dw_part_elems(lg[l], kSpec[l]));
+      part += dw_part_elems(lg[l], kSpec[l]);
     }
-    part = std::max(part, (size_t)512 * 17);
     if (!rc) rc |= dalloc(L, &W.xt, xt);
     if (!rc) rc |= dalloc(L, &W.gt, gt);
     if (!rc) rc |= dalloc(L, &W.part, part);
@@ -184,35 +183,43 @@ void backward(PyroNet *N, Work &W, const bf16 *x0) {
   const float *P = N->params;
   float *G = N->grads;
   const G3 &g0 = W.g0, &g1 = W.g1, &g2 = W.g2;
-  launch_head_bwd(g0, W.d0, W.gy, P + N->wh, W.gd0, W.part, G + N->wh, G + N->bh, false, s);
+  DwSums D;
+  float *part = W.part + HEAD_PART;
+  // the weight gradient's partials of a layer, summed at the end
+  auto conv_dw = [&](const G3 &g, int l, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre) {
+    launch_conv_dw(g, kSpec[l], a, ga, b, gpre, W.xt, W.gt, part, G + N->w[l], G + N->b[l], D, s);
+    part += dw_part_elems(g, kSpec[l]);
+  };
+  launch_head_bwd(g0, W.d0, W.gy, P + N->wh, W.gd0, W.part, G + N->wh, G + N->bh, D, s);
   // d0 = conv([up(d1), s0])
-  launch_conv_dw(g0, kSpec[L0C], W.d1, g1, W.s0, W.gd0, W.xt, W.gt, W.part, G + N->w[L0C], G + N->b[L0C], false, s);
+  conv_dw(g0, L0C, W.d1, g1, W.s0, W.gd0);
   launch_conv3(g0, nullptr, g1, 0, W.gd0, 16, N->wpt[L0C], nullptr, 48, false, W.gcat0, s);
   launch_unup_relu(g0, W.gcat0, 48, 32, g1, W.d1, W.gd1, s);
   // d1 = conv([up(c2), s1])
-  launch_conv_dw(g1, kSpec[L1C], W.c2, g2, W.s1, W.gd1, W.xt, W.gt, W.part, G + N->w[L1C], G + N->b[L1C], false, s);
+  conv_dw(g1, L1C, W.c2, g2, W.s1, W.gd1);
   launch_conv3(g1, nullptr, g2, 0, W.gd1, 32, N->wpt[L1C], nullptr, 96, false, W.gcat1, s);
   launch_unup_relu(g1, W.gcat1, 96, 64, g2, W.c2, W.gc2, s);
   // c2 = conv(a2)
-  launch_conv_dw(g2, kSpec[L2B], nullptr, g2, W.a2, W.gc2, W.xt, W.gt, W.part, G + N->w[L2B], G + N->b[L2B], false, s);
+  conv_dw(g2, L2B, nullptr, g2, W.a2, W.gc2);
   launch_conv3(g2, nullptr, g2, 0, W.gc2, 64, N->wpt[L2B], nullptr, 64, false, W.ga2, s);
   launch_relu_bwd(g2.n() * 64, W.a2, W.ga2, s);
   // a2 = conv(p2)
-  launch_conv_dw(g2, kSpec[L2A], nullptr, g2, W.p2, W.ga2, W.xt, W.gt, W.part, G + N->w[L2A], G + N->b[L2A], false, s);
+  conv_dw(g2, L2A, nullptr, g2, W.p2, W.ga2);
   launch_conv3(g2, nullptr, g2, 0, W.ga2, 64, N->wpt[L2A], nullptr, 32, false, W.gp2, s);
   // s1: decoder concat + pooling
   launch_skip_grad(g1, W.gcat1, 96, 64, g2, W.gp2, W.s1, 32, W.gs1, s);
-  launch_conv_dw(g1, kSpec[L1B], nullptr, g1, W.a1, W.gs1, W.xt, W.gt, W.part, G + N->w[L1B], G + N->b[L1B], false, s);
+  conv_dw(g1, L1B, nullptr, g1, W.a1, W.gs1);
   launch_conv3(g1, nullptr, g1, 0, W.gs1, 32, N->wpt[L1B], nullptr, 32, false, W.ga1, s);
   launch_relu_bwd(g1.n() * 32, W.a1, W.ga1, s);
-  launch_conv_dw(g1, kSpec[L1A], nullptr, g1, W.p1, W.ga1, W.xt, W.gt, W.part, G + N->w[L1A], G + N->b[L1A], false, s);
+  conv_dw(g1, L1A, nullptr, g1, W.p1, W.ga1);
   launch_conv3(g1, nullptr, g1, 0, W.ga1, 32, N->wpt[L1A], nullptr, 16, false, W.gp1, s);
   // s0
   launch_skip_grad(g0, W.gcat0, 48, 32, g1, W.gp1, W.s0, 16, W.gs0, s);
-  launch_conv_dw(g0, kSpec[L0B], nullptr, g0, W.a0, W.gs0, W.xt, W.gt, W.part, G + N->w[L0B], G + N->b[L0B], false, s);
+  conv_dw(g0, L0B, nullptr, g0, W.a0, W.gs0);
   launch_conv3(g0, nullptr, g0, 0, W.gs0, 16, N->wpt[L0B], nullptr, 16, false, W.ga0, s);
   launch_relu_bwd(g0.n() * 16, W.a0, W.ga0, s);
-  launch_conv_in_dw(g0, x0, W.ga0, W.xt, W.gt, W.part, G + N->w0a, G + N->b0a, false, s);
+  launch_conv_in_dw(g0, x0, W.ga0, W.xt, W.gt, part, G + N->w0a, G + N->b0a, D, s);
+  launch_dw_reduce(D, s);
 }
 
 int nsync(PyroNet *N) {
@@ -706,10 +713,12 @@ int pyro_debug_conv_dw(int ca, int cb, int cout, uint32_t nx, uint32_t ny, uint3
   if (!rc && ca) rc = up(a, nh * ca, da);
   if (!rc) rc = up(g, n * cout, dg);
   if (!rc) {
+    DwSums D;
     if (cb == 2)
-      launch_conv_in_dw(gg, dbb, dg, xt, gt, part, ddw, ddb, false, nullptr);
+      launch_conv_in_dw(gg, dbb, dg, xt, gt, part, ddw, ddb, D, nullptr);
     else
-      launch_conv_dw(gg, c, da, gh, dbb, dg, xt, gt, part, ddw, ddb, false, nullptr);
+      launch_conv_dw(gg, c, da, gh, dbb, dg, xt, gt, part, ddw, ddb, D, nullptr);
+    launch_dw_reduce(D, nullptr);
     if (hipDeviceSynchronize() != hipSuccess) rc = PYRO_E_HIP;
     if (!rc && hipMemcpy(dW, ddw, (size_t)cout * c.cin() * 27 * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
       rc = PYRO_E_HIP;

@@ -82,16 +82,35 @@ DwPlan dw_plan(const G3 &g, const ConvSpec &c);
 size_t dw_xt_elems(const G3 &g, const ConvSpec &c);
 size_t dw_gt_elems(const G3 &g, const ConvSpec &c);
 size_t dw_part_elems(const G3 &g, const ConvSpec &c);
+// Gradients whose partials are still to be summed; each entry's partials are
+// its own until launch_dw_reduce.
+constexpr int DW_SUMS = 8;
+constexpr int HEAD_PART = 512 * 17;  // partials of the head's gradients
+struct DwSums {
+  struct Entry {
+    const float *part, *bpart;
+    float *dW, *db;
+    int cout, cin, rows_x, S;
+    uint32_t block0;
+  };
+  int n = 0;  // layers
+  uint32_t blocks = 0;
+  const float *hpart = nullptr;  // the head's
+  float *dwh = nullptr, *dbh = nullptr;
+  Entry e[DW_SUMS];
+};
 void launch_conv_dw(const G3 &g, const ConvSpec &c, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre,
-                    bf16 *xt, bf16 *gt, float *part, float *dW, float *db, bool accumulate, hipStream_t s);
+                    bf16 *xt, bf16 *gt, float *part, float *dW, float *db, DwSums &sums, hipStream_t s);
 // first-layer weight gradient (x0 has 2 channels)
 void launch_conv_in_dw(const G3 &g, const bf16 *x0, const bf16 *gpre, bf16 *xt, bf16 *gt, float *part, float *dW,
-                       float *db, bool accumulate, hipStream_t s);
+                       float *db, DwSums &sums, hipStream_t s);
+// the gradients from the partials of all entries
+void launch_dw_reduce(const DwSums &sums, hipStream_t s);
 
 // backward glue
-// gd0[v][c] = bf16(gy[v] * wh[c]) where d0[v][c] > 0 else 0; dwh, dbh partial sums
+// gd0[v][c] = bf16(gy[v] * wh[c]) where d0[v][c] > 0 else 0; dwh, dbh as HEAD_PART partial sums
 void launch_head_bwd(const G3 &g, const bf16 *d0, const float *gy, const float *wh, bf16 *gd0, float *part,
-                     float *dwh, float *dbh, bool accumulate, hipStream_t s);
+                     float *dwh, float *dbh, DwSums &sums, hipStream_t s);
 // gcoarse[u][c] = bf16(sum over children v of u of gcat[v][c] (c < ca)) where act[u][c] > 0
 void launch_unup_relu(const G3 &g, const bf16 *gcat, int ctot, int ca, const G3 &gc, const bf16 *act, bf16 *gcoarse,
                       hipStream_t s);
