@@ -150,8 +150,25 @@ struct ConvArgs {
   int anx, any;  // half-resolution grid of `a`
   const bf16 *a, *b, *wp;
   const float *bias;
+  const bf16 *act;  // without RELU, if not null: the result is 0 where act is not positive
   bf16 *out;
 };
+// act at a voxel's four channels from co on, positive if there is no act (a
+// pass of its own over the gradient and act took 25 us a training step at
+// 80x160x80, the reads here 4).  A
+// voxel outside the grid reads one inside: no branch, all loads in flight.
+template <int COUT>
+__device__ __forceinline__ bf16x4 act_at(const ConvArgs &p, int x, int y, int z, int co) {
+  bf16x4 m = {tobf(1.0f), tobf(1.0f), tobf(1.0f), tobf(1.0f)};
+  if (p.act) {
+    x = x < p.nx ? x : p.nx - 1;
+    y = y < p.ny ? y : p.ny - 1;
+    z = z < p.nz ? z : p.nz - 1;
+    m = *reinterpret_cast<const bf16x4 *>(
+        p.act + ((size_t)x + (size_t)p.nx * ((size_t)y + (size_t)p.ny * (size_t)z)) * COUT + co);
+  }
+  return m;
+}
 
 // footprint offset (in voxels) of tap t relative to footprint voxel (col, w, nb)
 __device__ __forceinline__ constexpr int tap_off(int t) {
@@ -298,6 +315,13 @@ __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
     wp += (size_t)(CCB == 32 ? 27 : 14) * COUT * 32;
   }
   const int gx = x0 + col, gy = y0 + w;
+  bf16x4 act[4][MB];
+  if (!RELU) {
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+      for (int m = 0; m < MB; m++) act[nb][m] = act_at<COUT>(p, gx, gy, z0 + nb, c0 + m * 16 + 4 * j);
+  }
   if (gx >= p.nx || gy >= p.ny) return;
 #pragma unroll
   for (int nb = 0; nb < 4; nb++) {
@@ -311,7 +335,7 @@ __global__ __launch_bounds__(256, 3) void k_conv3(ConvArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         float t = acc[m][nb][i] + (p.bias ? p.bias[co + i] : 0.0f);
-        if (RELU) t = t > 0.0f ? t : 0.0f;
+        if (RELU ? !(t > 0.0f) : !(bf(act[nb][m][i]) > 0.0f)) t = 0.0f;
         o[i] = tobf(t);
       }
       *reinterpret_cast<bf16x4 *>(p.out + v * COUT + co) = o;
@@ -442,6 +466,13 @@ __global__ __launch_bounds__(256, 2) void k_conv3_16(ConvArgs p) {
     }
   }
   const int gx = x0 + col;
+  bf16x4 act[4][4];
+  if (!RELU) {
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+#pragma unroll
+      for (int y = 0; y < 4; y++) act[z][y] = act_at<16>(p, gx, y0 + wy + y, z0 + wz + z, 4 * j);
+  }
   if (gx >= p.nx) return;
   float bias[4];
 #pragma unroll
@@ -457,7 +488,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3_16(ConvArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         float t = acc[z][y][i] + bias[i];
-        if (RELU) t = t > 0.0f ? t : 0.0f;
+        if (RELU ? !(t > 0.0f) : !(bf(act[z][y][i]) > 0.0f)) t = 0.0f;
         o[i] = tobf(t);
       }
       *reinterpret_cast<bf16x4 *>(p.out + v * 16 + 4 * j) = o;
@@ -466,11 +497,11 @@ __global__ __launch_bounds__(256, 2) void k_conv3_16(ConvArgs p) {
 }
 
 bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *b, int cb, const bf16 *wp,
-                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s) {
+                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s, const bf16 *act) {
   ConvArgs p;
   p.nx = g.nx; p.ny = g.ny; p.nz = g.nz;
   p.anx = ga.nx; p.any = ga.ny;
-  p.a = a; p.b = b; p.wp = wp; p.bias = bias; p.out = out;
+  p.a = a; p.b = b; p.wp = wp; p.bias = bias; p.act = act; p.out = out;
   const unsigned nb = (unsigned)(((g.nx + CV_TX - 1) / CV_TX) * ((g.ny + CV_TY - 1) / CV_TY) *
                                  ((g.nz + CV_TZ - 1) / CV_TZ));
   const unsigned nb16 = (unsigned)(((g.nx + CV_TX - 1) / CV_TX) * ((g.ny + CS_Y - 1) / CS_Y) *
@@ -658,20 +689,6 @@ void launch_pool(const G3 &g, const bf16 *in, int c, bf16 *out, hipStream_t s) {
 }
 
 // ------------------------------------------------------------ backward glue
-__global__ __launch_bounds__(256) void k_relu_bwd(uint32_t n8, const bf16 *__restrict__ act, bf16 *__restrict__ g) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= n8) return;
-  const bf16x8 a = *reinterpret_cast<const bf16x8 *>(act + 8 * (size_t)i);
-  bf16x8 v = *reinterpret_cast<const bf16x8 *>(g + 8 * (size_t)i);
-#pragma unroll
-  for (int k = 0; k < 8; k++)
-    if (!(bf(a[k]) > 0.0f)) v[k] = tobf(0.0f);
-  *reinterpret_cast<bf16x8 *>(g + 8 * (size_t)i) = v;
-}
-void launch_relu_bwd(uint32_t n, const bf16 *act, bf16 *g, hipStream_t s) {
-  k_relu_bwd<<<nblk(n / 8), 256, 0, s>>>(n / 8, act, g);
-}
-
 __global__ __launch_bounds__(256) void k_unup_relu(int nx, int ny, int nz, const bf16 *__restrict__ gcat, int ctot,
                                                    int ca, const bf16 *__restrict__ act, bf16 *__restrict__ gc) {
   const int cnx = (nx + 1) / 2, cny = (ny + 1) / 2, cnz = (nz + 1) / 2;

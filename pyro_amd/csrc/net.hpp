@@ -61,9 +61,11 @@ void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s);
 void launch_pack_bf16(const float *w, uint32_t n, bf16 *out, hipStream_t s);
 
 // out[v][0..cout) = act(bias + sum_taps W * in), in = [up(a), b]; false (and
-// nothing launched) for a channel combination the network does not use
+// nothing launched) for a channel combination the network does not use.  With
+// act (and not relu) out is 0 where act[v][c] is not positive: the gradient
+// before a ReLU.
 bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *b, int cb, const bf16 *wp,
-                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s);
+                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s, const bf16 *act = nullptr);
 // first layer (2 input channels): a0 = relu(b + W * x0) on MFMA, weights
 // packed by launch_pack_conv_in into [2][16][32] BF16
 void launch_pack_conv_in(const float *W, bf16 *wp, hipStream_t s);
@@ -117,8 +119,6 @@ void launch_unup_relu(const G3 &g, const bf16 *gcat, int ctot, int ca, const G3 
 // gs[v][c] = bf16((gcat[v][off + c] + gp[parent][c] / cnt(parent)) ) where s[v][c] > 0 else 0
 void launch_skip_grad(const G3 &g, const bf16 *gcat, int ctot, int off, const G3 &gc, const bf16 *gp, const bf16 *s,
                       int c, bf16 *gs, hipStream_t st);
-// g[v][c] = act[v][c] > 0 ? g : 0   (in place)
-void launch_relu_bwd(uint32_t n, const bf16 *act, bf16 *g, hipStream_t s);
 
 // input / output transforms of the solver
 // x0[v] = (bf16(r[v] * inv), fluid ? 1 : 0)
