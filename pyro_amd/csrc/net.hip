@@ -193,12 +193,12 @@ void backward(PyroNet *N, Work &W, const bf16 *x0) {
   launch_head_bwd(g0, W.d0, W.gy, P + N->wh, W.gd0, W.part, G + N->wh, G + N->bh, D, s);
   // d0 = conv([up(d1), s0])
   conv_dw(g0, L0C, W.d1, g1, W.s0, W.gd0);
-  launch_conv3(g0, nullptr, g1, 0, W.gd0, 16, N->wpt[L0C], nullptr, 48, false, W.gcat0, s);
-  launch_unup_relu(g0, W.gcat0, 48, 32, g1, W.d1, W.gd1, s);
+  launch_conv3(g0, nullptr, g1, 0, W.gd0, 16, N->wpt[L0C], nullptr, 48, false, W.gcat0, s, nullptr, 32);
+  launch_unup_relu(g0, W.gcat0, 32, g1, W.d1, W.gd1, s);
   // d1 = conv([up(c2), s1])
   conv_dw(g1, L1C, W.c2, g2, W.s1, W.gd1);
-  launch_conv3(g1, nullptr, g2, 0, W.gd1, 32, N->wpt[L1C], nullptr, 96, false, W.gcat1, s);
-  launch_unup_relu(g1, W.gcat1, 96, 64, g2, W.c2, W.gc2, s);
+  launch_conv3(g1, nullptr, g2, 0, W.gd1, 32, N->wpt[L1C], nullptr, 96, false, W.gcat1, s, nullptr, 64);
+  launch_unup_relu(g1, W.gcat1, 64, g2, W.c2, W.gc2, s);
   // c2 = conv(a2)
   conv_dw(g2, L2B, nullptr, g2, W.a2, W.gc2);
   launch_conv3(g2, nullptr, g2, 0, W.gc2, 64, N->wpt[L2B], nullptr, 64, false, W.ga2, s, W.a2);
@@ -206,13 +206,13 @@ void backward(PyroNet *N, Work &W, const bf16 *x0) {
   conv_dw(g2, L2A, nullptr, g2, W.p2, W.ga2);
   launch_conv3(g2, nullptr, g2, 0, W.ga2, 64, N->wpt[L2A], nullptr, 32, false, W.gp2, s);
   // s1: decoder concat + pooling
-  launch_skip_grad(g1, W.gcat1, 96, 64, g2, W.gp2, W.s1, 32, W.gs1, s);
+  launch_skip_grad(g1, W.gcat1 + (size_t)g1.n() * 64, W.gp2, W.s1, 32, W.gs1, s);
   conv_dw(g1, L1B, nullptr, g1, W.a1, W.gs1);
   launch_conv3(g1, nullptr, g1, 0, W.gs1, 32, N->wpt[L1B], nullptr, 32, false, W.ga1, s, W.a1);
   conv_dw(g1, L1A, nullptr, g1, W.p1, W.ga1);
   launch_conv3(g1, nullptr, g1, 0, W.ga1, 32, N->wpt[L1A], nullptr, 16, false, W.gp1, s);
   // s0
-  launch_skip_grad(g0, W.gcat0, 48, 32, g1, W.gp1, W.s0, 16, W.gs0, s);
+  launch_skip_grad(g0, W.gcat0 + (size_t)g0.n() * 32, W.gp1, W.s0, 16, W.gs0, s);
   conv_dw(g0, L0B, nullptr, g0, W.a0, W.gs0);
   launch_conv3(g0, nullptr, g0, 0, W.gs0, 16, N->wpt[L0B], nullptr, 16, false, W.ga0, s, W.a0);
   launch_conv_in_dw(g0, x0, W.ga0, W.xt, W.gt, part, G + N->w0a, G + N->b0a, D, s);

@@ -63,9 +63,11 @@ void launch_pack_bf16(const float *w, uint32_t n, bf16 *out, hipStream_t s);
 // out[v][0..cout) = act(bias + sum_taps W * in), in = [up(a), b]; false (and
 // nothing launched) for a channel combination the network does not use.  With
 // act (and not relu) out is 0 where act[v][c] is not positive: the gradient
-// before a ReLU.
+// before a ReLU.  With split (a multiple of 16, cout > 16) out is
+// [v][0..split) and, after all voxels, [v][split..cout).
 bool launch_conv3(const G3 &g, const bf16 *a, const G3 &ga, int ca, const bf16 *b, int cb, const bf16 *wp,
-                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s, const bf16 *act = nullptr);
+                  const float *bias, int cout, bool relu, bf16 *out, hipStream_t s, const bf16 *act = nullptr,
+                  int split = 0);
 // first layer (2 input channels): a0 = relu(b + W * x0) on MFMA, weights
 // packed by launch_pack_conv_in into [2][16][32] BF16
 void launch_pack_conv_in(const float *W, bf16 *wp, hipStream_t s);
@@ -113,12 +115,11 @@ void launch_dw_reduce(const DwSums &sums, hipStream_t s);
 // gd0[v][c] = bf16(gy[v] * wh[c]) where d0[v][c] > 0 else 0; dwh, dbh as HEAD_PART partial sums
 void launch_head_bwd(const G3 &g, const bf16 *d0, const float *gy, const float *wh, bf16 *gd0, float *part,
                      float *dwh, float *dbh, DwSums &sums, hipStream_t s);
-// gcoarse[u][c] = bf16(sum over children v of u of gcat[v][c] (c < ca)) where act[u][c] > 0
-void launch_unup_relu(const G3 &g, const bf16 *gcat, int ctot, int ca, const G3 &gc, const bf16 *act, bf16 *gcoarse,
+// gcoarse[u][c] = bf16(sum over children v of u of gcat[v][c]) where act[u][c] > 0
+void launch_unup_relu(const G3 &g, const bf16 *gcat, int ca, const G3 &gc, const bf16 *act, bf16 *gcoarse,
                       hipStream_t s);
-// gs[v][c] = bf16((gcat[v][off + c] + gp[parent][c] / cnt(parent)) ) where s[v][c] > 0 else 0
-void launch_skip_grad(const G3 &g, const bf16 *gcat, int ctot, int off, const G3 &gc, const bf16 *gp, const bf16 *s,
-                      int c, bf16 *gs, hipStream_t st);
+// gs[v][c] = bf16((gc[v][c] + gp[parent][c] / cnt(parent)) ) where s[v][c] > 0 else 0
+void launch_skip_grad(const G3 &g, const bf16 *gc, const bf16 *gp, const bf16 *s, int c, bf16 *gs, hipStream_t st);
 
 // input / output transforms of the solver
 // x0[v] = (bf16(r[v] * inv), fluid ? 1 : 0)
