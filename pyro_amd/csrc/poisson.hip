@@ -57,7 +57,7 @@ struct PyroPoisson {
   hipEvent_t ev_rr = nullptr;      // its copy
   double *cgpart = nullptr, *dev = nullptr;  // fused-CG partial sums and the iteration's scalars
   double nfluid = 0.0;
-  unsigned int *count = nullptr;  // device fluid-cell counter
+  unsigned int *count = nullptr;  // on the device: [0] fluid cells, [1] flags changed
   hipStream_t stream = nullptr;
   // solve timing, and the order between a simulation's stream and this one
   hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr, ev_sim = nullptr, ev_done = nullptr;
@@ -73,11 +73,12 @@ struct PyroPoisson {
   // seal_off[k] .. seal_off[k+1]-1), once per right-hand side
   uint8_t *fprev = nullptr;          // level-0 flags at the last labelling
   uint8_t *cc_open = nullptr;        // open[root]
-  unsigned int *cc_flag = nullptr;   // [0] sealed-cell counter, [1] flags changed
+  unsigned int *cc_flag = nullptr;   // sealed-cell counter
   uint32_t *seal_idx = nullptr, *seal_off = nullptr;
   uint32_t seal_cap = 0, seal_comp = 0, seal_cells = 0;
   int seal_mode = 1;                 // 0 never, 1 all methods but VCYCLE, 2 all
-  bool labelled = false, b_fresh = true;
+  bool formed = false;               // codes, count and labels are those of the level-0 flags
+  bool b_fresh = true;
 };
 
 namespace {
@@ -278,7 +279,6 @@ int relabel(PyroPoisson *P) {
   if (rc) return rc;
   P->seal_comp = (uint32_t)off.size() - 1;
   P->seal_cells = cnt;
-  P->labelled = true;
   P->b_fresh = true;
   return 0;
 }
@@ -287,22 +287,28 @@ int relabel(PyroPoisson *P) {
 // formed again only when those changed (fourteen launches otherwise spent on
 // every solved step).
 int set_flags_device(PyroPoisson *P, const uint8_t *sim_flags) {
-  PCHK(hipMemsetAsync(P->count, 0, 2 * sizeof(unsigned int), P->stream));
-  k_flags_from_sim<<<nblocks(P->n), 256, 0, P->stream>>>(P->n, sim_flags, P->pc[0].f, P->fprev, P->count + 1);
-  unsigned int c[2] = {0, 0};
-  PCHK(hipMemcpyAsync(c, P->count, sizeof(c), hipMemcpyDeviceToHost, P->stream));
-  int rc = sync(P);
-  if (rc) return rc;
-  if (!c[1] && P->labelled) return 0;
-  P->labelled = false;  // until the labels below are complete
-  launch_mg_setup(P->pc, P->nl_pc, P->stream);
-  k_count_fluid<<<COUNT_BLOCKS, 256, 0, P->stream>>>(P->n, P->pc[0].f, P->count);
-  PCHK(hipMemcpyAsync(c, P->count, sizeof(unsigned int), hipMemcpyDeviceToHost, P->stream));
-  rc = sync(P);
-  if (rc) return rc;
-  P->nfluid = (double)c[0];
-  P->nfluid1 = -1.0;
-  return relabel(P);
+  auto compare = [&](bool &changed) -> int {
+    PCHK(hipMemsetAsync(P->count + 1, 0, sizeof(unsigned int), P->stream));
+    k_flags_from_sim<<<nblocks(P->n), 256, 0, P->stream>>>(P->n, sim_flags, P->pc[0].f, P->fprev, P->count + 1);
+    unsigned int c = 0;
+    PCHK(hipMemcpyAsync(&c, P->count + 1, sizeof(c), hipMemcpyDeviceToHost, P->stream));
+    const int rc = sync(P);
+    changed = c != 0;
+    return rc;
+  };
+  auto form = [&]() -> int {
+    launch_mg_setup(P->pc, P->nl_pc, P->stream);
+    PCHK(hipMemsetAsync(P->count, 0, sizeof(unsigned int), P->stream));
+    k_count_fluid<<<COUNT_BLOCKS, 256, 0, P->stream>>>(P->n, P->pc[0].f, P->count);
+    unsigned int c = 0;
+    PCHK(hipMemcpyAsync(&c, P->count, sizeof(c), hipMemcpyDeviceToHost, P->stream));
+    const int rc = sync(P);
+    if (rc) return rc;
+    P->nfluid = (double)c;
+    P->nfluid1 = -1.0;
+    return relabel(P);
+  };
+  return follow_flags(P->formed, compare, form);
 }
 
 // b = the simulation's level-0 right-hand side, x = its level-0 phi (warm) or 0
@@ -403,6 +409,7 @@ int pyro_poisson_create(uint32_t nx, uint32_t ny, uint32_t nz, float h, const ui
   launch_mg_setup(P->pc, P->nl_pc, P->stream);
   if (sync(P)) return bail(PYRO_E_HIP);
   if ((rc = relabel(P))) return bail(rc);
+  P->formed = true;
   *out = P;
   return 0;
 }

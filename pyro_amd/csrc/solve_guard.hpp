@@ -1,6 +1,7 @@
-// solve_guard.hpp -- the residual watch of the iterative pressure solves
-// (poisson.hip).  Plain C++ without HIP so that the host test
-// tests/native/solve_guard_check.cpp compiles it with g++.
+// solve_guard.hpp -- control flow of the pressure solves (poisson.hip) whose
+// failures cannot be had on demand: the residual watch of the iterations, and
+// what follows the solid flags.  Plain C++ without HIP so that the host tests
+// tests/native/solve_guard_check.cpp and flags_check.cpp compile it with g++.
 //
 // Every relative residual a solve reads goes through ResidWatch::step:
 //  - NaN or Inf stops the solve with an error (a NaN residual would pass
@@ -27,6 +28,22 @@ struct ResidWatch {
     return Watch::Go;
   }
 };
+
+// What a handle has formed from its solid flags (neighbour codes, fluid count,
+// labels) follows new flags.  compare(changed) stores them and reports whether
+// they differ, form() forms everything anew; both return 0 or an error.  The
+// new flags are stored before the outcome is known, so nothing counts as formed
+// until it is: after an error (or a throw) the next call forms everything.
+template <class Compare, class Form>
+int follow_flags(bool &formed, Compare compare, Form form) {
+  const bool was = formed;
+  formed = false;
+  bool changed = true;
+  int rc = compare(changed);
+  if (!rc && (changed || !was)) rc = form();
+  formed = rc == 0;
+  return rc;
+}
 
 }  // namespace pyro
 #endif
