@@ -549,8 +549,14 @@ __global__ __launch_bounds__(NT) void k_react(const Params *__restrict__ P, Geo 
       // the condensation gate is 0 or 1: most of a scene is cold air, and its
       // waves skip ten of the twenty divisions and two of the four
       // exponentials (254 -> 228 us at pool 2 cm).  Non-finite values take the
-      // full path.
-      const bool fin = (T - T) + (yf - yf) == 0.0f;
+      // full path, and so do a step without length and coefficients that make
+      // 0 / 0 or 0 inf of what is left out: finite, and positive where they
+      // divide (uniform: a compare each and a mask).
+      constexpr int POS = 0x180, POS0 = 0x1c0;  // finite > 0, >= +0
+      const bool plain = __builtin_amdgcn_classf(dt, POS) & __builtin_amdgcn_classf(P->tau_min, POS) &
+                         __builtin_amdgcn_classf(P->s_o2, POS) & __builtin_amdgcn_classf(P->dhc, POS0) &
+                         __builtin_amdgcn_classf(P->soot_form, POS0) & __builtin_amdgcn_classf(P->soot_ox, POS0);
+      const bool fin = plain && (T - T) + (yf - yf) == 0.0f;
       float rho, q = 0.0f;
       if (!(T <= P->t_ign - 100.0f && fin)) {
         rho = rhoOf(P, T);
@@ -588,7 +594,7 @@ __global__ __launch_bounds__(NT) void k_react(const Params *__restrict__ P, Geo 
       S += (q - prr) / (rho * cpOf(T) * T);
       float sp = fmax_(spongeSideR(P, g, x, z), spongeTopR(P, g, y));
       // no sponge: dec = 1 - exp(-0) = 0 changes nothing (a finite T and yo)
-      if (!(sp == 0.0f && (T - T) + (yo - yo) == 0.0f)) {
+      if (!(plain && sp == 0.0f && (T - T) + (yo - yo) == 0.0f)) {
         float dec = 1.0f - pexp(-dt * 4.0f * sp);
         T = mixf_(T, P->t0, dec);
         yf *= 1.0f - dec;
