@@ -2275,7 +2275,11 @@ static void launch_mg_tail(const MgLevel *lv, int t, int nl, int iters, float om
 void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
   LvArgs a = lv_args(L);
   const int ncol = L.d[0] * L.d[1];
-  const bool colz = L.wdir == 1.0f && ncol <= CO_NT;
+  // the column solve takes integer counts, a thread a column and 22 slots
+  const bool colz = L.wdir == 1.0f && ncol <= CO_NT && L.d[2] + 1 <= 22;
+  // Eight pairs a thread lose to the column solve where there is one, and win
+  // over sweep launches where the columns are too long for it: 48x8x24 224 us
+  // in sweeps, 175 in the tail; 72x8x24 231, 207; 22x22x22 254, 198.
   if (tail_fits(&L, 0, 1) && (!colz || tail_k(L) < 8)) {
     launch_mg_tail(&L, 0, 1, iters, omega, s);
     return;
@@ -2287,7 +2291,7 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
     k_mg_coarse_z<12><<<1, colt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
     return;
   }
-  if (colz && L.d[2] + 1 <= 22) {
+  if (colz) {
     // waves run on SIMD w % 4.  Per iteration (both colours) a SIMD issues
     // ZJ slots for each of its column waves plus two for each of its waves
     // holding extra cells: take the extra-cell layout when its busiest SIMD
