@@ -1436,8 +1436,9 @@ static void launch_mg_sweep2(const MgLevel &L, const MgLevel *C, const float *pi
 
 // ---------------------------------------------------------------- coarse
 // All red-black SOR iterations of the coarsest level (sim.rs:472-473: 80
-// iterations, omega = 1.6): in the tail's workgroup up to about 12 k cells, in
-// one workgroup with a thread per column (below), or else as sweep launches.
+// iterations, omega = 1.6): in the tail's workgroup (up to 16 k cells, by
+// their shape), in one workgroup with a thread per column (below), or else as
+// sweep launches (launch_mg_coarse has the rule).
 constexpr int CO_NT = 1024;
 constexpr int CO_PAD_MAX = 36000;  // floats of the column solve's LDS (144 KB)
 
@@ -1822,12 +1823,13 @@ __device__ __forceinline__ void tail_own(const TailLv &L, TAIL_SH, TailOwn<K> &W
   }
 }
 
-// Two red-black sweeps (omega 1) over the owned pairs.
+// Red-black sweeps over the owned pairs.
 template <int K, bool ICNT>
-__device__ __forceinline__ void tail_sweeps(const TailLv &L, TAIL_SH, int k, const TailOwn<K> &W) {
+__device__ __forceinline__ void tail_sweeps(const TailLv &L, TAIL_SH, int k, const TailOwn<K> &W, int sweeps,
+                                            float omega) {
   const float2 *ct = ctab + 64 * k;
   const int py = L.py, pz = L.pz;
-  for (int s = 0; s < 2; s++) {
+  for (int s = 0; s < sweeps; s++) {
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       float *A = sp + c * TL_CS;
@@ -1875,7 +1877,7 @@ __device__ __forceinline__ void tail_sweeps(const TailLv &L, TAIL_SH, int k, con
         }
 #pragma unroll
         for (int q = 0; q < KC; q++) {
-          const float nv = mixf_(cen[q], qs[q], 1.0f);
+          const float nv = mixf_(cen[q], qs[q], omega);
           if (!((W.cd[j0 + q] >> (8 * c)) & (uint32_t)(NC_SOLID | NC_NONE))) A[W.li[j0 + q]] = nv;
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -2144,11 +2146,11 @@ __global__ __launch_bounds__(TL_NT) void k_mg_tail(TailArgs) {
   }
   auto smooth = [&](int l) __attribute__((always_inline)) {
     if (l == 0) {
-      tail_sweeps<KT, ICNT>(a.l[0], sp, bl, cl, ct, 0, W);
+      tail_sweeps<KT, ICNT>(a.l[0], sp, bl, cl, ct, 0, W, 2, 1.0f);
     } else {
       TailOwn<2> I;
       tail_own<2, true>(a.l[l], sp, bl, cl, ct, I);
-      tail_sweeps<2, ICNT>(a.l[l], sp, bl, cl, ct, l, I);
+      tail_sweeps<2, ICNT>(a.l[l], sp, bl, cl, ct, l, I, 2, 1.0f);
     }
   };
   for (int l = 0; l < a.nl - 1; l++) {
@@ -2156,7 +2158,8 @@ __global__ __launch_bounds__(TL_NT) void k_mg_tail(TailArgs) {
     if (l == 0) tail_restrict<false>(a.l[0], a.l[1], sp, bl, cl, ct);
     else tail_restrict<true>(a.l[l], a.l[l + 1], sp, bl, cl, ct);
   }
-  if (a.nl == 1) tail_sor<KC, ICNT, false>(a.l[0], sp, bl, cl, ct, 0, a.iters, a.omega);
+  if constexpr (KC == 0) tail_sweeps<KT, ICNT>(a.l[0], sp, bl, cl, ct, 0, W, a.iters, a.omega);
+  else if (a.nl == 1) tail_sor<KC, ICNT, false>(a.l[0], sp, bl, cl, ct, 0, a.iters, a.omega);
   else tail_sor<KC, ICNT, true>(a.l[a.nl - 1], sp, bl, cl, ct, a.nl - 1, a.iters, a.omega);
   for (int l = a.nl - 2; l >= 0; l--) {
     tail_prolong(a.l[l + 1], a.l[l], sp, bl, cl, ct, (solid >> (l + 1)) & 1u);
@@ -2185,7 +2188,8 @@ __global__ __launch_bounds__(TL_NT) void k_mg_tail(TailArgs) {
 // Pairs per thread of the coarsest solve: the fewest with which the level's
 // columns, cut into z segments, fit the workgroup (0: none do).  Fewer pairs
 // on more lanes shorten the pass: 0.17 us at K = 1 (8x12x8), 0.35 at 2
-// (12x20x12), 0.6 at 4 (14x30x14).
+// (12x20x12), 0.6 at 4 (14x30x14).  A coarsest level alone takes its sweeps
+// over the owned pairs instead where no segments fit (KC = 0 of k_mg_tail).
 static int tail_k(const MgLevel &L) {
   const int cols = ((L.d[0] + 1) / 2) * L.d[1];
   for (int k : {1, 2, 4, 8})
@@ -2202,7 +2206,7 @@ static int tail_floats(const MgLevel &L) {  // LDS words of one colour's pairs w
 // per thread) the tail took 94 us against 39 us and six launches of 4.7 us.
 static bool tail_fits(const MgLevel *lv, int t, int nl) {
   int64_t words = 0, inner = 0;
-  if (nl - t > TL_MAX || !tail_k(lv[nl - 1])) return false;
+  if (nl - t > TL_MAX || (t < nl - 1 && !tail_k(lv[nl - 1]))) return false;
   for (int l = t; l < nl; l++) {
     const MgLevel &L = lv[l];
     if (L.n > 2u * TL_NT * TL_K) return false;
@@ -2257,6 +2261,11 @@ static void launch_mg_tail(const MgLevel *lv, int t, int nl, int iters, float om
   const int kc = tail_k(lv[nl - 1]);
   const int kt = a.l[0].np <= 2 * TL_NT ? 2 : a.l[0].np <= 4 * TL_NT ? 4 : TL_K;
   switch (kc) {
+    case 0:
+      if (kt == 2) launch_tail<2, 0>(a, icnt, s);
+      else if (kt == 4) launch_tail<TL_TOP, 0>(a, icnt, s);
+      else launch_tail<TL_K, 0>(a, icnt, s);
+      break;
     case 1:
       if (kt == 2) launch_tail<2, 1>(a, icnt, s);
       else launch_tail<TL_TOP, 1>(a, icnt, s);
@@ -2279,8 +2288,15 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
   const bool colz = L.wdir == 1.0f && ncol <= CO_NT && L.d[2] + 1 <= 22;
   // Eight pairs a thread lose to the column solve where there is one, and win
   // over sweep launches where the columns are too long for it: 48x8x24 224 us
-  // in sweeps, 175 in the tail; 72x8x24 231, 207; 22x22x22 254, 198.
-  if (tail_fits(&L, 0, 1) && (!colz || tail_k(L) < 8)) {
+  // in sweeps, 175 in the tail; 72x8x24 231, 207; 22x22x22 254, 198.  Too many
+  // columns for the tail's solve (thin, wide levels) run its sweeps on the
+  // owned pairs, which cost a pass per 2048 pairs: four V-cycles on 1100x2x2
+  // 1118 us in sweep launches, 670 so; 200x12x3 1134, 743; 250x9x5 (5625
+  // pairs) 1212, 1017; 120x18x6 (6480) 1144, 1287.  Rows below four cells have
+  // only the single sweeps beside it: 3x700x2 2564, 840.
+  const int tk = tail_k(L), np = ((L.d[0] + 1) / 2) * L.d[1] * L.d[2];
+  const bool tail = tk ? !colz || tk < 8 : !colz && (np <= 6 * TL_NT || !sweep2_fits(L));
+  if (tail && tail_fits(&L, 0, 1)) {
     launch_mg_tail(&L, 0, 1, iters, omega, s);
     return;
   }
