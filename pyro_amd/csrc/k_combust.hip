@@ -353,15 +353,29 @@ __global__ __launch_bounds__(NT) void k_solid(const Params *__restrict__ P, Geo 
 
 // The step's solid and curl stages in one launch: curl reads only the velocity
 // and writes only curl, which solid neither reads nor writes.  The first ns
-// blocks take the solid tiles, tile j, j + ns, ... each, and the rest the
-// curl, so the few tiles with ray marches, which lie together in the grid,
-// start first, on different CUs and XCDs, and the dense, memory-bound curl
-// fills the CUs meanwhile.  Eight tiles' flags are loaded at once: nearly all
-// tiles are empty.  (One block for both stages of a tile left the ray marches
-// to the XCD whose part of the grid holds them, at the end of its part:
-// 160x240x160 88 us, 50 now; 160x320x160 79, 56; 320x480x320 720, 541.  512
-// or 2048 blocks, 16 tiles at once or fewer registers are slower.)
-constexpr int SOLID_BLOCKS = 1024, SOLID_BATCH = 8;
+// blocks take the solid tiles, positions j, j + ns, ... of solid_order each,
+// and the rest the curl, so the tiles with ray marches start first and the
+// dense, memory-bound curl fills the CUs meanwhile.  Eight tiles' flags are
+// loaded at once: nearly all tiles are empty.
+//
+// Two kinds of scene set the order and the number of blocks.  Fuel in one
+// place (us at 160x240x160, 160x320x160, 320x480x320): with one block for both
+// stages of a tile its ray marches all went to the XCD whose part of the grid
+// holds them, 98, 76 and 798; here 50, 53 and 560.  Solids all over (posts at
+// 144^3 and 176^3, blocks at 128^3): 131, 251 and 91 with one block a tile;
+// 164, 273 and 141 with the tiles dealt out singly to 1024 blocks, where the
+// marches of neighbouring tiles no longer share an XCD's cache and a block's
+// tiles at 128^3 are whole planes apart, all of them solid or all empty; 122,
+// 238 and 91 here.  Fewer blocks are faster by up to 5 % with fuel in one
+// place (1024: 530 at 320x480x320, 15.6 instead of 17.4 at 80x160x80) and up to
+// a half slower with solids all over; runs of 4 and 64 tiles lose in both.  The
+// number is no power of two, as the planes often are.
+constexpr int SOLID_RUN = 16, SOLID_GROUP = 8 * SOLID_RUN, SOLID_BLOCKS = 35 * SOLID_GROUP, SOLID_BATCH = 8;
+// Tile at position k < nt: runs of consecutive tiles, each on one XCD (k % 8).
+__device__ __forceinline__ int solid_order(int k, int nt) {
+  const int r = k % SOLID_GROUP, g = k - r;
+  return g + SOLID_GROUP > nt ? k : g + (r & 7) * SOLID_RUN + (r >> 3);
+}
 template <bool STATS>
 __global__ __launch_bounds__(NT) void k_solid_curl(const Params *__restrict__ P, Geo g, int ns,
                                                     const float4 *__restrict__ solIn, float4 *__restrict__ solOut,
@@ -385,21 +399,23 @@ __global__ __launch_bounds__(NT) void k_solid_curl(const Params *__restrict__ P,
   }
   __shared__ SolidLds L;
   solid_kinds(P, L);
-  for (int t0 = (int)blockIdx.x; t0 < nt; t0 += SOLID_BATCH * ns) {
+  for (int k0 = (int)blockIdx.x; k0 < nt; k0 += SOLID_BATCH * ns) {
     uint8_t f[SOLID_BATCH];
     bool any = STATS;
 #pragma unroll
     for (int u = 0; u < SOLID_BATCH; u++) {
-      const uint32_t t = (uint32_t)t0 + (uint32_t)(ns * u), i = t * NT + threadIdx.x;
-      f[u] = (int)t < nt && i < g.n ? flags[i] : 0;
+      const int k = k0 + ns * u;
+      const uint32_t i = (uint32_t)solid_order(k, nt) * NT + threadIdx.x;
+      f[u] = k < nt && i < g.n ? flags[i] : 0;
     }
 #pragma unroll
     for (int u = 0; u < SOLID_BATCH; u++) any |= f[u] != 0;
     if (!__syncthreads_or(any)) continue;
 #pragma unroll 1
     for (int u = 0; u < SOLID_BATCH; u++) {
-      const int t = t0 + ns * u;
-      if (t >= nt) break;
+      const int k = k0 + ns * u;
+      if (k >= nt) break;
+      const int t = solid_order(k, nt);
       solid_tile<STATS>(P, g, L, solIn, solOut, pyr, flags, s0, part, (uint32_t)t * NT, (uint32_t)xcd_block(t, nt), f[0]);
 #pragma unroll
       for (int v = 0; v + 1 < SOLID_BATCH; v++) f[v] = f[v + 1];  // f[0]: the next tile's
