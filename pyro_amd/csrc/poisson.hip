@@ -100,8 +100,10 @@ int sync(PyroPoisson *P) {
 }
 // r.r of the iteration just enqueued, read by the host.  While it waits, the
 // card goes on with the next V-cycle's first sweeps (head), whose right-hand
-// side is there already; if the iteration was the last one they are not used.
-// Waiting with nothing enqueued left the card idle for some 20 us an iteration.
+// side is there already.  With nothing enqueued the card is idle for some 20 us
+// an iteration; after the last iteration the sweeps are of no use, two launches
+// of 28 us each at 8 M cells and 207 at 49 M.  So the head is left out where
+// the iteration under way is expected to be the last (ResidWatch).
 int read_rr(PyroPoisson *P, bool head, double *rr) {
   PCHK(hipMemcpyAsync(P->rr_host, P->dev + 2, sizeof(double), hipMemcpyDeviceToHost, P->stream));
   PCHK(hipEventRecord(P->ev_rr, P->stream));
@@ -511,14 +513,16 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     if (!rc) watch(0);
     MgLevel &L0 = P->pc[0];
     if (!rc && !diverged && rel > tol) launch_to_f32(n, P->r, L0.b, P->stream);
+    bool head = false;
     while (!rc && !diverged && rel > tol && it < max_iters) {
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, it ? VPart::Rest : VPart::All);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, head ? VPart::Rest : VPart::All);
       launch_add_f32_to_f64(n, L0.phi, P->x, P->stream);
       cycles++;
       it++;
       launch_resid_rr(L0, P->x, P->b, L0.b, P->cgpart, P->dev, P->stream);
       double rr = 0.0;
-      rc = read_rr(P, true, &rr);
+      head = it < max_iters && rw.expects_more(tol);
+      rc = read_rr(P, head, &rr);
       if (rc) break;
       rel = std::sqrt(rr / bb);
       if (watch(it)) break;
@@ -533,9 +537,10 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     bool use_net = method == PYRO_SOLVER_LEARNED;
     MgLevel &L0 = P->pc[0];
     // z = M(r): in L0.phi (z64 null), or in P->z where the network had a part
-    // in it; L0.b holds (float)r when b32_ready.  dev[3] = z.q with_dot.
+    // in it; L0.b holds (float)r when b32_ready, and the V-cycle's head is
+    // under way with it when head (read_rr).  dev[3] = z.q with_dot.
     const double *z64 = nullptr;
-    auto apply_m = [&](double rr_now, bool with_dot, bool b32_ready) -> int {
+    auto apply_m = [&](double rr_now, bool with_dot, bool b32_ready, bool head) -> int {
       z64 = nullptr;
       if (use_net) {
         bool ok = false;
@@ -554,9 +559,8 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         fallbacks++;
         b32_ready = false;
       }
-      // b32_ready: the V-cycle's head is under way (read_rr)
       if (!b32_ready) launch_to_f32(n, P->r, L0.b, P->stream);
-      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, b32_ready ? VPart::Rest : VPart::All);
+      enqueue_vcycle(P->pc, P->nl_pc, P->coarse_iters_pc, P->stream, true, head ? VPart::Rest : VPart::All);
       if (with_dot) launch_dot_zq(n, L0.phi, P->q, P->cgpart, P->dev, P->stream);
       return 0;
     };
@@ -566,7 +570,7 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
     if (bb <= 0.0) bb = 1.0;
     if (!rc) watch(0);
     if (!rc && !diverged && rel > tol) {
-      rc = apply_m(rel * rel * bb, false, false);
+      rc = apply_m(rel * rel * bb, false, false, false);
       cycles++;
       if (!rc && z64) PCHK(hipMemcpyAsync(P->p, z64, n * sizeof(double), hipMemcpyDeviceToDevice, P->stream));
       if (!rc && !z64) launch_to_f64(n, L0.phi, P->p, P->stream);
@@ -577,11 +581,12 @@ int pyro_poisson_solve(PyroPoisson *P, int method, double tol, int max_iters, Py
         pending = true;
         it++;
         double rr = 0.0;
-        rc = read_rr(P, !use_net, &rr);
+        const bool head = !use_net && it < max_iters && rw.expects_more(tol);
+        rc = read_rr(P, head, &rr);
         if (rc) break;
         rel = std::sqrt(rr / bb);
         if (watch(it) || rel <= tol) break;
-        rc = apply_m(rr, true, !use_net);  // z, dev[3] z.q
+        rc = apply_m(rr, true, !use_net, head);  // z, dev[3] z.q
         if (rc) break;
         cycles++;
         launch_step_p(n, P->dev, L0.phi, z64, P->p, P->x, P->stream);
