@@ -401,7 +401,6 @@ void launch_mg_prolong(const MgLevel &C, const MgLevel &F, hipStream_t s) {
 // a launch a level and kind took 4 to 5 us each, seven of them in every step.
 // The levels' blocks follow one another; the table is indexed where it lies,
 // in the kernel arguments (a copy would be indexed in scratch memory).
-constexpr int SU_MAX = 12;
 typedef const __attribute__((address_space(1))) uint8_t *gcu8;
 typedef __attribute__((address_space(1))) uint8_t *gu8;
 struct SetupLevel {
@@ -412,7 +411,7 @@ struct SetupLevel {
 };
 struct SetupArgs {
   int nl, first;  // levels, first level written (coarse flags)
-  SetupLevel l[SU_MAX];
+  SetupLevel l[MG_MAX];
 };
 
 // The codes of a cell, or of four cells along x at once.

@@ -101,10 +101,10 @@ __global__ __launch_bounds__(256) void k_pack_conv(PackArgs) {
   if (e >= p.total) return;
   p.wp[e] = packed_weight((const float *)p.W, p.cout, p.cin, p.ca_e, p.cb_e, p.cout_e, p.transposed != 0, e);
 }
-void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s) {
+void launch_pack_jobs(const PackJob *jobs, int n, hipStream_t s) {
   PackArgs a;
   uint32_t blocks = 0;
-  a.n = n < PACK_MAX ? n : PACK_MAX;
+  a.n = n;
   for (int k = 0; k < a.n; k++) {
     const ConvSpec &c = jobs[k].c;
     PackEntry &p = a.e[k];
@@ -123,8 +123,8 @@ void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s) {
   k_pack_conv<<<blocks, 256, 0, s>>>(a);
 }
 void launch_pack_conv(const float *W, const ConvSpec &c, bool transposed, bf16 *wp, hipStream_t s) {
-  const PackJob j{W, wp, c, transposed};
-  launch_pack_convs(&j, 1, s);
+  const PackJob j[1] = {{W, wp, c, transposed}};
+  launch_pack_convs(j, s);
 }
 __global__ __launch_bounds__(256) void k_pack_bf16(const float *__restrict__ w, uint32_t n, bf16 *__restrict__ o) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;

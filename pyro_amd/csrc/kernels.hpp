@@ -64,6 +64,7 @@ void launch_velocity_noise(const Fields &f, float amp, uint32_t seed, hipStream_
 void launch_set_step(Params *P, float dt, float time, float ign_on, uint32_t frame, hipStream_t s);
 
 // Multigrid on one level hierarchy (mg.wgsl).
+constexpr int MG_MAX = 12;  // levels of any hierarchy; 2^31 cells halve to 512 in eight
 struct MgLevel {
   int d[3];
   float h, hh;   // spacing and h*h (f32)
@@ -80,7 +81,7 @@ struct MgLevel {
   uint32_t n;
 };
 // Coarse flags and neighbour codes of every level (once per step).
-void launch_mg_setup(const MgLevel *L, int nl, hipStream_t s);
+void launch_mg_setup(const MgLevel *L, int nl, hipStream_t s);  // nl <= MG_MAX
 // One red-black sweep (colour 0 then 1) reading phi from pin, writing pout.
 void launch_mg_sweep(const MgLevel &L, const float *pin, float *pout, float omega, hipStream_t s, bool fine);
 void launch_mg_restrict(const MgLevel &F, const MgLevel &C, hipStream_t s);

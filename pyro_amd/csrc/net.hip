@@ -153,12 +153,11 @@ int work_alloc(Work &W, const G3 &g, bool train) {
 void repack(PyroNet *N) {
   launch_pack_conv_in(N->params + N->w0a, N->w0a_bf, N->stream);
   PackJob jobs[2 * NCONV];
-  static_assert(2 * NCONV <= PACK_MAX, "one launch packs every conv");
   for (int l = 0; l < NCONV; l++) {
     jobs[2 * l] = {N->params + N->w[l], N->wp[l], kSpec[l], false};
     jobs[2 * l + 1] = {N->params + N->w[l], N->wpt[l], kSpec[l], true};
   }
-  launch_pack_convs(jobs, 2 * NCONV, N->stream);
+  launch_pack_convs(jobs, N->stream);
 }
 
 void forward(PyroNet *N, Work &W, const bf16 *x0) {
@@ -184,6 +183,7 @@ void backward(PyroNet *N, Work &W, const bf16 *x0) {
   float *G = N->grads;
   const G3 &g0 = W.g0, &g1 = W.g1, &g2 = W.g2;
   DwSums D;
+  static_assert(NCONV + 1 <= DW_SUMS, "an entry a layer");
   float *part = W.part + HEAD_PART;
   // the weight gradient's partials of a layer, summed at the end
   auto conv_dw = [&](const G3 &g, int l, const bf16 *a, const G3 &ga, const bf16 *b, const bf16 *gpre) {

@@ -57,7 +57,12 @@ struct PackJob {
   ConvSpec c;
   bool transposed;
 };
-void launch_pack_convs(const PackJob *jobs, int n, hipStream_t s);
+void launch_pack_jobs(const PackJob *jobs, int n, hipStream_t s);
+template <int N>
+void launch_pack_convs(const PackJob (&jobs)[N], hipStream_t s) {
+  static_assert(N <= PACK_MAX, "more copies than a launch's table holds");
+  launch_pack_jobs(jobs, N, s);
+}
 void launch_pack_bf16(const float *w, uint32_t n, bf16 *out, hipStream_t s);
 
 // out[v][0..cout) = act(bias + sum_taps W * in), in = [up(a), b]; false (and

@@ -46,7 +46,7 @@ struct PyroPoisson {
   int d[3] = {0, 0, 0};
   float h = 0.0f;
   uint32_t n = 0;
-  MgLevel pc[12];
+  MgLevel pc[MG_MAX];
   int nl_pc = 0;
   MgLevel ref[4];
   int nl_ref = 0;
@@ -354,7 +354,7 @@ int pyro_poisson_create(uint32_t nx, uint32_t ny, uint32_t nz, float h, const ui
   float hl = h;
   int rc = 0;
   bool ref_open = true;
-  for (int l = 0; l < 12 && !rc; l++) {
+  for (int l = 0; l < MG_MAX && !rc; l++) {
     MgLevel &L = P->pc[P->nl_pc++];
     L.d[0] = d[0]; L.d[1] = d[1]; L.d[2] = d[2];
     L.h = hl;

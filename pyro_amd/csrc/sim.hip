@@ -34,6 +34,7 @@ int fail(int code, const std::string &m) {
   } while (0)
 
 constexpr int MG_LEVELS = 4;     // sim.rs:13
+static_assert(MG_LEVELS <= MG_MAX);
 constexpr int COARSE_ITERS = 80;  // sim.rs:14
 }  // namespace
 
