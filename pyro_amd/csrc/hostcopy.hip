@@ -15,10 +15,14 @@
 namespace pyro {
 namespace {
 
-// Four threads with two 4 MiB slots each: a copy of 134 MB in and back took
-// 9.9 + 13.4 ms through the runtime and 5.9 + 3.7 ms this way (three arrays of
-// 256^3 doubles), 6.9 + 4.7 with eight 2 MiB pairs and 12.4 + 6.4 with 512 KiB
-// ones (each chunk costs the link about 20 us); eight 4 MiB pairs gain nothing.
+// Four threads with two 4 MiB slots each.  Two arrays of 256^3 doubles in (268
+// MB) and one back (134 MB) took 9.9 + 13.4 ms through the runtime and 5.9 + 3.7
+// ms this way, 6.9 + 4.7 with eight 2 MiB pairs and 12.4 + 6.4 with 512 KiB ones
+// (each chunk costs the link about 20 us); eight 4 MiB pairs gain nothing.
+// Making the pool and giving it back costs about 0.4 ms, so a handle that is
+// made, solves once and is closed breaks even at 9 MB an array (104^3: its
+// copies and its closing 3.00 ms before, 3.05 now) and gains from there (128^3
+// 4.7, 4.2; 160^3 8.2, 6.4).
 constexpr unsigned THREADS = 4;      // workers, the calling thread among them
 constexpr size_t CHUNK = 4u << 20;   // bytes of a slot; two slots a worker
 constexpr size_t SMALL = 8u << 20;   // below this the runtime's copy is as fast

@@ -9,7 +9,8 @@
 // The reference dispatches the coarsest level's 80 red-black SOR iterations
 // as 160 separate passes; here they run in one workgroup with phi, b and the
 // solid mask on chip (160 KB of LDS per CU on gfx950), one barrier per colour
-// pass, or, where a level is too large for that, as 40 launches.
+// pass, or, where a level is too large for that, as sweep launches: 40 of two
+// sweeps each, or 80 single ones where two do not pay (sweep2_fits).
 #include "kernels.hpp"
 
 namespace pyro {
@@ -858,7 +859,7 @@ __global__ __launch_bounds__(SW_NT) void k_mg_sweep(LvArgs a, int ntx, int nty, 
 // colour-0 neighbours by then; colour-1 values go straight to pout with their
 // pair's colour-0 cell, since no other cell reads them in this sweep.  The
 // next four planes are in registers meanwhile, loaded a whole step ahead.
-// Against a tile at a time: 1.9 loads and 1.2 updates a cell instead of 3.75
+// Against a tile at a time: 2.1 loads and 1.2 updates a cell instead of 3.75
 // and 1.5, and the loads overlap the updates; 563 MB read from beyond the L2
 // instead of 788 at 320x480x320 (443 are compulsory), and 41 M VALU
 // instructions instead of 70.  Loads two steps ahead (95 registers) gave
@@ -1401,10 +1402,10 @@ __global__ __launch_bounds__(S2_NT) void k_mg_sweep2(LvArgs a, int ntx, int nty,
 // Rows that are no multiple of four cells take k_mg_sweep one element at a
 // time, and there the line lies higher: a solve at 97x61x118 5594 us before,
 // 4101 now; 129^3 (2.1 M) 9721 without, 9325 with; 193x121x235 (5.5 M) 17.45
-// ms, 17.38; 255^3 30.8, 31.9.
+// ms, 17.38 (no more than two runs differ); 255^3 30.8, 31.9.
 constexpr uint32_t S2_MAX = 900000u, S2_MAX_ODD = 4000000u;
 // The prolongation joins them up to here: every cell of the rings is prolonged
-// too (3.75 times the tile).  A solve at 97x61x118 (its 698 k cells) 3.93 ms
+// too (6 times the tile).  A solve at 97x61x118 (its 698 k cells) 3.93 ms
 // with it in the launch, 3.78 without; 129^3 9.07 and 8.44; 96^3 2.84 and
 // 2.77; with a line of 50 k instead, four V-cycles at 80x160x80 (128 k) 465 us
 // against 458.
@@ -1470,7 +1471,6 @@ constexpr int CZ_ZERO = CO_NT, CZ_PLANE = CO_NT + 64, CZ_EX_NT = 768;
 
 template <int ZJ, bool EX = false>
 __global__ __launch_bounds__(EX ? CZ_EX_NT : CO_NT) void k_mg_coarse_z(LvArgs a, const float *__restrict__ b,
-                                                                        const uint8_t *__restrict__ f,
                                                                         const uint8_t *__restrict__ nc,
                                                                         float *__restrict__ p, int iters,
                                                                         float omega) {
@@ -2303,7 +2303,7 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
   // still run every colour pass's arithmetic on the CU
   const int colt = ((ncol + 63) / 64) * 64;
   if (colz && L.d[2] + 1 <= 12) {
-    k_mg_coarse_z<12><<<1, colt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
+    k_mg_coarse_z<12><<<1, colt, 0, s>>>(a, L.b, L.nc, L.phi, iters, omega);
     return;
   }
   if (colz) {
@@ -2324,14 +2324,14 @@ void launch_mg_coarse(const MgLevel &L, int iters, float omega, hipStream_t s) {
     const bool ex = full >= 64 && full <= CZ_EX_NT && ncol > full && (ncol - full) * zh <= full && load_ex < load_col;
     if (zj == 21) {
       if (ex)
-        k_mg_coarse_z<21, true><<<1, full, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
+        k_mg_coarse_z<21, true><<<1, full, 0, s>>>(a, L.b, L.nc, L.phi, iters, omega);
       else
-        k_mg_coarse_z<21><<<1, colt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
+        k_mg_coarse_z<21><<<1, colt, 0, s>>>(a, L.b, L.nc, L.phi, iters, omega);
     } else {
       if (ex)
-        k_mg_coarse_z<22, true><<<1, full, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
+        k_mg_coarse_z<22, true><<<1, full, 0, s>>>(a, L.b, L.nc, L.phi, iters, omega);
       else
-        k_mg_coarse_z<22><<<1, colt, 0, s>>>(a, L.b, L.f, L.nc, L.phi, iters, omega);
+        k_mg_coarse_z<22><<<1, colt, 0, s>>>(a, L.b, L.nc, L.phi, iters, omega);
     }
     return;
   }
