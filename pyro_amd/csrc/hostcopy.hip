@@ -61,8 +61,13 @@ class Pool {
     if (slots_) (void)hipHostFree(slots_);
   }
   hipError_t run(char *dst, const char *src, size_t bytes, hipStream_t s, bool in) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
+    // the slots' events are of the stream's device, which the caller need not
+    // have made current
+    int cur = 0;
+    hipDevice_t dev = 0;
+    hipError_t e = hipStreamGetDevice(s, &dev);
+    if (e == hipSuccess) e = hipGetDevice(&cur);
+    if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
     if (e != hipSuccess) return e;
     {
       std::lock_guard<std::mutex> l(m_);
@@ -75,6 +80,7 @@ class Pool {
     work(0);
     std::unique_lock<std::mutex> l(m_);
     done_.wait(l, [&] { return left_ == 0; });
+    if (cur != dev) note_locked(hipSetDevice(cur));
     return err_;
   }
 
@@ -107,10 +113,13 @@ class Pool {
       if (--left_ == 0) done_.notify_one();
     }
   }
+  void note_locked(hipError_t e) {
+    if (err_ == hipSuccess) err_ = e;
+  }
   void note(hipError_t e) {
     if (e == hipSuccess) return;
     std::lock_guard<std::mutex> l(m_);
-    if (err_ == hipSuccess) err_ = e;
+    note_locked(e);
   }
   // waits until slot j is free, and has an event of the job's device for it
   hipError_t ready(unsigned j, int dev) {
