@@ -78,13 +78,15 @@ struct PyroNet {
 };
 
 namespace {
+// Zeroed on the stream whose kernels use it first: hipMemset runs on the null
+// stream and returns before it is done, and the streams here do not wait for it.
 template <class T>
-int dalloc(std::vector<void *> &list, T **p, size_t count) {
+int dalloc(std::vector<void *> &list, T **p, size_t count, hipStream_t s) {
   void *v = nullptr;
   const size_t bytes = count * sizeof(T) < 256 ? 256 : count * sizeof(T);
   if (hipMalloc(&v, bytes) != hipSuccess) return nfail(PYRO_E_OOM, "hipMalloc failed");
   list.push_back(v);
-  if (hipMemset(v, 0, bytes) != hipSuccess) return nfail(PYRO_E_HIP, "hipMemset failed");
+  if (hipMemsetAsync(v, 0, bytes, s) != hipSuccess) return nfail(PYRO_E_HIP, "hipMemsetAsync failed");
   *p = static_cast<T *>(v);
   return 0;
 }
@@ -93,7 +95,7 @@ void free_list(std::vector<void *> &list) {
   list.clear();
 }
 
-int work_alloc(Work &W, const G3 &g, bool train) {
+int work_alloc(Work &W, const G3 &g, bool train, hipStream_t s) {
   if (!W.allocs.empty() && W.g0 == g && (W.train || !train)) return 0;
   free_list(W.allocs);
   W.g0 = g;
@@ -103,32 +105,32 @@ int work_alloc(Work &W, const G3 &g, bool train) {
   const size_t n0 = g.n(), n1 = W.g1.n(), n2 = W.g2.n();
   auto &L = W.allocs;
   int rc = 0;
-  rc |= dalloc(L, &W.x0, n0 * 2);
-  if (!rc) rc |= dalloc(L, &W.a0, n0 * 16);
-  if (!rc) rc |= dalloc(L, &W.s0, n0 * 16);
-  if (!rc) rc |= dalloc(L, &W.p1, n1 * 16);
-  if (!rc) rc |= dalloc(L, &W.a1, n1 * 32);
-  if (!rc) rc |= dalloc(L, &W.s1, n1 * 32);
-  if (!rc) rc |= dalloc(L, &W.p2, n2 * 32);
-  if (!rc) rc |= dalloc(L, &W.a2, n2 * 64);
-  if (!rc) rc |= dalloc(L, &W.c2, n2 * 64);
-  if (!rc) rc |= dalloc(L, &W.d1, n1 * 32);
-  if (!rc) rc |= dalloc(L, &W.d0, n0 * 16);
-  if (!rc) rc |= dalloc(L, &W.y, n0);
+  rc |= dalloc(L, &W.x0, n0 * 2, s);
+  if (!rc) rc |= dalloc(L, &W.a0, n0 * 16, s);
+  if (!rc) rc |= dalloc(L, &W.s0, n0 * 16, s);
+  if (!rc) rc |= dalloc(L, &W.p1, n1 * 16, s);
+  if (!rc) rc |= dalloc(L, &W.a1, n1 * 32, s);
+  if (!rc) rc |= dalloc(L, &W.s1, n1 * 32, s);
+  if (!rc) rc |= dalloc(L, &W.p2, n2 * 32, s);
+  if (!rc) rc |= dalloc(L, &W.a2, n2 * 64, s);
+  if (!rc) rc |= dalloc(L, &W.c2, n2 * 64, s);
+  if (!rc) rc |= dalloc(L, &W.d1, n1 * 32, s);
+  if (!rc) rc |= dalloc(L, &W.d0, n0 * 16, s);
+  if (!rc) rc |= dalloc(L, &W.y, n0, s);
   if (!rc && train) {
-    rc |= dalloc(L, &W.gy, n0);
-    if (!rc) rc |= dalloc(L, &W.gd0, n0 * 16);
-    if (!rc) rc |= dalloc(L, &W.gcat0, n0 * 48);
-    if (!rc) rc |= dalloc(L, &W.gd1, n1 * 32);
-    if (!rc) rc |= dalloc(L, &W.gcat1, n1 * 96);
-    if (!rc) rc |= dalloc(L, &W.gc2, n2 * 64);
-    if (!rc) rc |= dalloc(L, &W.ga2, n2 * 64);
-    if (!rc) rc |= dalloc(L, &W.gp2, n2 * 32);
-    if (!rc) rc |= dalloc(L, &W.gs1, n1 * 32);
-    if (!rc) rc |= dalloc(L, &W.ga1, n1 * 32);
-    if (!rc) rc |= dalloc(L, &W.gp1, n1 * 16);
-    if (!rc) rc |= dalloc(L, &W.gs0, n0 * 16);
-    if (!rc) rc |= dalloc(L, &W.ga0, n0 * 16);
+    rc |= dalloc(L, &W.gy, n0, s);
+    if (!rc) rc |= dalloc(L, &W.gd0, n0 * 16, s);
+    if (!rc) rc |= dalloc(L, &W.gcat0, n0 * 48, s);
+    if (!rc) rc |= dalloc(L, &W.gd1, n1 * 32, s);
+    if (!rc) rc |= dalloc(L, &W.gcat1, n1 * 96, s);
+    if (!rc) rc |= dalloc(L, &W.gc2, n2 * 64, s);
+    if (!rc) rc |= dalloc(L, &W.ga2, n2 * 64, s);
+    if (!rc) rc |= dalloc(L, &W.gp2, n2 * 32, s);
+    if (!rc) rc |= dalloc(L, &W.gs1, n1 * 32, s);
+    if (!rc) rc |= dalloc(L, &W.ga1, n1 * 32, s);
+    if (!rc) rc |= dalloc(L, &W.gp1, n1 * 16, s);
+    if (!rc) rc |= dalloc(L, &W.gs0, n0 * 16, s);
+    if (!rc) rc |= dalloc(L, &W.ga0, n0 * 16, s);
     // weight-gradient scratch: operands of the largest layer, partials of all
     const G3 lg[NCONV] = {W.g0, W.g1, W.g1, W.g2, W.g2, W.g1, W.g0};
     size_t xt = dw_xt_elems(W.g0, ConvSpec{0, 2, 16}), gt = dw_gt_elems(W.g0, ConvSpec{0, 2, 16});
@@ -138,10 +140,10 @@ int work_alloc(Work &W, const G3 &g, bool train) {
       gt = std::max(gt, dw_gt_elems(lg[l], kSpec[l]));
       part += dw_part_elems(lg[l], kSpec[l]);
     }
-    if (!rc) rc |= dalloc(L, &W.xt, xt);
-    if (!rc) rc |= dalloc(L, &W.gt, gt);
-    if (!rc) rc |= dalloc(L, &W.part, part);
-    if (!rc) rc |= dalloc(L, &W.lpart, 2 * LOSS_BLOCKS + 2);
+    if (!rc) rc |= dalloc(L, &W.xt, xt, s);
+    if (!rc) rc |= dalloc(L, &W.gt, gt, s);
+    if (!rc) rc |= dalloc(L, &W.part, part, s);
+    if (!rc) rc |= dalloc(L, &W.lpart, 2 * LOSS_BLOCKS + 2, s);
   }
   if (rc) {
     free_list(W.allocs);
@@ -250,7 +252,7 @@ const char *net_error() { return g_nerr.c_str(); }
 
 int net_apply64(PyroNet *N, const G3 &g, const double *r, const uint8_t *flags, double rr, double nfluid, double h,
                 double *z, hipStream_t s) {
-  int rc = work_alloc(N->inf, g, false);
+  int rc = work_alloc(N->inf, g, false, s);
   if (rc) return rc;
   const double rms = nfluid > 0.0 ? std::sqrt(rr / nfluid) : 0.0;
   if (!(rms > 0.0) || !std::isfinite(rms)) return nfail(PYRO_E_INVALID, "zero or non-finite residual");
@@ -281,8 +283,8 @@ int net_add_pair64(PyroNet *N, const G3 &g, const double *b, const double *phi, 
   }
   Sample S;
   std::vector<void *> &L = N->allocs;
-  int rc = dalloc(L, &S.x0, (size_t)g.n() * 2);
-  if (!rc) rc = dalloc(L, &S.t, (size_t)g.n());
+  int rc = dalloc(L, &S.x0, (size_t)g.n() * 2, s);
+  if (!rc) rc = dalloc(L, &S.t, (size_t)g.n(), s);
   if (rc) return rc;
   launch_net_input64(g, b, flags, 1.0 / rms, S.x0, s);
   launch_net_target64(g, phi, flags, 1.0 / (hh * rms * (double)N->out_scale), S.t, s);
@@ -325,19 +327,20 @@ int pyro_net_create(uint64_t seed, PyroNet **out) {
   N->bh = o; o += 1;
   N->np = o;
   int rc = 0;
-  rc |= dalloc(N->allocs, &N->params, o);
-  if (!rc) rc |= dalloc(N->allocs, &N->grads, o);
-  if (!rc) rc |= dalloc(N->allocs, &N->am, o);
-  if (!rc) rc |= dalloc(N->allocs, &N->av, o);
-  if (!rc) rc |= dalloc(N->allocs, &N->w0a_bf, 2 * 16 * 32);
+  rc |= dalloc(N->allocs, &N->params, o, N->stream);
+  if (!rc) rc |= dalloc(N->allocs, &N->grads, o, N->stream);
+  if (!rc) rc |= dalloc(N->allocs, &N->am, o, N->stream);
+  if (!rc) rc |= dalloc(N->allocs, &N->av, o, N->stream);
+  if (!rc) rc |= dalloc(N->allocs, &N->w0a_bf, 2 * 16 * 32, N->stream);
   for (int l = 0; l < NCONV && !rc; l++) {
     const ConvSpec &c = kSpec[l];
-    rc |= dalloc(N->allocs, &N->wp[l], (size_t)conv_groups(c.ca, c.cb, c.cout) * c.cout * 32);
-    if (!rc) rc |= dalloc(N->allocs, &N->wpt[l], (size_t)conv_groups(0, c.cout, c.cin()) * c.cin() * 32);
+    rc |= dalloc(N->allocs, &N->wp[l], (size_t)conv_groups(c.ca, c.cb, c.cout) * c.cout * 32, N->stream);
+    if (!rc) rc |= dalloc(N->allocs, &N->wpt[l], (size_t)conv_groups(0, c.cout, c.cin()) * c.cin() * 32, N->stream);
   }
-  if (!rc) rc |= dalloc(N->allocs, &N->dpart, DOT_PART);
-  if (!rc) rc |= dalloc(N->allocs, &N->dout, 4);
+  if (!rc) rc |= dalloc(N->allocs, &N->dpart, DOT_PART, N->stream);
+  if (!rc) rc |= dalloc(N->allocs, &N->dout, 4, N->stream);
   if (rc) return bail(rc);
+  if (nsync(N)) return bail(PYRO_E_HIP);  // zeroed before the upload below, which is not on this stream
   // He-normal weights (std sqrt(2 / fan_in)), zero biases, small head
   std::vector<float> h(o, 0.0f);
   Rng R{seed};
@@ -410,7 +413,7 @@ int pyro_net_forward(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, const fl
   int rc = check_dims(nx, ny, nz);
   if (rc) return rc;
   const G3 g{(int)nx, (int)ny, (int)nz};
-  rc = work_alloc(N->inf, g, false);
+  rc = work_alloc(N->inf, g, false, N->stream);
   if (rc) return rc;
   float *tmp = N->inf.y;  // host x0 staged through y (n floats) twice
   const size_t n = g.n();
@@ -428,7 +431,7 @@ int pyro_net_backward(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, const f
   int rc = check_dims(nx, ny, nz);
   if (rc) return rc;
   const G3 g{(int)nx, (int)ny, (int)nz};
-  rc = work_alloc(N->tr, g, true);
+  rc = work_alloc(N->tr, g, true, N->stream);
   if (rc) return rc;
   const size_t n = g.n();
   for (int half = 0; half < 2; half++) {
@@ -473,8 +476,8 @@ int pyro_net_dataset_add(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, cons
   if (!N->data.empty() && !(N->data_g == g)) return nfail(PYRO_E_INVALID, "training pairs must share one grid");
   const size_t n = g.n();
   Sample S;
-  rc = dalloc(N->allocs, &S.x0, n * 2);
-  if (!rc) rc = dalloc(N->allocs, &S.t, n);
+  rc = dalloc(N->allocs, &S.x0, n * 2, N->stream);
+  if (!rc) rc = dalloc(N->allocs, &S.t, n, N->stream);
   if (rc) return rc;
   float *tmp = nullptr;
   if (hipMalloc(&tmp, n * sizeof(float)) != hipSuccess) return nfail(PYRO_E_OOM, "hipMalloc failed");
@@ -515,7 +518,7 @@ int pyro_net_train(PyroNet *N, int first, int count, int steps, float lr, uint64
   if (!N || steps < 0 || !(lr > 0.0f)) return nfail(PYRO_E_INVALID, "bad argument");
   if (N->data.empty()) return nfail(PYRO_E_STATE, "empty training set");
   if (first < 0 || count < 1 || first + count > (int)N->data.size()) return nfail(PYRO_E_INVALID, "bad pair range");
-  int rc = work_alloc(N->tr, N->data_g, true);
+  int rc = work_alloc(N->tr, N->data_g, true, N->stream);
   if (rc) return rc;
   if (N->losses_cap < steps) {
     if (N->losses) {
@@ -526,7 +529,7 @@ int pyro_net_train(PyroNet *N, int first, int count, int steps, float lr, uint64
           break;
         }
     }
-    rc = dalloc(N->allocs, &N->losses, (size_t)steps);
+    rc = dalloc(N->allocs, &N->losses, (size_t)steps, N->stream);
     if (rc) return rc;
     N->losses_cap = steps;
   }
@@ -554,7 +557,7 @@ int pyro_net_train(PyroNet *N, int first, int count, int steps, float lr, uint64
 int pyro_net_eval(PyroNet *N, int first, int count, double *mean_loss) {
   if (!N || !mean_loss || first < 0 || count < 1 || first + count > (int)N->data.size())
     return nfail(PYRO_E_INVALID, "bad argument");
-  int rc = work_alloc(N->tr, N->data_g, true);
+  int rc = work_alloc(N->tr, N->data_g, true, N->stream);
   if (rc) return rc;
   double sum = 0.0;
   for (int k = first; k < first + count; k++) {
@@ -577,7 +580,7 @@ int pyro_net_time_forward(PyroNet *N, uint32_t nx, uint32_t ny, uint32_t nz, int
   int rc = check_dims(nx, ny, nz);
   if (rc) return rc;
   const G3 g{(int)nx, (int)ny, (int)nz};
-  rc = work_alloc(N->inf, g, false);
+  rc = work_alloc(N->inf, g, false, N->stream);
   if (rc) return rc;
   forward(N, N->inf, N->inf.x0);
   hipEvent_t a, b;
@@ -600,10 +603,10 @@ int pyro_debug_mfma(const float *a, const float *b, float *d) {
   std::vector<void *> L;
   bf16 *da, *db;
   float *dd, *tmp;
-  int rc = dalloc(L, &da, 512);
-  if (!rc) rc = dalloc(L, &db, 512);
-  if (!rc) rc = dalloc(L, &dd, 256);
-  if (!rc) rc = dalloc(L, &tmp, 512);
+  int rc = dalloc(L, &da, 512, nullptr);
+  if (!rc) rc = dalloc(L, &db, 512, nullptr);
+  if (!rc) rc = dalloc(L, &dd, 256, nullptr);
+  if (!rc) rc = dalloc(L, &tmp, 512, nullptr);
   if (!rc) {
     if (hipMemcpy(tmp, a, 512 * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) rc = PYRO_E_HIP;
     launch_f32_to_bf16(512, tmp, da, nullptr);
@@ -639,13 +642,13 @@ int pyro_debug_conv(int ca, int cb, int cout, int transposed, int relu, uint32_t
   const size_t n = g.n(), nh = gh.n();
   const size_t nwp = first ? 1024 : (size_t)(transposed ? conv_groups(0, cout, c.cin()) * c.cin() : conv_groups(ca, cb, cout) * cout) * 32;
   const size_t big = std::max(std::max(n * in_b, nh * (size_t)(ca ? ca : 1)), n * out_c);
-  rc = dalloc(L, &dbb, n * in_b);
-  if (!rc && ca) rc = dalloc(L, &da, nh * ca);
-  if (!rc) rc = dalloc(L, &wp, nwp);
-  if (!rc) rc = dalloc(L, &dout, n * out_c);
-  if (!rc) rc = dalloc(L, &tmp, big);
-  if (!rc) rc = dalloc(L, &dW, (size_t)cout * c.cin() * 27);
-  if (!rc && bias && !transposed) rc = dalloc(L, &dbias, cout);
+  rc = dalloc(L, &dbb, n * in_b, nullptr);
+  if (!rc && ca) rc = dalloc(L, &da, nh * ca, nullptr);
+  if (!rc) rc = dalloc(L, &wp, nwp, nullptr);
+  if (!rc) rc = dalloc(L, &dout, n * out_c, nullptr);
+  if (!rc) rc = dalloc(L, &tmp, big, nullptr);
+  if (!rc) rc = dalloc(L, &dW, (size_t)cout * c.cin() * 27, nullptr);
+  if (!rc && bias && !transposed) rc = dalloc(L, &dbias, cout, nullptr);
   auto up = [&](const float *h, size_t cnt, bf16 *dst) {
     if (hipMemcpy(tmp, h, cnt * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) return PYRO_E_HIP;
     launch_f32_to_bf16((uint32_t)cnt, tmp, dst, nullptr);
@@ -692,15 +695,15 @@ int pyro_debug_conv_dw(int ca, int cb, int cout, uint32_t nx, uint32_t ny, uint3
   bf16 *da = nullptr, *dbb, *dg, *xt, *gt;
   float *tmp, *ddw, *ddb, *part;
   const size_t big = std::max(std::max(n * cb, n * cout), nh * (size_t)(ca ? ca : 1));
-  rc = dalloc(L, &dbb, n * cb);
-  if (!rc && ca) rc = dalloc(L, &da, nh * ca);
-  if (!rc) rc = dalloc(L, &dg, n * cout);
-  if (!rc) rc = dalloc(L, &xt, dw_xt_elems(gg, c));
-  if (!rc) rc = dalloc(L, &gt, dw_gt_elems(gg, c));
-  if (!rc) rc = dalloc(L, &part, dw_part_elems(gg, c));
-  if (!rc) rc = dalloc(L, &tmp, big);
-  if (!rc) rc = dalloc(L, &ddw, (size_t)cout * c.cin() * 27);
-  if (!rc) rc = dalloc(L, &ddb, cout);
+  rc = dalloc(L, &dbb, n * cb, nullptr);
+  if (!rc && ca) rc = dalloc(L, &da, nh * ca, nullptr);
+  if (!rc) rc = dalloc(L, &dg, n * cout, nullptr);
+  if (!rc) rc = dalloc(L, &xt, dw_xt_elems(gg, c), nullptr);
+  if (!rc) rc = dalloc(L, &gt, dw_gt_elems(gg, c), nullptr);
+  if (!rc) rc = dalloc(L, &part, dw_part_elems(gg, c), nullptr);
+  if (!rc) rc = dalloc(L, &tmp, big, nullptr);
+  if (!rc) rc = dalloc(L, &ddw, (size_t)cout * c.cin() * 27, nullptr);
+  if (!rc) rc = dalloc(L, &ddb, cout, nullptr);
   auto up = [&](const float *h, size_t cnt, bf16 *dst) {
     if (hipMemcpy(tmp, h, cnt * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) return PYRO_E_HIP;
     launch_f32_to_bf16((uint32_t)cnt, tmp, dst, nullptr);

@@ -82,6 +82,8 @@ struct PyroPoisson {
 };
 
 namespace {
+// Zeroed on the null stream: a synchronous copy follows in pyro_poisson_create,
+// before P->stream (which does not wait for the null stream) uses any of it.
 template <class T>
 int palloc(PyroPoisson *P, T **ptr, size_t count) {
   void *v = nullptr;

@@ -78,6 +78,8 @@ struct PyroSim {
 
 namespace {
 
+// Zeroed on the null stream, for which s->stream does not wait and the host not
+// either: a synchronous copy or a wait has to follow before the first use.
 int dalloc(PyroSim *s, void **p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes < 16 ? 16 : bytes);
   if (e != hipSuccess) return fail(PYRO_E_OOM, std::string("hipMalloc(") + std::to_string(bytes) + "): " + hipGetErrorString(e));
@@ -508,6 +510,7 @@ int pyro_sim_render_pack(PyroSim *s, void *host_dst, size_t bytes) {
   if (!s->render) {
     int rc = dalloc(s, &s->render, need);
     if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(nullptr));
   }
   if (!s->copy_stream) HIPCHK(hipStreamCreateWithFlags(&s->copy_stream, hipStreamNonBlocking));
   if (!s->ev_packed) HIPCHK(hipEventCreateWithFlags(&s->ev_packed, hipEventDisableTiming));
