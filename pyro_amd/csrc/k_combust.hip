@@ -366,10 +366,10 @@ __global__ __launch_bounds__(NT) void k_solid(const Params *__restrict__ P, Geo 
 // 164, 273 and 141 with the tiles dealt out singly to 1024 blocks, where the
 // marches of neighbouring tiles no longer share an XCD's cache and a block's
 // tiles at 128^3 are whole planes apart, all of them solid or all empty; 122,
-// 238 and 91 here.  Fewer blocks are faster by up to 5 % with fuel in one
-// place (1024: 530 at 320x480x320, 15.6 instead of 17.4 at 80x160x80) and up to
-// a half slower with solids all over; runs of 4 and 64 tiles lose in both.  The
-// number is no power of two, as the planes often are.
+// 238 and 91 here.  Fewer blocks are faster by 2 to 4 us with fuel in one
+// place (1024: 15.1 instead of 17.4 at 80x160x80, 20.8 and 24.6 at 112x240x112)
+// and up to a half slower with solids all over; runs of 4 and 64 tiles lose in
+// both.  The number is no power of two, as the planes often are.
 constexpr int SOLID_RUN = 16, SOLID_GROUP = 8 * SOLID_RUN, SOLID_BLOCKS = 35 * SOLID_GROUP, SOLID_BATCH = 8;
 // Tile at position k < nt: runs of consecutive tiles, each on one XCD (k % 8).
 __device__ __forceinline__ int solid_order(int k, int nt) {
